@@ -60,6 +60,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 
 HBM_PEAK_GBS = 8000.0
+WINDOW_ROWS = 131072  # levels of this many nodes or more are swept in windows (m3::sweep_window)
 
 # HBM bytes per launch of the dominant kernel, measured with two rocprofv3
 # counter passes (FETCH_SIZE x 2.0000 + WRITE_SIZE x 1.0000, factors from the
@@ -67,7 +68,6 @@ HBM_PEAK_GBS = 8000.0
 # profiles/c1_k_smooth_hbm_traffic.md.  Keyed by (config, kernel); other
 # configs and kernels report null.
 MEASURED_TRAFFIC = {
-    ("c1", "k_smooth<B16P,float,6,1,3,true>"): 319414234,
 }
 
 
@@ -79,9 +79,10 @@ def sweep_bytes(nnzb, nnod, blk_val_bytes=72, vec_bytes=8):
     """Algorithmic bytes of one fused Jacobi sweep r = r0 - K d; d' = d + w D^-1 r
     on the fine level: every stored 3x3 block once (its nine values,
     blk_val_bytes: 72 in FP64, 20 in the packed BF16 layout of eight BF16
-    values and an FP32 v8; + int32 column), the row table, and per row the
-    vectors d (gather, perfect reuse), r0, D^-1 read and d' written."""
-    return nnzb * (blk_val_bytes + 4) + nnod * 4 + nnod * 3 * 4 * vec_bytes
+    values and an FP32 v8; + its column: an int32, or a two-byte place in the
+    window on the levels that are swept in windows), the row table, and per
+    row the vectors d (gather, perfect reuse), r0, D^-1 read and d' written."""
+    return nnzb * (blk_val_bytes + (2 if nnod >= WINDOW_ROWS else 4)) + nnod * 4 + nnod * 3 * 4 * vec_bytes
 
 
 def cpu_threads():
@@ -142,7 +143,7 @@ def roofline(ctx, mesh, api, run_once, form, config):
     t_all, b_all, n_all = tsw + pr["t_vcycle_other"], bsw + pr["b_vcycle_other"], nsw + pr["n_vcycle_other"]
     vc = b_all / t_all / 1e9
     log(f"V-cycle: {n_all} launches, {t_all * 1e3:.2f} ms, {b_all / 1e9:.2f} GB -> {vc:.0f} GB/s")
-    kern = "k_smooth<double,double,6,1,2,true>" if form == "fp64" else "k_smooth<B16P,float,6,1,3,true>"
+    kern = ("k_sweep_win" if nnod >= WINDOW_ROWS else "k_sweep") + ("<double,double,6>" if form == "fp64" else "<B16P,float,6>")
     cp = round(api.copy_rate(1 << 30, 20), 1)   # plain copy kernel of 1 GiB, read + write bytes
     log(f"copy kernel: {cp:.0f} GB/s")
     return dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",

@@ -459,7 +459,7 @@ __global__ __launch_bounds__(64) void k_assemble(AsmArgs a) {
     const double *blk = s_Kl + 9 * (lo ? na * (na + 1) / 2 + nb : nb * (nb + 1) / 2 + na);
     for (int cc = 0; cc < 3; ++cc)
       for (int dd = 0; dd < 3; ++dd)
-        atomicAdd(a.K.val + (3 * cc + dd) * a.K.nslot + pos, lo ? blk[3 * cc + dd] : blk[3 * dd + cc]);
+        atomicAdd(a.K.val + kval(pos, 3 * cc + dd), lo ? blk[3 * cc + dd] : blk[3 * dd + cc]);
   }
   // ---------------- G (rotated): G_rot[a,:,v] = RR_a' G[a,:,v]; it depends
   // on the geometry only, so the host skips it when the mesh is unchanged
@@ -615,7 +615,7 @@ __global__ __launch_bounds__(64) void k_rap(RapArgs a) {
     for (int cc = 0; cc < 3; ++cc)
       for (int dd = 0; dd < 3; ++dd) {
         const double v = 0.5 * (s_Kc[3 * na + cc][3 * nb + dd] + s_Kc[3 * nb + dd][3 * na + cc]);
-        atomicAdd(a.K.val + (3 * cc + dd) * a.K.nslot + pos, v);
+        atomicAdd(a.K.val + kval(pos, 3 * cc + dd), v);
       }
   }
 }
@@ -667,7 +667,7 @@ __global__ __launch_bounds__(64 * GK_ROWS) void k_gatherK(SellView K, int64_t nr
   __syncthreads();
   for (int t = lane; t < len * 9; t += 64) {
     const int k = t / 9, v = t - 9 * k;
-    K.val[v * K.nslot + base + 64 * (int64_t)k] = A[t];
+    K.val[kval(base + 64 * (int64_t)k, v)] = A[t];
   }
 }
 
@@ -675,17 +675,17 @@ __global__ __launch_bounds__(64 * GK_ROWS) void k_gatherK(SellView K, int64_t nr
 // of contributing element blocks (each a contiguous 72-byte block of Kel,
 // transposed when the element's local row node precedes its column node) is
 // added in list order and the nine values are written once, coalesced over
-// the slots of a wave; padding slots have empty lists and get zeros.  p16
+// the slots of a wave; padding slots have empty lists and are never read.  p16
 // (finest level): the same block also in the mixed V-cycle's packed BF16
-// layout, eight BF16 in one 16-byte group at p16 + 4 slot (v_2i in the low
-// half of word i) and (v8 in FP32, column) at p16 + 4 nslot + 2 slot.
+// layout (p16_words, p16_v8).
 __global__ __launch_bounds__(256) void k_gatherK_slots(SellView K, const int64_t *cptr, const int32_t *clist,
-                                                       const double *Kel, float *p16) {
+                                                       const double *Kel, uint32_t *p16) {
   const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (s >= K.nslot) return;
   double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  const int64_t m1 = cptr[s + 1];
-  for (int64_t m = cptr[s]; m < m1; ++m) {
+  const int64_t m0 = cptr[s], m1 = cptr[s + 1];
+  if (m0 == m1) return;
+  for (int64_t m = m0; m < m1; ++m) {
     const int32_t code = clist[m];
     const double *kb = Kel + 9 * (int64_t)(code >> 1);
     double v[9];
@@ -701,8 +701,10 @@ __global__ __launch_bounds__(256) void k_gatherK_slots(SellView K, const int64_t
       for (int t = 0; t < 9; ++t) acc[t] += v[t];
     }
   }
+  typedef double d2w __attribute__((ext_vector_type(2)));
 #pragma unroll
-  for (int t = 0; t < 9; ++t) K.val[t * K.nslot + s] = acc[t];
+  for (int t = 0; t < 8; t += 2) *reinterpret_cast<d2w *>(K.val + kval(s, t)) = d2w{acc[t], acc[t + 1]};
+  K.val[kval(s, 8)] = acc[8];
   if (p16) {
     typedef uint32_t u4w __attribute__((ext_vector_type(4)));
     u4w g;
@@ -710,9 +712,8 @@ __global__ __launch_bounds__(256) void k_gatherK_slots(SellView K, const int64_t
     g.y = bf16_rne(acc[2]) | (bf16_rne(acc[3]) << 16);
     g.z = bf16_rne(acc[4]) | (bf16_rne(acc[5]) << 16);
     g.w = bf16_rne(acc[6]) | (bf16_rne(acc[7]) << 16);
-    *reinterpret_cast<u4w *>(p16 + 4 * s) = g;
-    p16[4 * K.nslot + 2 * s] = (float)acc[8];
-    p16[4 * K.nslot + 2 * s + 1] = __int_as_float(K.col[s]);
+    *reinterpret_cast<u4w *>(p16 + p16_words(s)) = g;
+    p16[p16_v8(s)] = __float_as_uint((float)acc[8]);
   }
 }
 
@@ -802,26 +803,29 @@ __global__ void k_kslots(int64_t nel, const int32_t *el2nod, SellView K, int32_t
 // identity at fixed dofs on the diagonal blocks, inverse diagonal
 // fixed dofs get a unit diagonal; p16 (finest level): the packed BF16 copy
 // that the slot gather wrote gets the same unit entries (v0 and v4 are the
-// low halves of words 0 and 2 of the block's group, v8 is the FP32 of its pair)
-__global__ void k_fix_diag(SellView K, const double *mask, int64_t nnod, double *dinv, float *p16) {
+// low halves of words 0 and 2 of the block's group).  dinv is in
+// the level's vector order (vpos: place of each node, NULL for the node order).
+__global__ void k_fix_diag(SellView K, const double *mask, const int32_t *vpos, int64_t nnod, double *dinv,
+                           uint32_t *p16) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= nnod) return;
   const int64_t pos = sell_find(K, (int)i, (int)i);
   if (pos < 0) return;
+  const int64_t o = 3 * (vpos ? (int64_t)vpos[i] : i);
   for (int c = 0; c < 3; ++c) {
-    double *b = K.val + (4 * c) * K.nslot + pos;
+    double *b = K.val + kval(pos, 4 * c);
     if (mask[3 * i + c] == 0.0) {
       *b = 1.0;
       if (p16) {
         if (c == 2) {
-          p16[4 * K.nslot + 2 * pos] = 1.0f;
+          p16[p16_v8(pos)] = __float_as_uint(1.0f);
         } else {
-          uint32_t *wd = reinterpret_cast<uint32_t *>(p16) + 4 * pos + 2 * c;
+          uint32_t *wd = p16 + p16_words(pos) + 2 * c;
           *wd = (*wd & 0xffff0000u) | bf16_rne(1.0);
         }
       }
     }
-    dinv[3 * i + c] = 1.0 / *b;
+    dinv[o + c] = 1.0 / *b;
   }
 }
 
@@ -937,10 +941,10 @@ void launch_gather_K(m3_ctx *c, int level) {
   LevelDev &f = c->L[level];
   if (level == 0) c->pack16_fresh = false;
   if (f.cptr.p) {
-    float *p16 = nullptr;
+    uint32_t *p16 = nullptr;
     if (level == 0 && c->nmg > 1) {  // the finest level's packed BF16 values, written in the same pass
-      if (f.K.val32.n != (size_t)(6 * f.K.nslot)) f.K.val32.alloc(6 * f.K.nslot);
-      p16 = f.K.val32.p;
+      if (f.K.val16.n != (size_t)(P16 * f.K.nslot)) f.K.val16.alloc(P16 * f.K.nslot);
+      p16 = f.K.val16.p;
     }
     hipLaunchKernelGGL(k_gatherK_slots, dim3((unsigned)((f.K.nslot + 255) / 256)), dim3(256), 0, c->stream,
                        f.K.view(), f.cptr.p, f.clist.p, f.Kel.p, p16);
@@ -1003,9 +1007,9 @@ void launch_slots(m3_ctx *c) {
 void launch_fix_diag(m3_ctx *c, int l) {
   LevelDev &lv = c->L[l];
   const int bs = 256;
-  float *p16 = (l == 0 && c->pack16_fresh) ? lv.K.val32.p : nullptr;
+  uint32_t *p16 = (l == 0 && c->pack16_fresh) ? lv.K.val16.p : nullptr;
   hipLaunchKernelGGL(k_fix_diag, dim3((unsigned)((lv.nnod + bs - 1) / bs)), dim3(bs), 0,
-                     c->stream, lv.K.view(), lv.mask.p, lv.nnod, lv.dinv.p, p16);
+                     c->stream, lv.K.view(), lv.mask.p, lv.K.vpos_p(), lv.nnod, lv.dinv.p, p16);
   HIPCHECK(hipGetLastError());
 }
 

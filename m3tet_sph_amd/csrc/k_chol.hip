@@ -1047,7 +1047,7 @@ void chol_analyse(m3_ctx *c) {
     }
     bw.end_height();
   }
-  // gather map from the coarse operator values (SoA, 9*nslot)
+  // gather map from the coarse operator values
   std::vector<int64_t> gsrc, gdst;
   for (int64_t n = 0; n < nn; ++n) {
     const int64_t base = K.base_of(n);
@@ -1061,7 +1061,7 @@ void chol_analyse(m3_ctx *c) {
           const int pb = inv[3 * (int64_t)m + b];
           if (pb < 0 || pa < pb) continue;
           const int32_t t = tile_of(pa / TS, pb / TS);
-          gsrc.push_back((int64_t)(3 * a + b) * K.nslot + slot);
+          gsrc.push_back(kval(slot, 3 * a + b));
           gdst.push_back((int64_t)t * TT + (pa % TS) + (int64_t)TS * (pb % TS));
         }
       }

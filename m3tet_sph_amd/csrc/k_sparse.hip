@@ -12,10 +12,13 @@
 // dofs; the operators carry an identity at those dofs, which makes every
 // iterate equal to the reference's reduced vectors padded with zeros.
 //
-// Precision: value type MT (double, float or bf16 bits) and vector type VT
-// (double or float) are template parameters; the FP64 path instantiates
-// MT=VT=double, the mixed path runs the whole V-cycle in FP32 with BF16
-// coarse-level matrix values.
+// Precision: value type MT and vector type VT are template parameters; the
+// FP64 path instantiates MT=VT=double, the mixed path runs the whole V-cycle
+// in FP32 on packed BF16 matrix values (MT=B16P).
+//
+// Vectors of a level are in K's vector order here (Sell): the node order on
+// small levels, a space-filling order on the levels whose sweeps run on
+// windows.  mgpcg_run takes and returns vectors in node order.
 #include "m3_internal.h"
 
 #include <hip/hip_ext.h>
@@ -24,185 +27,259 @@
 
 namespace {
 
-template <class T>
-__device__ inline float to_f(T v);
-template <>
-__device__ inline float to_f<float>(float v) { return v; }
-template <>
-__device__ inline float to_f<uint16_t>(uint16_t v) {
-  return __uint_as_float(((uint32_t)v) << 16);
-}
-
-template <class MT>
-__device__ inline double mval(const MT *p);
-template <>
-__device__ inline double mval<double>(const double *p) { return *p; }
-template <>
-__device__ inline double mval<float>(const float *p) { return (double)*p; }
-
-// BF16 values of the finest level in packed groups per slot: (v0..v7) as
-// eight BF16 (round to nearest even) in one 16-byte group at val + 4 slot
-// (32-bit words, v_2i in the low half of word i), and v8 in FP32 with the
-// block's column (its bits) at val + 4 nslot + 2 slot: 24 bytes per block,
-// one 16-byte and one 8-byte load instead of nine values and a column of 4
-// bytes each, every load still one contiguous segment per wave
+// BF16 values in packed groups (kval's counterpart p16_words / p16_v8): eight
+// BF16 (round to nearest even) in one 16-byte load and v8 in FP32, 20 bytes
+// per block
 struct B16P {
-  float f;
+  uint32_t w;
 };
-typedef float f2v __attribute__((ext_vector_type(2)));
+typedef double d2v __attribute__((ext_vector_type(2)));
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 __device__ inline float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ inline float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 // bytes of the nine values of one stored block
 template <class MT>
 constexpr double block_value_bytes() {
-  return std::is_same<MT, B16P>::value ? 8 * 2.0 + 4.0 : 9.0 * sizeof(MT);
+  return std::is_same<MT, B16P>::value ? 4.0 * P16 : 9.0 * sizeof(MT);
 }
 
-template <class MT, class VT>
-struct Acc;  // accumulation type: double for FP64, float otherwise
-template <>
-struct Acc<double, double> { using T = double; };
-template <>
-struct Acc<float, float> { using T = float; };
-template <>
-struct Acc<uint16_t, float> { using T = float; };
-template <>
-struct Acc<B16P, float> { using T = float; };
-
-template <class MT>
-__device__ inline auto ldv(const MT *p) {
-  if constexpr (std::is_same<MT, uint16_t>::value) return to_f<uint16_t>(*p);
-  else return *p;
-}
-
-// streaming load (matrix values and columns are read once per sweep; keeping
-// them out of the way leaves the L2 to the gathered vector)
+// streaming load
 template <bool NT, class T>
 __device__ inline T lds_(const T *p) {
   if constexpr (NT) return __builtin_nontemporal_load(p);
   else return *p;
 }
-template <bool NT, class MT>
-__device__ inline auto ldm(const MT *p) {
-  if constexpr (std::is_same<MT, uint16_t>::value) return to_f<uint16_t>(lds_<NT>(p));
-  else return lds_<NT>(p);
+
+// one 3x3 block of a group of 64 slots as a lane holds it
+template <class MT, bool NT>
+struct Blk;
+template <bool NT>
+struct Blk<double, NT> {
+  d2v a[4];
+  double e;
+  __device__ inline void load(const double *val, int64_t group, int lane) {
+    const double *v = val + 576 * group;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] = lds_<NT>(reinterpret_cast<const d2v *>(v + 128 * j) + lane);
+    e = lds_<NT>(v + 512 + lane);
+  }
+  __device__ inline void apply(double x0, double x1, double x2, double &y0, double &y1, double &y2) const {
+    y0 += a[0].x * x0 + a[0].y * x1 + a[1].x * x2;
+    y1 += a[1].y * x0 + a[2].x * x1 + a[2].y * x2;
+    y2 += a[3].x * x0 + a[3].y * x1 + e * x2;
+  }
+};
+template <bool NT>
+struct Blk<B16P, NT> {
+  u4v g;
+  float e;
+  __device__ inline void load(const B16P *val, int64_t group, int lane) {
+    const B16P *v = val + 64 * P16 * group;
+    g = lds_<NT>(reinterpret_cast<const u4v *>(v) + lane);
+    e = lds_<NT>(reinterpret_cast<const float *>(v + 256) + lane);
+  }
+  __device__ inline void apply(float x0, float x1, float x2, float &y0, float &y1, float &y2) const {
+    y0 += bf_lo(g.x) * x0 + bf_hi(g.x) * x1 + bf_lo(g.y) * x2;
+    y1 += bf_hi(g.y) * x0 + bf_lo(g.z) * x1 + bf_hi(g.z) * x2;
+    y2 += bf_lo(g.w) * x0 + bf_hi(g.w) * x1 + e * x2;
+  }
+};
+
+// the vectors of a sweep: MODE bits 1: y = K x; 2: r = r0 - K x (to r_out
+// unless NULL); 4: d_out = x + w Dinv r; 8: partial sums of x . K x per workgroup
+template <class VT>
+struct SweepVec {
+  const VT *x, *r0, *dinv;
+  VT w;
+  VT *y, *r_out, *d_out;
+  double *part;
+};
+template <class VT, int MODE>
+__device__ inline void sweep_out(const SweepVec<VT> &v, int64_t o, VT kx, double &dot) {
+  if (MODE & 1) v.y[o] = kx;
+  if (MODE & 2) {
+    const VT q = v.r0[o] - kx;
+    if (v.r_out) v.r_out[o] = q;
+    if (MODE & 4) v.d_out[o] = v.x[o] + v.w * v.dinv[o] * q;
+  }
+  if (MODE & 8) dot += (double)v.x[o] * (double)kx;
+}
+// sum of s over the workgroup's NW waves, in order, to part[blockIdx.x]
+template <int NW>
+__device__ inline void block_part(double s, double *sh, double *part) {
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = sh[0];
+    for (int j = 1; j < NW; ++j) t += sh[j];
+    part[blockIdx.x] = t;
+  }
 }
 
-template <class MT, class VT, int MODE, int TPR, int UNR, bool NT>
-__global__ __launch_bounds__(256) void k_smooth(SellT<MT> K, int64_t nrow, const VT *__restrict__ x,
-                                                const VT *__restrict__ r0, const VT *__restrict__ dinv,
-                                                VT w, VT *__restrict__ y, VT *__restrict__ r_out,
-                                                VT *__restrict__ d_out, double *__restrict__ part) {
-  using A = typename Acc<MT, VT>::T;
-  const int64_t gt = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t q = gt / TPR;  // position in the slices; the row it holds:
-  const int64_t row = q < nrow ? (K.perm ? (int64_t)K.perm[q] : q) : q;
-  const int sub = (int)(gt % TPR);
-  A y0 = 0, y1 = 0, y2 = 0;
-  if (q < nrow) {
-    const int64_t base = K.slice_ptr[q >> 6] + (q & 63);
-    const int len = K.rowlen[row];
-    const int64_t ns = K.nslot;
-    const MT *v = K.val;
-    int k = sub;
-    for (; k + (UNR - 1) * TPR < len; k += UNR * TPR) {
-      int64_t pp[UNR], cc[UNR];
-      float c8[UNR];
+// Sweep of a level without windows: one slice of 64 rows per workgroup, its
+// stored blocks dealt to W waves (wave w takes blocks w, w + W, ...: every load
+// still one contiguous stretch per wave), partial sums added in LDS.  These
+// levels are latency-bound: a vertex row of 65 blocks is a chain of dependent
+// column and vector loads, and one wave per slice leaves the chip empty.  5,778
+// rows, FP64 / BF16: four lanes per row 22.7 us, W = 4 / 8 / 16: 9.5 / 7.8 /
+// 7.9 us and 5.7 / 4.8 / 4.7 us; 43,554 rows: four lanes per row 37.6 and 15.3
+// us, W = 4 / 8 / 16: 26.8 / 23.6 / 20.5 us and 10.3 / 9.3 / 8.6 us.
+template <class MT, class VT, int MODE, int W, int UNR>
+__global__ __launch_bounds__(64 * W) void k_sweep(SweepPat K, const MT *__restrict__ val, SweepVec<VT> v) {
+  __shared__ VT sh[W][192];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t q = (int64_t)blockIdx.x * 64 + lane;
+  const int64_t g0 = K.slice_ptr[blockIdx.x] >> 6;
+  const int len = q < K.n ? K.len[q] : 0;
+  VT y0 = 0, y1 = 0, y2 = 0;
+  auto blocks = [&](int k0, auto cnt) {
+    constexpr int N = decltype(cnt)::value;
+    int cc[N];
+    VT x[N][3];
+    Blk<MT, false> b[N];
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        pp[u] = base + (int64_t)(k + u * TPR) * 64;
-        if constexpr (std::is_same<MT, B16P>::value) {
-          const f2v pc = lds_<NT>(reinterpret_cast<const f2v *>(reinterpret_cast<const float *>(v) + 4 * ns) + pp[u]);
-          c8[u] = pc.x;
-          cc[u] = 3 * (int64_t)__float_as_int(pc.y);
-        } else {
-          cc[u] = 3 * (int64_t)lds_<NT>(K.col + pp[u]);
-        }
-      }
-      A xx[UNR][3];
+    for (int u = 0; u < N; ++u) {
+      cc[u] = lds_<false>(K.col + (g0 + k0 + u * W) * 64 + lane);
+      b[u].load(val, g0 + k0 + u * W, lane);
+    }
 #pragma unroll
-      for (int u = 0; u < UNR; ++u)
+    for (int u = 0; u < N; ++u)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) xx[u][j] = (A)x[cc[u] + j];
+      for (int j = 0; j < 3; ++j) x[u][j] = v.x[3 * (int64_t)cc[u] + j];
 #pragma unroll
-      for (int u = 0; u < UNR; ++u) {
-        const int64_t p = pp[u];
-        if constexpr (std::is_same<MT, B16P>::value) {
-          const u4v g = lds_<NT>(reinterpret_cast<const u4v *>(v) + p);
-          y0 += bf_lo(g.x) * xx[u][0] + bf_hi(g.x) * xx[u][1] + bf_lo(g.y) * xx[u][2];
-          y1 += bf_hi(g.y) * xx[u][0] + bf_lo(g.z) * xx[u][1] + bf_hi(g.z) * xx[u][2];
-          y2 += bf_lo(g.w) * xx[u][0] + bf_hi(g.w) * xx[u][1] + c8[u] * xx[u][2];
-        } else {
-          y0 += (A)ldm<NT>(v + p) * xx[u][0] + (A)ldm<NT>(v + ns + p) * xx[u][1] +
-                (A)ldm<NT>(v + 2 * ns + p) * xx[u][2];
-          y1 += (A)ldm<NT>(v + 3 * ns + p) * xx[u][0] + (A)ldm<NT>(v + 4 * ns + p) * xx[u][1] +
-                (A)ldm<NT>(v + 5 * ns + p) * xx[u][2];
-          y2 += (A)ldm<NT>(v + 6 * ns + p) * xx[u][0] + (A)ldm<NT>(v + 7 * ns + p) * xx[u][1] +
-                (A)ldm<NT>(v + 8 * ns + p) * xx[u][2];
-        }
-      }
-    }
-    for (; k < len; k += TPR) {
-      const int64_t p = base + (int64_t)k * 64;
-      float c8 = 0;
-      int64_t cc;
-      if constexpr (std::is_same<MT, B16P>::value) {
-        const f2v pc = lds_<NT>(reinterpret_cast<const f2v *>(reinterpret_cast<const float *>(v) + 4 * ns) + p);
-        c8 = pc.x;
-        cc = 3 * (int64_t)__float_as_int(pc.y);
-      } else {
-        cc = 3 * (int64_t)lds_<NT>(K.col + p);
-      }
-      const A x0 = (A)x[cc], x1 = (A)x[cc + 1], x2 = (A)x[cc + 2];
-      if constexpr (std::is_same<MT, B16P>::value) {
-        const u4v g = lds_<NT>(reinterpret_cast<const u4v *>(v) + p);
-        y0 += bf_lo(g.x) * x0 + bf_hi(g.x) * x1 + bf_lo(g.y) * x2;
-        y1 += bf_hi(g.y) * x0 + bf_lo(g.z) * x1 + bf_hi(g.z) * x2;
-        y2 += bf_lo(g.w) * x0 + bf_hi(g.w) * x1 + c8 * x2;
-      } else {
-        y0 += (A)ldm<NT>(v + p) * x0 + (A)ldm<NT>(v + ns + p) * x1 + (A)ldm<NT>(v + 2 * ns + p) * x2;
-        y1 += (A)ldm<NT>(v + 3 * ns + p) * x0 + (A)ldm<NT>(v + 4 * ns + p) * x1 + (A)ldm<NT>(v + 5 * ns + p) * x2;
-        y2 += (A)ldm<NT>(v + 6 * ns + p) * x0 + (A)ldm<NT>(v + 7 * ns + p) * x1 + (A)ldm<NT>(v + 8 * ns + p) * x2;
-      }
-    }
-  }
-  if (TPR > 1) {
-    for (int off = TPR / 2; off > 0; off >>= 1) {
-      y0 += __shfl_xor(y0, off, TPR);
-      y1 += __shfl_xor(y1, off, TPR);
-      y2 += __shfl_xor(y2, off, TPR);
-    }
-  }
-  if (q < nrow && sub == 0) {
-    const int64_t o = 3 * row;
-    if (MODE & 1) { y[o] = (VT)y0; y[o + 1] = (VT)y1; y[o + 2] = (VT)y2; }
-    if (MODE & 2) {
-      const A q0 = (A)r0[o] - y0, q1 = (A)r0[o + 1] - y1, q2 = (A)r0[o + 2] - y2;
-      if (r_out) { r_out[o] = (VT)q0; r_out[o + 1] = (VT)q1; r_out[o + 2] = (VT)q2; }
-      if (MODE & 4) {
-        d_out[o] = (VT)((A)x[o] + (A)w * (A)dinv[o] * q0);
-        d_out[o + 1] = (VT)((A)x[o + 1] + (A)w * (A)dinv[o + 1] * q1);
-        d_out[o + 2] = (VT)((A)x[o + 2] + (A)w * (A)dinv[o + 2] * q2);
-      }
-    }
+    for (int u = 0; u < N; ++u) b[u].apply(x[u][0], x[u][1], x[u][2], y0, y1, y2);
+  };
+  int k = w;
+  for (; k + (UNR - 1) * W < len; k += UNR * W) blocks(k, std::integral_constant<int, UNR>{});
+  for (; k < len; k += W) blocks(k, std::integral_constant<int, 1>{});
+  sh[w][3 * lane] = y0;
+  sh[w][3 * lane + 1] = y1;
+  sh[w][3 * lane + 2] = y2;
+  __syncthreads();
+  double dot = 0;
+  if (threadIdx.x < 192) {
+    VT s = sh[0][threadIdx.x];
+#pragma unroll
+    for (int j = 1; j < W; ++j) s += sh[j][threadIdx.x];
+    const int64_t o = 192 * (int64_t)blockIdx.x + threadIdx.x;
+    if (o < 3 * K.n) sweep_out<VT, MODE>(v, o, s, dot);
   }
   if (MODE & 8) {
-    double s = 0;
-    if (q < nrow && sub == 0) {
-      const int64_t o = 3 * row;
-      s = (double)x[o] * (double)y0 + (double)x[o + 1] * (double)y1 + (double)x[o + 2] * (double)y2;
-    }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    __shared__ double sh[4];
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {  // the block's waves in order
-      double t = sh[0];
-      for (int j = 1; j < (int)(blockDim.x >> 6); ++j) t += sh[j];
-      part[blockIdx.x] = t;
-    }
+    __shared__ double ds[W];
+    block_part<W>(dot, ds, v.part);
   }
+}
+
+// Sweep on windows: one window of rows per workgroup (they lie close together
+// in space, about ten stored blocks share a column).  The window's part of x is
+// gathered once into LDS through the window's list, so the matrix streams with
+// no dependent load behind it, with two-byte places instead of four-byte
+// columns, and x leaves the caches about twice per sweep instead of filling
+// them.  Rounds of SW_TEAMS slices, SW_W waves each; a window's rows are sorted
+// by length, so the slices of one round are alike.  The sums go through LDS
+// into vector order, so that the vectors are read and written in whole lines.
+// HBM-bound: 337,986 rows, FP64 183 us with one wave per slice and gathers from
+// memory -> 132 us (5.5 TB/s on the bytes each array needs once), BF16 63.5 ->
+// 43.6 us; 2,662,530 rows 1,338 -> 1,024 us and 424 -> 328 us (5.8 TB/s).
+// Windows of 1,024 rows, four waves per slice or 16 waves per workgroup are
+// within 5 % or slower; eight waves a SIMD matter in BF16 (57.6 us with five).
+// RES: the values stay in the last-level cache between sweeps: cached loads and
+// a contiguous range of windows per XCD (43.2 -> 39.5 us alone for the BF16
+// values of 337,986 rows, which take 210 MB); streaming loads otherwise (FP64
+// there 149 us with cached loads).
+constexpr int SW_WIN = 512, SW_NW = 8, SW_W = 2, SW_TEAMS = SW_NW / SW_W;
+template <class MT, class VT, int MODE, int UNR, bool RES>
+__global__ __launch_bounds__(64 * SW_NW, (std::is_same<MT, double>::value ? 4 : 8)) void k_sweep_win(
+    SweepPat K, int nwin, int umax, const MT *__restrict__ val, SweepVec<VT> v) {
+  extern __shared__ __align__(16) unsigned char sw_lds[];
+  VT *xs = reinterpret_cast<VT *>(sw_lds);  // the window's gathered part of x
+  VT *ys = xs + 3 * umax;                   // K x of the window's rows, in vector order
+  int b = blockIdx.x;
+  if (RES) {  // workgroups go to the eight XCDs in turn
+    const int per = (nwin + 7) / 8;
+    b = (b & 7) * per + (b >> 3);
+    if (b >= nwin) b = -1;
+  }
+  double dot = 0;
+  if (b >= 0) {
+    const int l0 = K.lptr[b], nl = K.lptr[b + 1] - l0;
+    for (int t = threadIdx.x; t < 3 * nl; t += 64 * SW_NW) {
+      const int i = t / 3;
+      xs[t] = v.x[3 * (int64_t)K.list[l0 + i] + (t - 3 * i)];
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, w = wave % SW_W, team = wave / SW_W;
+    __syncthreads();
+#pragma unroll 1
+    for (int rd = 0; rd < SW_WIN / (64 * SW_TEAMS); ++rd) {
+      const int64_t sl = (int64_t)b * (SW_WIN / 64) + rd * SW_TEAMS + team;
+      const int64_t q = sl * 64 + lane;
+      VT y0 = 0, y1 = 0, y2 = 0;
+      VT *yr = ys;
+      if (q < K.n) {
+        const int64_t g0 = K.slice_ptr[sl] >> 6;
+        const int len = K.len[q];
+        yr += 3 * K.lrow[q];
+        auto blocks = [&](int k0, auto cnt) {
+          constexpr int N = decltype(cnt)::value;
+          int cc[N];
+          Blk<MT, !RES> bk[N];
+#pragma unroll
+          for (int u = 0; u < N; ++u) {
+            const int64_t g = g0 + k0 + u * SW_W;
+            cc[u] = lds_<!RES>(K.idx + g * 64 + lane);
+            bk[u].load(val, g, lane);
+          }
+#pragma unroll
+          for (int u = 0; u < N; ++u) {
+            const VT *xp = xs + 3 * cc[u];
+            bk[u].apply(xp[0], xp[1], xp[2], y0, y1, y2);
+          }
+        };
+        int k = w;
+        for (; k + (UNR - 1) * SW_W < len; k += UNR * SW_W) blocks(k, std::integral_constant<int, UNR>{});
+        for (; k < len; k += SW_W) blocks(k, std::integral_constant<int, 1>{});
+      }
+      // the slice's waves add their sums in turn (a row belongs to one lane of each)
+#pragma unroll
+      for (int j = 0; j < SW_W; ++j) {
+        if (w == j && q < K.n) {
+          yr[0] = j == 0 ? y0 : yr[0] + y0;
+          yr[1] = j == 0 ? y1 : yr[1] + y1;
+          yr[2] = j == 0 ? y2 : yr[2] + y2;
+        }
+        __syncthreads();
+      }
+    }
+    const int64_t o0 = 3 * (int64_t)b * SW_WIN;
+    for (int t = threadIdx.x; t < 3 * SW_WIN && o0 + t < 3 * K.n; t += 64 * SW_NW)
+      sweep_out<VT, MODE>(v, o0 + t, ys[t], dot);
+  }
+  if (MODE & 8) {
+    __shared__ double ds[SW_NW];
+    block_part<SW_NW>(dot, ds, v.part);
+  }
+}
+
+// vectors between the node order and a level's vector order
+__global__ void k_to_places(int64_t n3, const int32_t *perm, const double *x, double *y) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n3) return;
+  const int64_t q = i / 3;
+  y[i] = x[3 * (int64_t)perm[q] + (i - 3 * q)];
+}
+__global__ void k_to_nodes(int64_t n3, const int32_t *perm, const double *x, double *y) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n3) return;
+  const int64_t q = i / 3;
+  y[3 * (int64_t)perm[q] + (i - 3 * q)] = x[i];
+}
+// r = mask b: b in node order, r and the mask in vector order
+__global__ void k_rhs_in(int64_t n3, const int32_t *perm, const uint8_t *vmask, const double *b, double *r) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n3) return;
+  const int64_t q = i / 3;
+  r[i] = (double)vmask[i] * b[perm ? 3 * (int64_t)perm[q] + (i - 3 * q) : i];
 }
 
 // generic scalar-block SELL SpMV with bs values per block, rows with 3
@@ -277,7 +354,7 @@ __global__ void k_spmv_M(SellView M, int64_t nrow, const double *x, double *y) {
 // prolongation with the add of the saved defect: df = dd + mask_f * (P dc)
 template <class VT, class WT>
 __global__ void k_prolong(int64_t nf, const int64_t *ptr, const int32_t *col, const WT *w,
-                          const double *mask, const VT *dc, const VT *dd, VT *df) {
+                          const uint8_t *mask, const VT *dc, const VT *dd, VT *df) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= nf) return;
   VT a0 = 0, a1 = 0, a2 = 0;
@@ -300,7 +377,7 @@ __global__ void k_prolong(int64_t nf, const int64_t *ptr, const int32_t *col, co
 // ~100 fine nodes), reduced with cross-lane shuffles.
 template <class VT, class WT>
 __global__ __launch_bounds__(256) void k_restrict(int64_t nc, const int64_t *ptr, const int32_t *col,
-                                                  const WT *w, const double *mask, const VT *rf, VT *rc,
+                                                  const WT *w, const uint8_t *mask, const VT *rf, VT *rc,
                                                   const VT *dinv, VT w1, VT *d1) {
   const int64_t j = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 4;
   const int sub = threadIdx.x & 15;
@@ -349,17 +426,6 @@ template <class A, class B>
 __global__ void k_convert(int64_t n, const A *x, B *y) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) y[i] = (B)x[i];
-}
-
-__global__ void k_to_bf16(int64_t n, const double *x, uint16_t *y) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  // round to nearest even
-  const float f = (float)x[i];
-  uint32_t u = __float_as_uint(f);
-  const uint32_t lsb = (u >> 16) & 1u;
-  u += 0x7fffu + lsb;
-  y[i] = (uint16_t)(u >> 16);
 }
 
 // ---- reductions (deterministic two-stage) -----------------------------------------
@@ -559,22 +625,19 @@ __global__ void k_precond_diag(int64_t n, const double *r, const double *Adi, do
   if (i < n) d[i] = r[i] * Adi[i];
 }
 
-// FP64 SoA values (v * ns + slot) -> packed BF16 groups (B16P layout; the
-// slot gather of K writes the same bits itself when it assembles the finest
-// level, k_gatherK_slots)
-__global__ void k_pack16(int64_t ns, const double *val, const int32_t *col, float *out) {
+// FP64 values -> packed BF16 groups (the slot gather of K writes the same bits
+// itself when it assembles the finest level, k_gatherK_slots)
+__global__ void k_pack16(int64_t ns, const double *val, uint32_t *out) {
   const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (p >= ns) return;
-  u4v g;
-  g.x = bf16_rne(val[p]) | (bf16_rne(val[ns + p]) << 16);
-  g.y = bf16_rne(val[2 * ns + p]) | (bf16_rne(val[3 * ns + p]) << 16);
-  g.z = bf16_rne(val[4 * ns + p]) | (bf16_rne(val[5 * ns + p]) << 16);
-  g.w = bf16_rne(val[6 * ns + p]) | (bf16_rne(val[7 * ns + p]) << 16);
-  *reinterpret_cast<u4v *>(out + 4 * p) = g;
-  f2v c;
-  c.x = (float)val[8 * ns + p];
-  c.y = __int_as_float(col[p]);
-  *reinterpret_cast<f2v *>(out + 4 * ns + 2 * p) = c;
+  uint32_t w[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const d2v v = *reinterpret_cast<const d2v *>(val + kval(p, 2 * j));
+    w[j] = bf16_rne(v.x) | (bf16_rne(v.y) << 16);
+  }
+  *reinterpret_cast<u4v *>(out + p16_words(p)) = u4v{w[0], w[1], w[2], w[3]};
+  out[p16_v8(p)] = __float_as_uint((float)val[kval(p, 8)]);
 }
 
 __global__ void k_zero64(int64_t n, double *x) {
@@ -590,59 +653,73 @@ namespace m3 {
 
 thread_local hipEvent_t prof_start = nullptr, prof_stop = nullptr;
 
-// threads per row for a level of n rows: one thread per row when the level
-// alone fills the GPU, four otherwise (on the 43,554-row c1 middle level,
-// 1 / 2 / 4 threads per row measured 2.78 / 2.86 / 2.95 solves/s)
-static int tpr_for(int64_t n) { return n >= 131072 ? 1 : 4; }
+// Windows of 512 rows pay once a level fills the chip with them; below, the
+// sweeps are latency-bound and the gather into LDS adds to the chain (BF16 /
+// FP64, windows of 512 against none: 92,178 rows 22.5 / 36.8 against 17.6 /
+// 42.9 us, 174,114 rows 27.1 / 74.5 against 30.3 / 89.7 us, 256,050 rows 33.9 /
+// 93.3 against 44.8 / 130 us).  Windows of 256 rows: 25.4 / 82.3 us on 174,114
+// rows, 34.1 / 102 us on 256,050.
+int sweep_window(int64_t n) { return n >= 131072 ? SW_WIN : 0; }
 
-// Workgroup of a one-thread-per-row sweep: one slice (one wave) when a
-// grid of four-slice workgroups would leave fewer than 16 per CU (c1 fine
-// level: 5,281 slices as 20-21 workgroups per CU instead of 5-6, 86.1
-// against 91.1 us; 128 threads 91.7 us), four slices otherwise (c2 fine
-// level: 619 against 681 us with one slice per workgroup)
-static inline int sweep_wg(int64_t n) { return nblk(n) < 4096 ? 64 : 256; }
-
-template <class MT, class VT, int MODE, int UNR, bool NT>
-static void launch_smooth_u(hipStream_t s, SellT<MT> K, int64_t n, const VT *x, const VT *r0, const VT *dinv,
-                            double w, VT *y, VT *r_out, VT *d_out, double *part) {
-  const int t = (MODE & 8) ? 1 : tpr_for(n);  // partial sums are indexed per workgroup (sweep_wg)
-  switch (t) {
-    case 2:
-      launch_timed(k_smooth<MT, VT, MODE, 2, UNR, NT>, dim3(nblk(2 * n)), dim3(256), s, K, n, x, r0, dinv, (VT)w,
-                   y, r_out, d_out, part);
-      break;
-    case 4:
-      launch_timed(k_smooth<MT, VT, MODE, 4, UNR, NT>, dim3(nblk(4 * n)), dim3(256), s, K, n, x, r0, dinv, (VT)w,
-                   y, r_out, d_out, part);
-      break;
-    default: {
-      const int wg = sweep_wg(n);
-      launch_timed(k_smooth<MT, VT, MODE, 1, UNR, NT>, dim3((unsigned)((n + wg - 1) / wg)), dim3(wg), s, K, n, x,
-                   r0, dinv, (VT)w, y, r_out, d_out, part);
-    }
-  }
+// do the values stay in the last-level cache (256 MB) between sweeps?
+template <class MT>
+static bool sweep_resident(const Sell &K) {
+  return (double)K.nnz * (block_value_bytes<MT>() + 2.0) < 230e6;
+}
+// workgroups of a sweep, each with its partial sum (MODE bit 8)
+template <class MT>
+static int sweep_grid(const Sell &K) {
+  if (!K.win) return (int)((K.nrow + 63) / 64);
+  return sweep_resident<MT>(K) ? (K.nwin + 7) / 8 * 8 : K.nwin;
 }
 
-// Two blocks in flight per thread (unrolling by 3 or 4 measured no faster on
-// the c1 fine level with nine separate value loads per block); three with the
-// packed FP32 values (c1 fine sweep 95.2 / 91.0 / 93.4 us for 2 / 3 / 4).  Streaming loads of the matrix on the fine level (3-4%
-// faster there, 5% less HBM traffic); the middle levels' matrices stay
-// cache-resident between sweeps and keep cached loads (streaming loads made
-// them 10-28% slower).  Remapping blocks so that each XCD sweeps one
-// contiguous row range measured 2x slower and is not used.
+// one sweep: the values val (K.val or the packed BF16 copy) on K's pattern
 template <class MT, class VT, int MODE>
-static void launch_smooth(hipStream_t s, SellT<MT> K, int64_t n, const VT *x, const VT *r0, const VT *dinv,
-                          double w, VT *y, VT *r_out, VT *d_out, double *part) {
-  if (n >= 131072)
-    launch_smooth_u<MT, VT, MODE, std::is_same<MT, B16P>::value ? 3 : 2, true>(s, K, n, x, r0, dinv, w, y, r_out,
-                                                                             d_out, part);
+static void launch_sweep(hipStream_t s, const Sell &K, const MT *val, const SweepVec<VT> &v) {
+  const SweepPat P = K.sweep();
+  if (K.win) {
+    constexpr int UNR = std::is_same<MT, double>::value ? 2 : 3;
+    const unsigned lds = (unsigned)(3 * ((size_t)K.umax + SW_WIN) * sizeof(VT));
+    auto go = [&](auto kern) {
+      if (lds > 64 * 1024)
+        HIPCHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)lds));
+      launch_timed_lds(kern, dim3((unsigned)sweep_grid<MT>(K)), dim3(64 * SW_NW), lds, s, P, K.nwin, K.umax, val, v);
+    };
+    if (sweep_resident<MT>(K)) go(k_sweep_win<MT, VT, MODE, UNR, true>);
+    else go(k_sweep_win<MT, VT, MODE, UNR, false>);
+  } else {
+    launch_timed(k_sweep<MT, VT, MODE, 16, 2>, dim3((unsigned)P.nsl), dim3(64 * 16), s, P, val, v);
+  }
+}
+void to_places(hipStream_t s, const LevelDev &lv, const double *x, double *y) {
+  const int64_t n3 = 3 * lv.nnod;
+  if (lv.K.vperm_p())
+    hipLaunchKernelGGL(k_to_places, dim3(nblk(n3)), dim3(256), 0, s, n3, lv.K.vperm_p(), x, y);
   else
-    launch_smooth_u<MT, VT, MODE, 2, false>(s, K, n, x, r0, dinv, w, y, r_out, d_out, part);
+    copy(s, x, y, n3);
+}
+void to_nodes(hipStream_t s, const LevelDev &lv, const double *x, double *y) {
+  const int64_t n3 = 3 * lv.nnod;
+  if (lv.K.vperm_p())
+    hipLaunchKernelGGL(k_to_nodes, dim3(nblk(n3)), dim3(256), 0, s, n3, lv.K.vperm_p(), x, y);
+  else
+    copy(s, x, y, n3);
 }
 
 void spmv_K(hipStream_t s, LevelDev &lv, const double *x, double *y) {
-  launch_smooth<double, double, 1>(s, lv.K.view(), lv.nnod, x, nullptr, nullptr, 0.0, y, nullptr, nullptr,
-                                   nullptr);
+  SweepVec<double> v{};
+  v.x = x;
+  v.y = y;
+  if (!lv.K.vperm_p()) {
+    launch_sweep<double, double, 1>(s, lv.K, lv.K.val.p, v);
+    return;
+  }
+  to_places(s, lv, x, lv.r0.p);
+  v.x = lv.r0.p;
+  v.y = lv.r1.p;
+  launch_sweep<double, double, 1>(s, lv.K, lv.K.val.p, v);
+  to_nodes(s, lv, lv.r1.p, y);
 }
 
 void spmv_G(hipStream_t s, Sell &G, const double *q, double *y, const double *mask) {
@@ -657,11 +734,11 @@ void spmv_M(hipStream_t s, Sell &M, const double *x, double *y) {
 }
 void prolong(hipStream_t s, LevelDev &fine, const double *dc, const double *dd, double *df) {
   hipLaunchKernelGGL((k_prolong<double, double>), dim3(nblk(fine.nnod)), dim3(256), 0, s, fine.nnod,
-                     fine.P_ptr.p, fine.P_col.p, fine.P_val.p, fine.mask.p, dc, dd, df);
+                     fine.P_ptr.p, fine.P_col.p, fine.P_val.p, fine.vmask.p, dc, dd, df);
 }
 void restrict_(hipStream_t s, LevelDev &fine, LevelDev &coarse, const double *rf, double *rc) {
   hipLaunchKernelGGL((k_restrict<double, double>), dim3(nblk(16 * coarse.nnod)), dim3(256), 0, s,
-                     coarse.nnod, fine.R_ptr.p, fine.R_col.p, fine.R_val.p, coarse.mask.p, rf, rc,
+                     coarse.nnod, fine.R_ptr.p, fine.R_col.p, fine.R_val.p, coarse.vmask.p, rf, rc,
                      (const double *)nullptr, 0.0, (double *)nullptr);
 }
 
@@ -670,10 +747,9 @@ static void add_scalar_impl(hipStream_t s, double *a, double v, int64_t n) {
 }
 
 // --------------------------------------------------------------------------------
-// V-cycle.  FP64: vectors double, matrices double.  Mixed: the residual is
-// converted to FP32, the cycle runs in FP32 with FP32 values on the finest
-// two levels... (levels >= 1 use BF16 values when bf16 copies exist), and the
-// defect is converted back to FP64.
+// V-cycle.  FP64: vectors and matrices double.  Mixed: the residual is
+// converted to FP32, the cycle runs in FP32 on the packed BF16 values (the
+// coarsest solve in FP64 on FP32 tiles), and the defect is converted back.
 // --------------------------------------------------------------------------------
 static const double WDOWN1[3] = {0.9, 0.4, 0.25}, WUP1[3] = {0.25, 0.4, 0.9};
 static const double WDOWN[3] = {0.25, 0.4, 0.9}, WUP[3] = {0.9, 0.4, 0.25};
@@ -691,28 +767,34 @@ static VecSet<float> vecs32(LevelDev &l) {
   return VecSet<float>{l.r0f.p, l.r1f.p, l.df.p, l.dnf.p, l.ddf.p, l.rrf.p, l.dinv32.p};
 }
 
+template <class MT>
+static const MT *level_values(const LevelDev &lv) {
+  if constexpr (std::is_same<MT, double>::value) return lv.K.val.p;
+  else return reinterpret_cast<const MT *>(lv.K.val16.p);
+}
+
 template <class MT, class VT>
-static void sweep(hipStream_t s, SellT<MT> K, int64_t n, const VT *x, const VT *r0, const VT *dinv,
-                  double w, VT *r_out, VT *d_out) {
-  if (d_out)
-    launch_smooth<MT, VT, 6>(s, K, n, x, r0, dinv, w, (VT *)nullptr, r_out, d_out, (double *)nullptr);
-  else
-    launch_smooth<MT, VT, 2>(s, K, n, x, r0, dinv, w, (VT *)nullptr, r_out, (VT *)nullptr, (double *)nullptr);
+static void sweep(hipStream_t s, const LevelDev &lv, const VT *x, const VT *r0, const VT *dinv, double w, VT *r_out,
+                  VT *d_out) {
+  SweepVec<VT> v{x, r0, dinv, (VT)w, nullptr, r_out, d_out, nullptr};
+  if (d_out) launch_sweep<MT, VT, 6>(s, lv.K, level_values<MT>(lv), v);
+  else launch_sweep<MT, VT, 2>(s, lv.K, level_values<MT>(lv), v);
 }
 
 // Algorithmic bytes (each stored array once, perfect reuse of the gathered
 // vector) of the V-cycle kernels, for the profile:
-//   sweep: every stored 3x3 block (values + int32 column), the row lengths,
-//          and nvec vectors of 3 components;
+//   sweep: every stored 3x3 block (values and int32 column, or two-byte place
+//          in the window), the row lengths, and nvec vectors of 3 components;
 //   restriction / prolongation: the weights and columns, the row pointers,
 //          the mask, the gathered vector once and the vectors read / written.
 template <class MT>
 static double sweep_bytes(const LevelDev &lv, int nvec, size_t vt) {
-  return (double)lv.K.nnz * (block_value_bytes<MT>() + 4.0) + 4.0 * lv.nnod + 3.0 * lv.nnod * nvec * vt;
+  return (double)lv.K.nnz * (block_value_bytes<MT>() + (lv.K.win ? 2.0 : 4.0)) + 4.0 * lv.nnod +
+         3.0 * lv.nnod * nvec * vt;
 }
 
-template <class VT, class Pick>
-static void vcycle_impl(m3_ctx *c, Pick pick_K, VecSet<VT> (*vs)(LevelDev &)) {
+template <class MT, class VT>
+static void vcycle_impl(m3_ctx *c, VecSet<VT> (*vs)(LevelDev &)) {
   hipStream_t s = c->stream;
   const int nm = c->nmg;
   const int pk = std::is_same<VT, double>::value ? 0 : 1;  // profile kind of the fine fused sweeps
@@ -725,28 +807,25 @@ static void vcycle_impl(m3_ctx *c, Pick pick_K, VecSet<VT> (*vs)(LevelDev &)) {
     // level 0: r0 and d = w1 Dinv r0 were written by k_entry
     // d (= w1 Dinv r0) is in v.d; rr = r0 is kept (v.r0 not overwritten)
     const int kind = l == 0 ? pk : 2;
-    pick_K(l, [&](auto K) {
-      using MT = std::remove_pointer_t<decltype(K.val)>;
-      const double b6 = sweep_bytes<MT>(lv, 4, sv), b2 = sweep_bytes<MT>(lv, 3, sv);
-      { ProfScope ps(c, kind, true, b6); sweep(s, K, lv.nnod, v.d, v.r0, v.dinv, wd[1], (VT *)nullptr, v.dn); }
-      { ProfScope ps(c, kind, true, b6); sweep(s, K, lv.nnod, v.dn, v.r0, v.dinv, wd[2], (VT *)nullptr, v.dd); }
-      { ProfScope ps(c, 2, true, b2); sweep(s, K, lv.nnod, v.dd, v.r0, v.dinv, 0.0, v.r1, (VT *)nullptr); }
-    });
+    const double b6 = sweep_bytes<MT>(lv, 4, sv), b2 = sweep_bytes<MT>(lv, 3, sv);
+    { ProfScope ps(c, kind, true, b6); sweep<MT, VT>(s, lv, v.d, v.r0, v.dinv, wd[1], nullptr, v.dn); }
+    { ProfScope ps(c, kind, true, b6); sweep<MT, VT>(s, lv, v.dn, v.r0, v.dinv, wd[2], nullptr, v.dd); }
+    { ProfScope ps(c, 2, true, b2); sweep<MT, VT>(s, lv, v.dd, v.r0, v.dinv, 0.0, v.r1, nullptr); }
     LevelDev &cl = c->L[l + 1];
     VecSet<VT> vc = vs(cl);
     const bool coarsest = (l + 1 == nm - 1);
     const double rb = (double)lv.R_col.n * (sv + 4.0) + (cl.nnod + 1.0) * sizeof(*lv.R_ptr.p) +
-                      3.0 * cl.nnod * 8.0 + 3.0 * lv.nnod * sv + 3.0 * cl.nnod * sv * (coarsest ? 1 : 3);
+                      3.0 * cl.nnod + 3.0 * lv.nnod * sv + 3.0 * cl.nnod * sv * (coarsest ? 1 : 3);
     ProfScope ps(c, 2, true, rb);
     if constexpr (std::is_same<VT, double>::value)
       launch_timed(k_restrict<double, double>, dim3(nblk(16 * cl.nnod)), dim3(256), s, (int64_t)cl.nnod,
                    (const int64_t *)lv.R_ptr.p, (const int32_t *)lv.R_col.p, (const double *)lv.R_val.p,
-                   (const double *)cl.mask.p, (const double *)v.r1, vc.r0,
+                   (const uint8_t *)cl.vmask.p, (const double *)v.r1, vc.r0,
                    coarsest ? (const double *)nullptr : vc.dinv, WDOWN[0], coarsest ? (double *)nullptr : vc.d);
     else
       launch_timed(k_restrict<float, float>, dim3(nblk(16 * cl.nnod)), dim3(256), s, (int64_t)cl.nnod,
                    (const int64_t *)lv.R_ptr.p, (const int32_t *)lv.R_col.p, (const float *)lv.R_val32.p,
-                   (const double *)cl.mask.p, (const float *)v.r1, vc.r0,
+                   (const uint8_t *)cl.vmask.p, (const float *)v.r1, vc.r0,
                    coarsest ? (const float *)nullptr : vc.dinv, (float)WDOWN[0], coarsest ? (float *)nullptr : vc.d);
   }
   // coarsest: FP64 Cholesky
@@ -766,25 +845,22 @@ static void vcycle_impl(m3_ctx *c, Pick pick_K, VecSet<VT> (*vs)(LevelDev &)) {
     // the level's result in d
     {
       const double pb = (double)lv.P_col.n * (sv + 4.0) + (lv.nnod + 1.0) * sizeof(*lv.P_ptr.p) +
-                        3.0 * lv.nnod * 8.0 + 3.0 * cl.nnod * sv + 3.0 * lv.nnod * sv * 2;
+                        3.0 * lv.nnod + 3.0 * cl.nnod * sv + 3.0 * lv.nnod * sv * 2;
       ProfScope ps(c, 2, true, pb);
       if constexpr (std::is_same<VT, double>::value)
         launch_timed(k_prolong<double, double>, dim3(nblk(lv.nnod)), dim3(256), s, (int64_t)lv.nnod,
                      (const int64_t *)lv.P_ptr.p, (const int32_t *)lv.P_col.p, (const double *)lv.P_val.p,
-                     (const double *)lv.mask.p, (const double *)vc.d, (const double *)v.dd, v.dn);
+                     (const uint8_t *)lv.vmask.p, (const double *)vc.d, (const double *)v.dd, v.dn);
       else
         launch_timed(k_prolong<float, float>, dim3(nblk(lv.nnod)), dim3(256), s, (int64_t)lv.nnod,
                      (const int64_t *)lv.P_ptr.p, (const int32_t *)lv.P_col.p, (const float *)lv.P_val32.p,
-                     (const double *)lv.mask.p, (const float *)vc.d, (const float *)v.dd, v.dn);
+                     (const uint8_t *)lv.vmask.p, (const float *)vc.d, (const float *)v.dd, v.dn);
     }
     const int kind = l == 0 ? pk : 2;
-    pick_K(l, [&](auto K) {
-      using MT = std::remove_pointer_t<decltype(K.val)>;
-      const double b6 = sweep_bytes<MT>(lv, 4, sv);
-      { ProfScope ps(c, kind, true, b6); sweep(s, K, lv.nnod, v.dn, v.r0, v.dinv, wu[0], (VT *)nullptr, v.d); }
-      { ProfScope ps(c, kind, true, b6); sweep(s, K, lv.nnod, v.d, v.r0, v.dinv, wu[1], (VT *)nullptr, v.dn); }
-      { ProfScope ps(c, kind, true, b6); sweep(s, K, lv.nnod, v.dn, v.r0, v.dinv, wu[2], (VT *)nullptr, v.d); }
-    });
+    const double b6 = sweep_bytes<MT>(lv, 4, sv);
+    { ProfScope ps(c, kind, true, b6); sweep<MT, VT>(s, lv, v.dn, v.r0, v.dinv, wu[0], nullptr, v.d); }
+    { ProfScope ps(c, kind, true, b6); sweep<MT, VT>(s, lv, v.d, v.r0, v.dinv, wu[1], nullptr, v.dn); }
+    { ProfScope ps(c, kind, true, b6); sweep<MT, VT>(s, lv, v.dn, v.r0, v.dinv, wu[2], nullptr, v.d); }
   }
 }
 
@@ -798,7 +874,7 @@ void vcycle(m3_ctx *c, const double *r, double *d, int precision) {
       launch_timed(k_entry<double>, dim3(nblk(n3)), dim3(256), s, n3, r, (const double *)f.dinv.p, WDOWN1[0],
                    f.r0.p, f.d.p);
     }
-    vcycle_impl<double>(c, [&](int l, auto fn) { fn(c->L[l].K.view()); }, vecs64);
+    vcycle_impl<double, double>(c, vecs64);
     ProfScope ps(c, 2, true, n3 * 16.0);
     launch_timed(k_copy, dim3(nblk(n3)), dim3(256), s, n3, (const double *)f.d.p, d);
   } else {
@@ -807,17 +883,7 @@ void vcycle(m3_ctx *c, const double *r, double *d, int precision) {
       launch_timed(k_entry<float>, dim3(nblk(n3)), dim3(256), s, n3, r, (const float *)f.dinv32.p,
                    (float)WDOWN1[0], f.r0f.p, f.df.p);
     }
-    vcycle_impl<float>(
-        c,
-        [&](int l, auto fn) {
-          if (l == 0) {
-            Sell &K = c->L[0].K;
-            fn(SellT<B16P>{K.slice_ptr.p, K.rowlen.p, K.col.p, reinterpret_cast<B16P *>(K.val32.p), K.nslot,
-                           K.perm_p(), K.ipos_p()});
-          }
-          else fn(c->L[l].K.view16());
-        },
-        vecs32);
+    vcycle_impl<B16P, float>(c, vecs32);
     ProfScope ps(c, 2, true, n3 * 12.0);
     launch_timed(k_convert<float, double>, dim3(nblk(n3)), dim3(256), s, n3, (const float *)f.df.p, d);
   }
@@ -833,19 +899,10 @@ void build_mixed(m3_ctx *c) {
   };
   for (int l = 0; l < c->nmg; ++l) {
     LevelDev &lv = c->L[l];
-    const int64_t nv = 9 * lv.K.nslot;
     const int64_t n3 = 3 * lv.nnod;
-    if (l < c->nmg - 1) {
-      if (l == 0) {  // packed BF16 groups (B16P) for the finest level's sweeps
-        if (!c->pack16_fresh) {
-          fit(lv.K.val32, 6 * lv.K.nslot);
-          hipLaunchKernelGGL(k_pack16, dim3(nblk(lv.K.nslot)), dim3(256), 0, s, lv.K.nslot, lv.K.val.p,
-                             lv.K.col.p, lv.K.val32.p);
-        }
-      } else {
-        fit(lv.K.val16, nv);
-        hipLaunchKernelGGL(k_to_bf16, dim3(nblk(nv)), dim3(256), 0, s, nv, lv.K.val.p, lv.K.val16.p);
-      }
+    if (l < c->nmg - 1 && !(l == 0 && c->pack16_fresh)) {  // packed BF16 groups for the sweeps
+      fit(lv.K.val16, P16 * lv.K.nslot);
+      hipLaunchKernelGGL(k_pack16, dim3(nblk(lv.K.nslot)), dim3(256), 0, s, lv.K.nslot, lv.K.val.p, lv.K.val16.p);
     }
     fit(lv.dinv32, n3);
     hipLaunchKernelGGL((k_convert<double, float>), dim3(nblk(n3)), dim3(256), 0, s, n3, lv.dinv.p,
@@ -934,14 +991,18 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
   const double nfree = (double)f.nfree;
   double *r = c->cg_r.p, *rl = c->cg_rlast.p, *d = c->cg_d.p, *q = c->cg_q.p, *Kq = c->cg_Kq.p;
   const int nb = red_blocks(n3);
+  const int32_t *perm = f.K.vperm_p();
+  double *xi = perm ? c->cg_x.p : x;  // the iterate in vector order
   // r = b - K x  (masked: fixed entries of b are zeroed); a caller that
   // passes x = 0 (x_zero) gets r = b without the product, the same values
   if (x_zero) {
-    hipLaunchKernelGGL(k_scale_mask, dim3(nblk(n3)), dim3(256), 0, s, n3, b, f.mask.p, r);
+    hipLaunchKernelGGL(k_rhs_in, dim3(nblk(n3)), dim3(256), 0, s, n3, perm, f.vmask.p, b, r);
+    if (perm) hipLaunchKernelGGL(k_zero64, dim3(nblk(n3)), dim3(256), 0, s, n3, xi);
   } else {
-    hipLaunchKernelGGL(k_scale_mask, dim3(nblk(n3)), dim3(256), 0, s, n3, b, f.mask.p, c->cg_b.p);
-    launch_smooth<double, double, 2>(s, f.K.view(), f.nnod, x, c->cg_b.p, (const double *)nullptr, 0.0,
-                                     (double *)nullptr, r, (double *)nullptr, (double *)nullptr);
+    hipLaunchKernelGGL(k_rhs_in, dim3(nblk(n3)), dim3(256), 0, s, n3, perm, f.vmask.p, b, c->cg_b.p);
+    if (perm) to_places(s, f, x, xi);
+    SweepVec<double> v{xi, c->cg_b.p, nullptr, 0.0, nullptr, r, nullptr, nullptr};
+    launch_sweep<double, double, 2>(s, f.K, f.K.val.p, v);
   }
   hipLaunchKernelGGL(k_dot, dim3(nb), dim3(RB), 0, s, n3, r, r, c->partial.p);
   hipLaunchKernelGGL(k_sum, dim3(1), dim3(RB), 0, s, c->partial.p, nb, c->scal.p + 5);
@@ -952,8 +1013,7 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
   if (!is_abs) tol = tol * rrms;
   if (hist) hist->push_back(rrms);
   int it = 0;
-  const int wgK = sweep_wg(f.nnod);  // partial sums of the K q product, one per workgroup of its launch
-  const unsigned gK = (unsigned)((f.nnod + wgK - 1) / wgK);
+  const int gK = sweep_grid<double>(f.K);  // partial sums of the K q product, one per workgroup of its launch
   hipLaunchKernelGGL(k_zero64, dim3(nblk(n3)), dim3(256), 0, s, n3, q);  // q = d + 0 q on the first step
   for (it = 1; it <= itmax; ++it) {
     vcycle(c, r, d, precision);
@@ -961,11 +1021,10 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
                        c->partial.p, nb);
     hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(RB), 0, s, c->partial.p, nb, c->scal.p, it == 1 ? 1 : 0);
     hipLaunchKernelGGL(k_cg_dir, dim3(nblk(n3)), dim3(256), 0, s, n3, d, q, c->scal.p);
-    launch_smooth<double, double, 9>(s, f.K.view(), f.nnod, q, (const double *)nullptr,
-                                     (const double *)nullptr, 0.0, Kq, (double *)nullptr, (double *)nullptr,
-                                     c->partial.p);
+    SweepVec<double> v{q, nullptr, nullptr, 0.0, Kq, nullptr, nullptr, c->partial.p};
+    launch_sweep<double, double, 9>(s, f.K, f.K.val.p, v);
     double *upart = c->partial.p + c->partial.n / 2;  // the SpMV's partials stay readable
-    hipLaunchKernelGGL(k_cg_alpha_update, dim3(nb), dim3(RB), 0, s, n3, x, q, r, rl, Kq, c->partial.p, (int)gK,
+    hipLaunchKernelGGL(k_cg_alpha_update, dim3(nb), dim3(RB), 0, s, n3, xi, q, r, rl, Kq, c->partial.p, gK,
                        c->scal.p, upart);
     hipLaunchKernelGGL(k_sum, dim3(1), dim3(RB), 0, s, upart, nb, c->scal.p + 5);
     HIPCHECK(hipMemcpyAsync(c->h_scal + 5, c->scal.p + 5, sizeof(double), hipMemcpyDeviceToHost, s));
@@ -975,6 +1034,7 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
     if (std::isnan(rrms)) throw M3Error(M3_E_NUMERIC, "NaN in CG residual");
     if (rrms < tol) break;
   }
+  if (perm) to_nodes(s, f, xi, x);
   HIPCHECK(hipGetLastError());
   return it > itmax ? itmax : it;
 }

@@ -20,7 +20,7 @@ void chol_analyse(m3_ctx *c);
 
 // ------------------------------------------------------------------ Sell build
 void Sell::build(int64_t nrow_, int64_t ncol_, const std::vector<int64_t> &ptr,
-                 const std::vector<int32_t> &cols, int bs_, int sigma) {
+                 const std::vector<int32_t> &cols, int bs_, const std::vector<int32_t> *place) {
   nrow = nrow_;
   ncol = ncol_;
   bs = bs_;
@@ -30,15 +30,12 @@ void Sell::build(int64_t nrow_, int64_t ncol_, const std::vector<int64_t> &ptr,
   for (int64_t r = 0; r < nrow; ++r) h_rowlen[r] = (int32_t)(ptr[r + 1] - ptr[r]);
   h_perm.clear();
   h_ipos.clear();
-  if (sigma > 0) {
-    h_perm.resize(nrow);
+  h_vperm.clear();
+  h_vpos.clear();
+  win = 0;
+  if (place) {
+    h_perm = *place;
     h_ipos.resize(nrow);
-    for (int64_t r = 0; r < nrow; ++r) h_perm[r] = (int32_t)r;
-    for (int64_t w0 = 0; w0 < nrow; w0 += sigma) {
-      const int64_t w1 = std::min(nrow, w0 + sigma);
-      std::stable_sort(h_perm.begin() + w0, h_perm.begin() + w1,
-                       [&](int32_t a, int32_t b) { return h_rowlen[a] > h_rowlen[b]; });
-    }
     for (int64_t q = 0; q < nrow; ++q) h_ipos[h_perm[q]] = (int32_t)q;
   }
   auto row_at = [&](int64_t q) { return h_perm.empty() ? q : (int64_t)h_perm[q]; };
@@ -64,7 +61,132 @@ void Sell::build(int64_t nrow_, int64_t ncol_, const std::vector<int64_t> &ptr,
   val.alloc((size_t)nslot * bs);
 }
 
+bool Sell::build_windows(const std::vector<int32_t> &order, int w, int cap) {
+  const int64_t nw = (nrow + w - 1) / w;
+  std::vector<std::vector<int32_t>> lists(nw);
+  std::vector<uint16_t> h_idx((size_t)nslot, 0);
+  std::vector<int32_t> h_plen(nrow), pos(nrow);
+  std::vector<uint16_t> h_lrow(nrow);
+  for (int64_t i = 0; i < nrow; ++i) pos[order[i]] = (int32_t)i;
+  bool fits = true;
+#pragma omp parallel reduction(&& : fits)
+  {
+    std::vector<int32_t> seen(ncol, -1), at(ncol);  // last window that holds an entry, its place there
+#pragma omp for schedule(dynamic, 4)
+    for (int64_t b = 0; b < nw; ++b) {
+      std::vector<int32_t> &L = lists[b];
+      const int64_t q0 = b * w, q1 = std::min(nrow, q0 + w);
+      auto each = [&](auto fn) {
+        for (int64_t q = q0; q < q1; ++q) {
+          const int len = h_rowlen[h_perm[q]];
+          const int64_t base = h_slice_ptr[q >> 6] + (q & 63);
+          h_plen[q] = len;
+          h_lrow[q] = (uint16_t)(pos[h_perm[q]] - q0);
+          for (int k = 0; k < len; ++k) fn(base + 64 * (int64_t)k, pos[h_col[base + 64 * (int64_t)k]]);
+        }
+      };
+      each([&](int64_t, int32_t i) {
+        if (seen[i] != (int32_t)b) {
+          seen[i] = (int32_t)b;
+          L.push_back(i);
+        }
+      });
+      std::sort(L.begin(), L.end());
+      for (size_t i = 0; i < L.size(); ++i) at[L[i]] = (int32_t)i;
+      if ((int64_t)L.size() > cap) fits = false;
+      else each([&](int64_t slot, int32_t i) { h_idx[slot] = (uint16_t)at[i]; });
+    }
+  }
+  if (!fits) return false;
+  std::vector<int32_t> h_lptr(nw + 1, 0), h_list;
+  umax = 0;
+  for (int64_t b = 0; b < nw; ++b) {
+    umax = std::max(umax, (int)lists[b].size());
+    h_lptr[b + 1] = h_lptr[b] + (int32_t)lists[b].size();
+  }
+  h_list.reserve(h_lptr[nw]);
+  for (const auto &L : lists) h_list.insert(h_list.end(), L.begin(), L.end());
+  win = w;
+  nwin = (int)nw;
+  plen.upload(h_plen);
+  lptr.upload(h_lptr);
+  list.upload(h_list);
+  idx.upload(h_idx);
+  lrow.upload(h_lrow);
+  h_vperm = order;
+  h_vpos.swap(pos);
+  vperm.upload(h_vperm);
+  vpos.upload(h_vpos);
+  return true;
+}
+
 namespace {
+
+// The nodes along a Hilbert curve of their coordinates (J. Skilling,
+// "Programming the Hilbert curve", AIP Conf. Proc. 707, 2004: axes to the
+// transposed Hilbert integer), 16 bits an axis; equal keys in index order.
+std::vector<int32_t> hilbert_order(const double *X, int64_t n) {
+  double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+  for (int64_t i = 0; i < n; ++i)
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = std::min(lo[k], X[3 * i + k]);
+      hi[k] = std::max(hi[k], X[3 * i + k]);
+    }
+  const double w = std::max({hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]});
+  constexpr int BITS = 16;
+  std::vector<std::pair<uint64_t, int32_t>> key(n);
+#pragma omp parallel for schedule(static)
+  for (int64_t i = 0; i < n; ++i) {
+    uint32_t x[3];
+    for (int k = 0; k < 3; ++k) x[k] = w > 0 ? (uint32_t)((X[3 * i + k] - lo[k]) / w * 65535.0) : 0u;
+    for (uint32_t q = 1u << (BITS - 1); q > 1; q >>= 1) {
+      const uint32_t m = q - 1;
+      for (int k = 0; k < 3; ++k) {
+        if (x[k] & q) {
+          x[0] ^= m;
+        } else {
+          const uint32_t t = (x[0] ^ x[k]) & m;
+          x[0] ^= t;
+          x[k] ^= t;
+        }
+      }
+    }
+    for (int k = 1; k < 3; ++k) x[k] ^= x[k - 1];
+    uint32_t t = 0;
+    for (uint32_t q = 1u << (BITS - 1); q > 1; q >>= 1)
+      if (x[2] & q) t ^= q - 1;
+    uint64_t code = 0;
+    for (int b = BITS - 1; b >= 0; --b)
+      for (int k = 0; k < 3; ++k) code = (code << 1) | (((x[k] ^ t) >> b) & 1u);
+    key[i] = {code, (int32_t)i};
+  }
+  // sorted in pieces, then merged pairwise
+  constexpr int PIECES = 16;
+  std::vector<int64_t> cut(PIECES + 1);
+  for (int p = 0; p <= PIECES; ++p) cut[p] = n * p / PIECES;
+#pragma omp parallel for schedule(dynamic, 1)
+  for (int p = 0; p < PIECES; ++p) std::sort(key.begin() + cut[p], key.begin() + cut[p + 1]);
+  for (int s = 1; s < PIECES; s *= 2) {
+#pragma omp parallel for schedule(dynamic, 1)
+    for (int p = 0; p < PIECES; p += 2 * s)
+      std::inplace_merge(key.begin() + cut[p], key.begin() + cut[p + s], key.begin() + cut[p + 2 * s]);
+  }
+  std::vector<int32_t> order(n);
+  for (int64_t i = 0; i < n; ++i) order[i] = key[i].second;
+  return order;
+}
+
+// Placement of a level whose sweeps run on windows of w rows: the Hilbert order
+// of the nodes, longest rows first inside every window.
+std::vector<int32_t> window_placement(const std::vector<int32_t> &order, int w, const std::vector<int64_t> &ptr) {
+  std::vector<int32_t> p = order;
+  const int64_t n = (int64_t)p.size();
+#pragma omp parallel for schedule(static)
+  for (int64_t a = 0; a < n; a += w)
+    std::stable_sort(p.begin() + a, p.begin() + std::min<int64_t>(n, a + w),
+                     [&](int32_t i, int32_t j) { return ptr[i + 1] - ptr[i] > ptr[j + 1] - ptr[j]; });
+  return p;
+}
 
 using clk = std::chrono::steady_clock;
 double secs(clk::time_point a, clk::time_point b) {
@@ -260,9 +382,17 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
       std::vector<int64_t> ptr;
       std::vector<int32_t> cols;
       adjacency(lv.h_el2nod, lv.nel, lv.nnod, 10, ALL10, 10, ALL10, ptr, cols);
-      // the finest level's rows sorted by length in windows of 256 rows (the
-      // fine sweeps stream it; the coarser levels stay cache-resident)
-      lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9, l == 0 ? 256 : 0);
+      const int w = l < nmg - 1 ? m3::sweep_window(lv.nnod) : 0;
+      if (w) {
+        M3_REQUIRE(m->GCOORD, M3_E_ARG, "missing GCOORD");
+        const std::vector<int32_t> order = hilbert_order(m->GCOORD, lv.nnod), place = window_placement(order, w, ptr);
+        lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9, &place);
+        mark("level connectivity + K pattern");
+        if (!lv.K.build_windows(order, w, m3::SWEEP_CAP)) lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
+        mark("sweep windows");
+      } else {
+        lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
+      }
       if (l < nmg - 1) lv.Kel.alloc((size_t)lv.nel * KEL);
       mark("level connectivity + K pattern");
     }
@@ -394,22 +524,32 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
       std::vector<double> P_val(m->Ic2f_val[l], m->Ic2f_val[l] + nnzP);
       for (int64_t k = 0; k < nnzP; ++k)
         M3_REQUIRE(P_col[k] >= 0 && P_col[k] < cl.nnod, M3_E_MESH, "Ic2f column out of range");
-      // transpose
-      std::vector<int64_t> R_ptr(cl.nnod + 1, 0);
-      for (int64_t k = 0; k < nnzP; ++k) R_ptr[P_col[k] + 1]++;
+      // both directions in the levels' vector orders: row q of P is the node at
+      // place q of the fine level
+      const std::vector<int32_t> &fperm = fl.K.h_vperm, &cipos = cl.K.h_vpos;
+      auto fnode = [&](int64_t q) { return fperm.empty() ? q : (int64_t)fperm[q]; };
+      std::vector<int64_t> PP(fl.nnod + 1, 0), R_ptr(cl.nnod + 1, 0);
+      for (int64_t q = 0; q < fl.nnod; ++q) PP[q + 1] = PP[q] + P_ptr[fnode(q) + 1] - P_ptr[fnode(q)];
+      std::vector<int32_t> PC(nnzP), R_col(nnzP);
+      std::vector<double> PV(nnzP), R_val(nnzP);
+#pragma omp parallel for schedule(static)
+      for (int64_t q = 0; q < fl.nnod; ++q)
+        for (int64_t k = P_ptr[fnode(q)], o = PP[q]; k < P_ptr[fnode(q) + 1]; ++k, ++o) {
+          PC[o] = cipos.empty() ? P_col[k] : cipos[P_col[k]];
+          PV[o] = P_val[k];
+        }
+      for (int64_t k = 0; k < nnzP; ++k) R_ptr[PC[k] + 1]++;
       for (int64_t j = 0; j < cl.nnod; ++j) R_ptr[j + 1] += R_ptr[j];
       std::vector<int64_t> fill(R_ptr.begin(), R_ptr.end() - 1);
-      std::vector<int32_t> R_col(nnzP);
-      std::vector<double> R_val(nnzP);
       for (int64_t i = 0; i < fl.nnod; ++i)
-        for (int64_t k = P_ptr[i]; k < P_ptr[i + 1]; ++k) {
-          const int64_t q = fill[P_col[k]]++;
+        for (int64_t k = PP[i]; k < PP[i + 1]; ++k) {
+          const int64_t q = fill[PC[k]]++;
           R_col[q] = (int32_t)i;
-          R_val[q] = P_val[k];
+          R_val[q] = PV[k];
         }
-      fl.P_ptr.upload(P_ptr);
-      fl.P_col.upload(P_col);
-      fl.P_val.upload(P_val);
+      fl.P_ptr.upload(PP);
+      fl.P_col.upload(PC);
+      fl.P_val.upload(PV);
       fl.R_ptr.upload(R_ptr);
       fl.R_col.upload(R_col);
       fl.R_val.upload(R_val);
@@ -511,6 +651,12 @@ int m3_set_bc(m3_ctx *c, const int64_t *ifix, const double *vfix, int64_t nfix) 
       LevelDev &lv = c->L[l];
       std::vector<double> ml(mask.begin(), mask.begin() + 3 * lv.nnod);
       lv.mask.upload(ml);
+      std::vector<uint8_t> vm(3 * lv.nnod);
+      for (int64_t q = 0; q < lv.nnod; ++q) {
+        const int64_t r = lv.K.h_vperm.empty() ? q : (int64_t)lv.K.h_vperm[q];
+        for (int k = 0; k < 3; ++k) vm[3 * q + k] = ml[3 * r + k] != 0.0;
+      }
+      lv.vmask.upload(vm);
       lv.nfree = (int64_t)std::count(ml.begin(), ml.end(), 1.0);
     }
     c->U0.upload(U0);
@@ -1061,8 +1207,16 @@ int m3_apply(m3_ctx *c, int32_t which, int32_t level, const double *x, double *y
       case 1: m3::spmv_G(s, c->G, dx.p, dy.p, nullptr); break;
       case 2: m3::spmv_GT(s, c->GT, dx.p, dy.p); break;
       case 3: m3::spmv_M(s, c->M, dx.p, dy.p); break;
-      case 4: m3::prolong(s, lv, dx.p, nullptr, dy.p); break;
-      case 5: m3::restrict_(s, lv, c->L[level + 1], dx.p, dy.p); break;
+      case 4:  // the transfers act on vector-ordered ones
+        m3::to_places(s, c->L[level + 1], dx.p, c->L[level + 1].r0.p);
+        m3::prolong(s, lv, c->L[level + 1].r0.p, nullptr, lv.r0.p);
+        m3::to_nodes(s, lv, lv.r0.p, dy.p);
+        break;
+      case 5:
+        m3::to_places(s, lv, dx.p, lv.r0.p);
+        m3::restrict_(s, lv, c->L[level + 1], lv.r0.p, c->L[level + 1].r0.p);
+        m3::to_nodes(s, c->L[level + 1], c->L[level + 1].r0.p, dy.p);
+        break;
     }
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(s));
@@ -1078,9 +1232,14 @@ int m3_get_vector(m3_ctx *c, int32_t which, int32_t level, double *out) {
     switch (which) {
       case 0: c->Fb.download(out, 3 * c->nnod); break;
       case 1: c->bc_rhs.download(out, 3 * c->nnod); break;
-      case 2: lv.dinv.download(out, 3 * lv.nnod);
-        for (int64_t i = 0; i < 3 * lv.nnod; ++i) out[i] = 1.0 / out[i];
+      case 2: {
+        const std::vector<double> di = lv.dinv.to_host();
+        for (int64_t q = 0; q < lv.nnod; ++q) {
+          const int64_t r = lv.K.h_vperm.empty() ? q : (int64_t)lv.K.h_vperm[q];
+          for (int k = 0; k < 3; ++k) out[3 * r + k] = 1.0 / di[3 * q + k];
+        }
         break;
+      }
       case 3: lv.mask.download(out, 3 * lv.nnod); break;
       case 4: c->LiMM.download(out, c->nV);
         for (int64_t i = 0; i < c->nV; ++i) out[i] = 1.0 / out[i];
@@ -1210,7 +1369,7 @@ int m3_get_operator(m3_ctx *c, int32_t level, int64_t *rowptr, int32_t *col, dou
       for (int k = 0; k < K.h_rowlen[r]; ++k, ++q) {
         const int64_t slot = base + (int64_t)k * 64;
         col[q] = K.h_col[slot];
-        for (int e = 0; e < 9; ++e) val[9 * q + e] = v[(size_t)e * K.nslot + slot];
+        for (int e = 0; e < 9; ++e) val[9 * q + e] = v[(size_t)kval(slot, e)];
       }
       rowptr[r + 1] = q;
     }

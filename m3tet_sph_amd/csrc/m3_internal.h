@@ -90,17 +90,14 @@ struct DBuf {
 
 // Sliced (SELL-64) block-sparse storage.  Rows are grouped in slices of 64 (one
 // wavefront); inside a slice the k-th stored block of each row sits at slot
-// slice_ptr[s] + 64*k + (row % 64), so the 64 lanes of a wave touch 64
-// consecutive slots.  Block values are stored structure-of-arrays,
-// val[v*nslot + slot] for v < bs, so every value load of a wave is one
-// contiguous 512-byte (FP64) segment.  Columns inside a row are sorted.
+// slice_ptr[s] + 64*k + (position % 64), so the 64 lanes of a wave touch 64
+// consecutive slots.  Matrices with fewer than nine values per block store
+// them structure-of-arrays, val[v*nslot + slot]; the 3x3 operators store each
+// group of 64 slots contiguously (kval).  Columns inside a row are sorted.
 //
-// Rows may be placed in the slices in another order than their index (SELL-C-
-// sigma: within windows of sigma rows, longer rows first, so that the lanes
-// of a wave that run out of blocks are contiguous and their cache lines are
-// not fetched): position q of the slices holds row perm[q], row r sits at
-// position ipos[r]; both are NULL for the identity placement.  rowlen is
-// indexed by row.
+// Rows may be placed in the slices in another order than their index:
+// position q of the slices holds row perm[q], row r sits at position
+// ipos[r]; both are NULL for the identity placement.  rowlen is indexed by row.
 template <class T>
 struct SellT {
   const int64_t *slice_ptr;
@@ -112,6 +109,22 @@ struct SellT {
   const int32_t *ipos;  // row -> position (NULL: identity)
 };
 using SellView = SellT<double>;
+
+// Index of value v (row-major in the 3x3 block) of slot p in a 3x3 operator:
+// the 64 slots of a group hold their 576 doubles together, values (0,1),
+// (2,3), (4,5), (6,7) as one 16-byte pair per lane and value 8 behind them, so
+// that a wave reads a group in four 16-byte and one 8-byte load per lane from
+// one contiguous stretch
+__host__ __device__ inline int64_t kval(int64_t p, int v) {
+  const int64_t lane = p & 63;
+  return 9 * (p - lane) + (v < 8 ? 128 * (v >> 1) + 2 * lane + (v & 1) : 512 + lane);
+}
+// The same for the packed BF16 copy of the mixed V-cycle, in 32-bit words: the
+// group's 64 lanes hold (v0..v7) as four words of two BF16 each (v_2i in the
+// low half), then v8 in FP32: 20 bytes per block
+constexpr int P16 = 5;  // words per slot
+__host__ __device__ inline int64_t p16_words(int64_t p) { return P16 * (p & ~(int64_t)63) + 4 * (p & 63); }
+__host__ __device__ inline int64_t p16_v8(int64_t p) { return P16 * (p & ~(int64_t)63) + 256 + (p & 63); }
 
 // BF16 bits of x rounded to nearest even (through FP32)
 __device__ inline uint32_t bf16_rne(double x) {
@@ -127,6 +140,23 @@ __device__ inline int64_t sell_base(const SellT<T> &K, int64_t row) {
   return K.slice_ptr[q >> 6] + (q & 63);
 }
 
+// What a sweep reads of a 3x3 operator besides its values (k_sparse.hip).
+// win == 0: the rows are in index order and col holds their columns.  win > 0:
+// the vectors are in a space-filling order of the nodes, win of them per
+// window; a window's rows sit in the slices by decreasing length, lrow being a
+// position's place in the window's stretch of the vectors; window b gathers the
+// entries list[lptr[b] .. lptr[b+1]) of the vector and idx is a slot's place
+// among them.
+struct SweepPat {
+  const int64_t *slice_ptr;
+  const int32_t *len;   // stored blocks per position
+  const int32_t *col;
+  const uint16_t *idx, *lrow;
+  const int32_t *lptr, *list;
+  int64_t n;
+  int32_t nsl;          // slices
+};
+
 struct Sell {
   int64_t nrow = 0, ncol = 0, nslot = 0, nnz = 0;
   int bs = 9;  // values per stored block
@@ -136,22 +166,35 @@ struct Sell {
   DBuf<int64_t> slice_ptr;
   DBuf<int32_t> rowlen, col, perm, ipos;
   DBuf<double> val;
-  DBuf<float> val32;     // finest level: the packed BF16 values of the mixed V-cycle (6 floats per slot)
-  DBuf<uint16_t> val16;  // bf16 bit patterns
+  DBuf<uint32_t> val16;  // packed BF16 copy of the mixed V-cycle (P16 words per slot)
+  // order of the level's vectors (empty: node order): node at each place,
+  // place of each node
+  std::vector<int32_t> h_vperm, h_vpos;
+  DBuf<int32_t> vperm, vpos;
+  // windowed sweeps (SweepPat): rows per window (0: none), windows, the most
+  // vector entries that one window gathers
+  int win = 0, nwin = 0, umax = 0;
+  DBuf<int32_t> plen, lptr, list;
+  DBuf<uint16_t> idx, lrow;
   // build from sorted per-row column lists (CSR); uploads pattern, allocates
-  // val; sigma > 0 sorts the rows by decreasing length within windows of
-  // sigma rows (a multiple of 64)
+  // val.  place (may be NULL): the row at each position
   void build(int64_t nrow_, int64_t ncol_, const std::vector<int64_t> &ptr,
-             const std::vector<int32_t> &cols, int bs_, int sigma = 0);
+             const std::vector<int32_t> &cols, int bs_, const std::vector<int32_t> *place = nullptr);
+  // window lists for windows of w rows of the vector order; false (and nothing
+  // kept) if one of them gathers more than cap entries
+  bool build_windows(const std::vector<int32_t> &order, int w, int cap);
   int64_t base_of(int64_t row) const {
     const int64_t q = h_ipos.empty() ? row : (int64_t)h_ipos[row];
     return h_slice_ptr[q >> 6] + (q & 63);
   }
   const int32_t *perm_p() const { return h_perm.empty() ? nullptr : perm.p; }
   const int32_t *ipos_p() const { return h_ipos.empty() ? nullptr : ipos.p; }
+  const int32_t *vperm_p() const { return h_vperm.empty() ? nullptr : vperm.p; }
+  const int32_t *vpos_p() const { return h_vpos.empty() ? nullptr : vpos.p; }
   SellView view() { return SellView{slice_ptr.p, rowlen.p, col.p, val.p, nslot, perm_p(), ipos_p()}; }
-  SellT<uint16_t> view16() {
-    return SellT<uint16_t>{slice_ptr.p, rowlen.p, col.p, val16.p, nslot, perm_p(), ipos_p()};
+  SweepPat sweep() const {
+    return SweepPat{slice_ptr.p, win ? plen.p : rowlen.p, col.p, idx.p, lrow.p, lptr.p, list.p, nrow,
+                    (int32_t)(h_slice_ptr.size() - 1)};
   }
 };
 
@@ -217,6 +260,10 @@ struct LevelDev {
   DBuf<int32_t> el2nod;
   Sell K;                          // 3x3 blocks
   DBuf<double> mask;               // 3*nnod, 1 free / 0 fixed
+  // What the V-cycle and the CG hold of this level is in K's vector order
+  // (the node order on small levels): the vectors below, dinv, vmask (the mask,
+  // a byte per dof) and the transfers
+  DBuf<uint8_t> vmask;
   DBuf<double> dinv;               // 3*nnod inverse diagonal (1 at fixed dofs)
   DBuf<float> dinv32;
   DBuf<double> Kel;                // nel*KEL rotated + masked element matrices
@@ -230,7 +277,8 @@ struct LevelDev {
   // block) + transposed), CSR over the slots
   DBuf<int64_t> cptr;
   DBuf<int32_t> clist;
-  // transfer to this level from level+1 (fine rows) and its transpose
+  // transfer to this level from level+1 (fine rows) and its transpose, rows
+  // and columns in the two levels' vector orders
   DBuf<int64_t> P_ptr, R_ptr;
   DBuf<int32_t> P_col, R_col;
   DBuf<double> P_val, R_val;
@@ -290,7 +338,7 @@ struct m3_ctx {
   bool have_mesh = false, have_bc = false, assembled = false, restricted = false,
        factored = false, have_mixed = false, have_fields = false;
   bool g_valid = false;  // G and G' assembled for the current mesh (they depend on it alone)
-  // the finest level's packed BF16 values (K.val32) written by the slot
+  // the finest level's packed BF16 values (K.val16) written by the slot
   // gather and patched by the diagonal fix of the last assembly, so that the
   // mixed V-cycle needs no separate packing pass
   bool pack16_fresh = false;
@@ -366,13 +414,18 @@ namespace m3 {
 // interval is the kernel's execution even when the host falls behind the GPU.
 extern thread_local hipEvent_t prof_start, prof_stop;
 
-// launch, with the profiling events attached when a ProfScope set them
+// launch (with lds bytes of dynamic LDS), with the profiling events attached
+// when a ProfScope set them
+template <typename... Args, typename F = void (*)(Args...)>
+inline void launch_timed_lds(F kernel, dim3 grid, dim3 block, unsigned lds, hipStream_t s, Args... args) {
+  if (prof_start)
+    hipExtLaunchKernelGGL(kernel, grid, block, lds, s, prof_start, prof_stop, 0, args...);
+  else
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
+}
 template <typename... Args, typename F = void (*)(Args...)>
 inline void launch_timed(F kernel, dim3 grid, dim3 block, hipStream_t s, Args... args) {
-  if (prof_start)
-    hipExtLaunchKernelGGL(kernel, grid, block, 0, s, prof_start, prof_stop, 0, args...);
-  else
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, args...);
+  launch_timed_lds(kernel, grid, block, 0, s, args...);
 }
 
 // time the one launch (through launch_timed) inside the scope when profiling
@@ -421,8 +474,15 @@ void launch_diag_inv(m3_ctx *c, int l);
 void launch_lumped_mm(m3_ctx *c);
 
 // sparse kernels
+// rows per sweep window of a level of n nodes (0: no windows), and the most
+// vector entries a window may gather (96 KB of LDS in FP64)
+int sweep_window(int64_t n);
+constexpr int SWEEP_CAP = 4096;
 void nan_flag(hipStream_t s, const double *x, int64_t n, int *flag);  // atomicOr(flag, 32) on a NaN
-void spmv_K(hipStream_t s, LevelDev &lv, const double *x, double *y);
+void spmv_K(hipStream_t s, LevelDev &lv, const double *x, double *y);  // node order; lv.r0 and lv.r1 are work space
+// vectors of a level between the node order and K's vector order
+void to_places(hipStream_t s, const LevelDev &lv, const double *x, double *y);
+void to_nodes(hipStream_t s, const LevelDev &lv, const double *x, double *y);
 void spmv_G(hipStream_t s, Sell &G, const double *q, double *y, const double *mask);
 void spmv_GT(hipStream_t s, Sell &GT, const double *z, double *y);
 void spmv_M(hipStream_t s, Sell &M, const double *x, double *y);

@@ -1,0 +1,59 @@
+"""The sweeps of the multigrid levels against the stored operator: levels below
+the window size limit (one slice per workgroup, its blocks dealt to waves), and
+levels that are swept in windows, with a last window that is not full, on
+generated shells and on the unstructured mesh file.  K x, the transfers and the
+diagonal against SciPy products of m3_get_operator's matrix; one velocity solve
+in both precisions against each other."""
+import os
+
+import numpy as np
+import pytest
+
+from tests.conftest import relerr
+
+pytestmark = pytest.mark.gpu
+GOLD = os.path.join(os.path.dirname(__file__), "golden", "EarthShell_n37k.mat")
+
+# nodes of the finest level: 5,778 (a last slice of 18 rows), 92,178, 174,114
+# (a last window of 34 rows), 289,174 of the file
+CASES = [dict(level=1, nlayer=2, nmg=2), dict(level=2, nlayer=1, nmg=3), dict(level=1, nlayer=2, nmg=4), None]
+
+
+@pytest.mark.parametrize("shape", CASES, ids=["small", "direct", "windows", "file"])
+def test_level_operators(shape):
+    from m3tet_sph_amd import api, fields as F, mesh as M
+    m = M.build_from_file(GOLD, nmg=2, device=0) if shape is None else M.build_shell(**shape, device=0)
+    T = (m.r_surf - m.GCOORD_SPH[:, 2]) / (m.r_surf - m.r_cmb) + 0.03 * np.sin(7 * m.GCOORD[:, 0])
+    Visc, Dens = F.material(T, 1e3)
+    ifix, vfix = F.plate_bcs(m)
+    ctx = api.StokesContext(m)
+    try:
+        ctx.set_bc(ifix, vfix)
+        ctx.assemble(Visc, Dens, F.physics())
+        ctx.restrict_stiffmat()
+        ctx.cholesky_factorization()
+        rng = np.random.default_rng(0)
+        for l in range(m.nmg):
+            K = api.get_operator(ctx, l)
+            x = rng.standard_normal(K.shape[1])
+            # sums of at most some 100 x 3 products in another order: n eps = 7e-14 at worst
+            assert relerr(ctx.apply(0, l, x), K @ x) < 1e-13
+            assert relerr(ctx.get_vector(2, l), K.diagonal()) < 1e-15
+            assert abs(K - K.T).max() <= 1e-12 * abs(K).max()
+        for l in range(m.nmg - 1):
+            P = api.intermesh_transfer_matrix(m, l)
+            mf, mc = ctx.get_vector(3, l), ctx.get_vector(3, l + 1)
+            xc, xf = rng.standard_normal(P.shape[1]), rng.standard_normal(P.shape[0])
+            assert relerr(ctx.apply(4, l, xc), mf * (P @ xc)) < 1e-13
+            assert relerr(ctx.apply(5, l, xf), mc * (P.T @ xf)) < 1e-13
+        b = ctx.get_vector(0) - ctx.get_vector(1)
+        x64, n64, _ = ctx.mgpcg(b, tol=1e-9, is_abs_tol=False, itmax=60)
+        x16, n16, _ = ctx.mgpcg(b, x=0.3 * x64, tol=1e-9, is_abs_tol=False, itmax=60, precision="mixed")
+        K0, free = api.get_operator(ctx, 0), ctx.get_vector(3, 0)
+        for x in (x64, x16):
+            r = free * (b - K0 @ x)
+            assert np.linalg.norm(r) < 2e-9 * np.linalg.norm(free * b)
+        # both stop at the same residual; the operator's conditioning is below 1e5 here
+        assert relerr(x16, x64) < 1e-4 and abs(n64 - n16) <= 3
+    finally:
+        ctx.close()
