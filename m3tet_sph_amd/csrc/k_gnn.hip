@@ -4,14 +4,11 @@
 //
 // Layout in HBM: vertex-major rows, h[i*64 + c] (BF16 bit patterns) for the
 // activations, FP32 for features, targets, gradients and parameters.  The
-// dense layers keep one output column per lane and that column of the weight
-// matrix in registers (128 VGPRs for a message-passing layer); the row
-// operand is broadcast from the lane that loaded it (v_readlane), so a wave
-// streams its rows from HBM once and never touches LDS.  Weight gradients
-// are block partial sums over row chunks (rows staged in LDS) followed by a
-// fixed-order reduction, which makes the gradient deterministic.  Every
-// product-accumulate is an FMA in a fixed order (bias first, then input
-// index ascending), which the CPU restatement follows.
+// dense layers run on the FP32 matrix cores with the weights in registers;
+// weight gradients are partial sums over row chunks followed by a fixed-order
+// reduction, which makes the gradient deterministic.  Every product-accumulate
+// of the forward pass is an FMA in a fixed order (bias first, then input index
+// ascending), which the CPU restatement follows.
 #include "m3_internal.h"
 
 #include <algorithm>
@@ -35,8 +32,6 @@ __device__ inline uint16_t f2bf(float f) {  // round to nearest even
   return (uint16_t)(u >> 16);
 }
 __device__ inline float bf2f(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
-__device__ inline float ld(const float *p) { return *p; }
-__device__ inline float ld(const uint16_t *p) { return bf2f(*p); }
 __device__ inline float lanebc(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
@@ -46,23 +41,24 @@ inline int nblk(int64_t n) { return (int)((n + 255) / 256); }
 // ---------------------------------------------------------------- features
 // s_u, s_p: RMS vertex speed and pressure of the base state; s_T: RMS of the
 // temperature's departure from the base state's temperature
-// (one workgroup of SCB threads: a fixed summation order, so the scales do
-// not depend on the launch)
-constexpr int SCB = 1024;
-__global__ __launch_bounds__(SCB) void k_scales(int64_t n, const double *U, const double *P, const double *T,
-                                                const double *Tb, double *sc) {
+// (SCB workgroups of 256 threads each, then one that adds their sums in order:
+// the summation order depends on n alone, so the scales do not depend on the
+// launch; one workgroup for all vertices took 28 us at 43,554 vertices, this 6.5)
+constexpr int SCB = 64;
+__global__ __launch_bounds__(256) void k_scales(int64_t n, const double *U, const double *P, const double *T,
+                                                const double *Tb, double *part) {
   double su = 0, sp = 0, st = 0;
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+  for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += 256 * SCB) {
     su += U[3 * i] * U[3 * i] + U[3 * i + 1] * U[3 * i + 1] + U[3 * i + 2] * U[3 * i + 2];
     sp += P[i] * P[i];
     st += (T[i] - Tb[i]) * (T[i] - Tb[i]);
   }
-  __shared__ double a[SCB], b[SCB], c[SCB];
+  __shared__ double a[256], b[256], c[256];
   a[threadIdx.x] = su;
   b[threadIdx.x] = sp;
   c[threadIdx.x] = st;
   __syncthreads();
-  for (int o = SCB / 2; o > 0; o >>= 1) {
+  for (int o = 128; o > 0; o >>= 1) {
     if ((int)threadIdx.x < o) {
       a[threadIdx.x] += a[threadIdx.x + o];
       b[threadIdx.x] += b[threadIdx.x + o];
@@ -71,11 +67,18 @@ __global__ __launch_bounds__(SCB) void k_scales(int64_t n, const double *U, cons
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    const double u = sqrt(a[0] / (double)n), p = sqrt(b[0] / (double)n), t = sqrt(c[0] / (double)n);
-    sc[0] = u > 0 ? u : 1.0;
-    sc[1] = p > 0 ? p : 1.0;
-    sc[2] = t > 0 ? t : 1.0;
+    part[blockIdx.x] = a[0];
+    part[SCB + blockIdx.x] = b[0];
+    part[2 * SCB + blockIdx.x] = c[0];
   }
+}
+__global__ __launch_bounds__(64) void k_scales_fin(int64_t n, const double *part, double *sc) {
+  if (threadIdx.x >= 3) return;
+  double s = 0;
+#pragma unroll 8
+  for (int j = 0; j < SCB; ++j) s += part[SCB * threadIdx.x + j];
+  const double u = sqrt(s / (double)n);
+  sc[threadIdx.x] = u > 0 ? u : 1.0;
 }
 
 __global__ void k_features(int64_t n, const double *T, const double *Tp, const double *visc, const double *U,
@@ -127,78 +130,137 @@ __global__ void k_chan_stats(int64_t rows, const float *X, int C, double *part) 
 }
 
 // ---------------------------------------------------------------- forward
-// h0 = relu(xn We + be), xn = (x - mu) / sigma; one wave per vertex, lane = column
+// h0 = relu(xn We + be), xn = (x - mu) / sigma; one wave per vertex, lane =
+// column; a lane normalises one feature and the wave broadcasts them
 __global__ __launch_bounds__(256) void k_enc(int64_t n, const float *X, const float *norm, const float *prm,
                                              float *Xn, uint16_t *H0) {
   const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const int64_t i = g >> 6;
-  const int c = (int)(g & 63);
+  const int c = (int)(g & 63), f = c & (NF - 1);
   if (i >= n) return;
+  const float xn = (X[NF * i + f] - norm[f]) / norm[NF + f];
   float acc = prm[OFF_BE + c];
-  for (int k = 0; k < NF; ++k) {
-    const float xk = (X[NF * i + k] - norm[k]) / norm[NF + k];
-    acc = fmaf(xk, prm[OFF_WE + k * WD + c], acc);
-  }
-  if (c < NF) Xn[NF * i + c] = (X[NF * i + c] - norm[c]) / norm[NF + c];
+#pragma unroll
+  for (int k = 0; k < NF; ++k) acc = fmaf(lanebc(xn, k), prm[OFF_WE + k * WD + c], acc);
+  if (c < NF) Xn[NF * i + c] = xn;
   H0[WD * i + c] = f2bf(fmaxf(acc, 0.f));
 }
 
-// m_i = mean of h over the neighbours of i (adjacency order)
+// m_i = mean of h over the neighbours of i (adjacency order).  Half a wave per
+// vertex, two channels a lane; the neighbour list is loaded once and the rows
+// of eight neighbours are in flight at a time (one neighbour after the other,
+// a chain of dependent loads: 51 us at 43,554 vertices and 14.5 neighbours;
+// this 14 us).
 __global__ __launch_bounds__(256) void k_agg(int64_t n, const int64_t *ptr, const int32_t *col, const uint16_t *H,
                                              uint16_t *M) {
   const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t i = g >> 6;
-  const int c = (int)(g & 63);
+  const int64_t i = g >> 5;
+  const int c = (int)(g & 31);
+  const int64_t b = i < n ? ptr[i] : 0, e = i < n ? ptr[i + 1] : 0;
+  const uint32_t *H2 = reinterpret_cast<const uint32_t *>(H);
+  float s0 = 0.f, s1 = 0.f;
+  for (int64_t p0 = b; p0 < e; p0 += 32) {
+    const int m = (int)min((int64_t)32, e - p0);
+    const int my = c < m ? col[p0 + c] : 0;
+    for (int q = 0; q < m; q += 8) {
+      uint32_t v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int j = __shfl(my, min(q + u, m - 1), 32);
+        v[u] = H2[(WD / 2) * (int64_t)j + c];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (q + u < m) {
+          s0 += __uint_as_float(v[u] << 16);
+          s1 += __uint_as_float(v[u] & 0xffff0000u);
+        }
+    }
+  }
   if (i >= n) return;
-  const int64_t b = ptr[i], e = ptr[i + 1];
-  float s = 0.f;
-  for (int64_t p = b; p < e; ++p) s += bf2f(H[WD * (int64_t)col[p] + c]);
-  M[WD * i + c] = f2bf(e > b ? s / (float)(e - b) : 0.f);
+  const float d = (float)(e - b);
+  const uint32_t lo = f2bf(e > b ? s0 / d : 0.f), hi = f2bf(e > b ? s1 / d : 0.f);
+  reinterpret_cast<uint32_t *>(M)[(WD / 2) * i + c] = lo | (hi << 16);
 }
 
-// z = relu([h, m] W + b); h' = h + z   (W: 128 x 64 row-major, then b)
+// FP32 matrix cores: v_mfma_f32_32x32x2, lane l holds A[l%32][l/32],
+// B[l/32][l%32] and of the result, element r, row 8 (r/4) + 4 (l/32) + r%4,
+// column l%32.  Measured on gfx950: an entry is the chain of two fused
+// multiply-adds fma(a1, b1, fma(a0, b0, c)), so a sum over ascending input
+// index has the bits of the scalar loop (bias first) that the CPU restatement
+// follows.
+typedef float f16v __attribute__((ext_vector_type(16)));
+__device__ inline int mf_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
+
+// z = relu([h, m] W + b); h' = h + z   (W: 128 x 64 row-major, then b).  A
+// workgroup stages 64 rows of [h, m] in LDS; a wave takes 32 of them and 32 of
+// the 64 columns: its half of W in 64 registers, 64 matrix instructions.  A
+// column per lane with the inputs broadcast by v_readlane took 42 us at 43,554
+// rows, rows read straight into the operands 17, this 16.6 us.
+constexpr int MT_LD = WD + 1;  // LDS row stride in words: rows fall into distinct banks
 __global__ __launch_bounds__(256) void k_mp(int64_t n, const uint16_t *H, const uint16_t *M, const float *Wl,
                                             uint16_t *Z, uint16_t *Hn) {
-  const int lane = threadIdx.x & 63;
-  const int64_t w0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-  const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  float wa[WD], wb[WD];
+  __shared__ uint32_t in[64][MT_LD];  // words 0..31: h, 32..63: m
+  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5, wave = threadIdx.x >> 6;
+  const int c = 32 * (wave & 1) + li, rt = 32 * (wave >> 1);
+  float wt[WD];  // W[2 s + lh][c]
 #pragma unroll
-  for (int k = 0; k < WD; ++k) {
-    wa[k] = Wl[k * WD + lane];
-    wb[k] = Wl[(WD + k) * WD + lane];
-  }
-  const float bias = Wl[2 * WD * WD + lane];
-  for (int64_t i = w0; i < n; i += nw) {
-    const float h = bf2f(H[WD * i + lane]), m = bf2f(M[WD * i + lane]);
-    float acc = bias;
+  for (int s = 0; s < WD; ++s) wt[s] = Wl[(2 * s + lh) * WD + c];
+  const float bias = Wl[2 * WD * WD + c];
+  const uint32_t *H2 = reinterpret_cast<const uint32_t *>(H), *M2 = reinterpret_cast<const uint32_t *>(M);
+  for (int64_t r0 = 64 * (int64_t)blockIdx.x; r0 < n; r0 += 64 * (int64_t)gridDim.x) {
+    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < WD; ++k) acc = fmaf(lanebc(h, k), wa[k], acc);
+    for (int q = 0; q < 8; ++q) {
+      const int t = threadIdx.x + 256 * q, r = t >> 5, w = t & 31;
+      const int64_t row = min(r0 + r, n - 1);
+      in[r][w] = H2[32 * row + w];
+      in[r][32 + w] = M2[32 * row + w];
+    }
+    __syncthreads();
+    f16v acc;
 #pragma unroll
-    for (int k = 0; k < WD; ++k) acc = fmaf(lanebc(m, k), wb[k], acc);
-    const float z = fmaxf(acc, 0.f);
-    Z[WD * i + lane] = f2bf(z);
-    Hn[WD * i + lane] = f2bf(h + z);
+    for (int r = 0; r < 16; ++r) acc[r] = bias;
+#pragma unroll
+    for (int s = 0; s < WD; ++s) {
+      const uint32_t u = in[rt + li][s];
+      const float a = __uint_as_float(lh ? u & 0xffff0000u : u << 16);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, wt[s], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int rr = rt + mf_row(r, lane);
+      if (r0 + rr < n) {
+        const uint32_t u = in[rr][c >> 1];
+        const float z = fmaxf(acc[r], 0.f), h = __uint_as_float(c & 1 ? u & 0xffff0000u : u << 16);
+        Z[WD * (r0 + rr) + c] = f2bf(z);
+        Hn[WD * (r0 + rr) + c] = f2bf(h + z);
+      }
+    }
   }
 }
 
-// y = h Wd + bd; lanes 0..3 each compute one output in input order
-__global__ __launch_bounds__(256) void k_dec(int64_t n, const uint16_t *H, const float *prm, float *Y) {
-  const int lane = threadIdx.x & 63;
-  const int o = lane & 3;
-  const int64_t w0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-  const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  float wd[WD];
+// y = h Wd + bd, a thread per row, in input order
+__global__ __launch_bounds__(64) void k_dec(int64_t n, const uint16_t *H, const float *prm, float *Y) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  uint4 in[8];
 #pragma unroll
-  for (int k = 0; k < WD; ++k) wd[k] = prm[OFF_WD + k * NO + o];
-  const float bias = prm[OFF_BD + o];
-  for (int64_t i = w0; i < n; i += nw) {
-    const float h = bf2f(H[WD * i + lane]);
-    float acc = bias;
+  for (int q = 0; q < 8; ++q) in[q] = reinterpret_cast<const uint4 *>(H + WD * i)[q];
+  float y[NO];
 #pragma unroll
-    for (int k = 0; k < WD; ++k) acc = fmaf(lanebc(h, k), wd[k], acc);
-    if (lane < NO) Y[NO * i + lane] = acc;
+  for (int o = 0; o < NO; ++o) y[o] = prm[OFF_BD + o];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const uint32_t u[4] = {in[q].x, in[q].y, in[q].z, in[q].w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float h = __uint_as_float(k & 1 ? u[k >> 1] & 0xffff0000u : u[k >> 1] << 16);
+#pragma unroll
+      for (int o = 0; o < NO; ++o) y[o] = fmaf(h, prm[OFF_WD + (8 * q + k) * NO + o], y[o]);
+    }
   }
+  reinterpret_cast<float4 *>(Y)[i] = float4{y[0], y[1], y[2], y[3]};
 }
 
 // ---------------------------------------------------------------- backward
@@ -269,107 +331,246 @@ __global__ void k_chan_dot(int64_t n, const float *Y, const float *Tg, const flo
   }
 }
 
-// dP = dH where the stored activation is positive
-__global__ void k_mask(int64_t ne, const float *dH, const uint16_t *Z, float *dP) {
-  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (e >= ne) return;
-  dP[e] = bf2f(Z[e]) > 0.f ? dH[e] : 0.f;
-}
-
-// dHn[i][k] = dH[i][k] + sum_c dP[i][c] W[k][c];  dM[i][k] = sum_c dP[i][c] W[64+k][c]
-__global__ __launch_bounds__(256) void k_mp_bwd(int64_t n, const float *dP, const float *Wl, const float *dH,
-                                                float *dHn, float *dM) {
-  const int lane = threadIdx.x & 63;
-  const int64_t w0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-  const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  float wa[WD], wb[WD];
+// With dP = dH where the stored activation Z is positive, 0 elsewhere:
+//   dHn[i][k] = dH[i][k] + sum_c dP[i][c] W[k][c]
+//   dM[i][k] = sum_c dP[i][c] W[64+k][c] / deg(i)   (ready for k_agg_bwd)
+// on the FP32 matrix cores as in k_mp: a workgroup stages 32 rows of dP in LDS,
+// each of its four waves takes 32 of the 128 outputs.  43,554 rows: scalar loop
+// and separate masking pass 41 us, rows read straight into the operands 43,
+// this 25 us.
+__global__ __launch_bounds__(256) void k_mp_bwd(int64_t n, const uint16_t *Z, const float *Wl, const int64_t *ptr,
+                                                const float *dH, float *dHn, float *dM) {
+  __shared__ float dP[32][MT_LD], dHs[32][MT_LD], deg[32];
+  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5, part = threadIdx.x >> 6;
+  const int k = 32 * (part & 1) + li;
+  // W by rows through LDS, a row per output (a lane's own row straight from
+  // memory is 32 lines per load)
+  __shared__ float ws[2 * WD][MT_LD];
+  for (int t = threadIdx.x; t < 2 * WD * WD; t += 256) ws[t >> 6][t & 63] = Wl[t];
+  __syncthreads();
+  float wt[WD / 2];  // W[output][2 s + lh]
 #pragma unroll
-  for (int c = 0; c < WD; ++c) {
-    wa[c] = Wl[lane * WD + c];
-    wb[c] = Wl[(WD + lane) * WD + c];
-  }
-  for (int64_t i = w0; i < n; i += nw) {
-    const float p = dP[WD * i + lane];
-    float sa = 0.f, sb = 0.f;
+  for (int s = 0; s < WD / 2; ++s) wt[s] = ws[32 * part + li][2 * s + lh];
+  for (int64_t r0 = 32 * (int64_t)blockIdx.x; r0 < n; r0 += 32 * (int64_t)gridDim.x) {
+    __syncthreads();
 #pragma unroll
-    for (int c = 0; c < WD; ++c) {
-      const float pc = lanebc(p, c);
-      sa = fmaf(pc, wa[c], sa);
-      sb = fmaf(pc, wb[c], sb);
+    for (int q = 0; q < 8; ++q) {
+      const int t = threadIdx.x + 256 * q, r = t >> 6, c = t & 63;
+      const int64_t o = WD * min(r0 + r, n - 1) + c;
+      const float d = dH[o];
+      dHs[r][c] = d;
+      dP[r][c] = bf2f(Z[o]) > 0.f ? d : 0.f;
     }
-    dHn[WD * i + lane] = dH[WD * i + lane] + sa;
-    dM[WD * i + lane] = sb;
+    if (threadIdx.x < 32) {
+      const int64_t i = min(r0 + (int)threadIdx.x, n - 1);
+      deg[threadIdx.x] = (float)(ptr[i + 1] - ptr[i]);
+    }
+    __syncthreads();
+    f16v acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < WD / 2; ++s)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(dP[li][2 * s + lh], wt[s], acc, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int rr = mf_row(r, lane);
+      if (r0 + rr >= n) continue;
+      if (part < 2) dHn[WD * (r0 + rr) + k] = dHs[rr][k] + acc[r];
+      else dM[WD * (r0 + rr) + k] = acc[r] / deg[rr];
+    }
   }
 }
 
-// dH[j][c] += sum over neighbours i of j of dM[i][c] / deg(i)  (symmetric graph)
+// dH[j][c] += sum over neighbours i of j of dM[i][c] (dM divided by deg(i)
+// already; symmetric graph).  As k_agg (62 us with one neighbour after the
+// other and a division each; this 18 us).
 __global__ __launch_bounds__(256) void k_agg_bwd(int64_t n, const int64_t *ptr, const int32_t *col, const float *dM,
                                                  float *dH) {
   const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t j = g >> 6;
-  const int c = (int)(g & 63);
-  if (j >= n) return;
-  float s = 0.f;
-  for (int64_t p = ptr[j]; p < ptr[j + 1]; ++p) {
-    const int64_t i = col[p];
-    s += dM[WD * i + c] / (float)(ptr[i + 1] - ptr[i]);
-  }
-  dH[WD * j + c] += s;
-}
-
-// partial weight gradient of one row chunk: part[blk][k*N + c] = sum_r A[r][k] D[r][c]
-// for k < K1+K2 (A = [A1, A2]) and the bias row k = K1+K2 (A = 1)
-constexpr int TR = 32;
-constexpr int MAXJ = ((2 * WD + 1) * WD + 255) / 256;
-template <class TA>
-__global__ __launch_bounds__(256) void k_wgrad(int64_t n, int64_t chunk, const TA *A1, int K1, const uint16_t *A2,
-                                               int K2, const float *D, int N, float *part) {
-  __shared__ float As[TR * 2 * WD];
-  __shared__ float Ds[TR * WD];
-  const int K = K1 + K2, nout = (K + 1) * N;
-  const int64_t r0 = blockIdx.x * chunk, r1 = min(n, r0 + chunk);
-  float acc[MAXJ];
+  const int64_t i = g >> 5;
+  const int c = (int)(g & 31);
+  const int64_t b = i < n ? ptr[i] : 0, e = i < n ? ptr[i + 1] : 0;
+  const float2 *D2 = reinterpret_cast<const float2 *>(dM);
+  float s0 = 0.f, s1 = 0.f;
+  for (int64_t p0 = b; p0 < e; p0 += 32) {
+    const int m = (int)min((int64_t)32, e - p0);
+    const int my = c < m ? col[p0 + c] : 0;
+    for (int q = 0; q < m; q += 8) {
+      float2 v[8];
 #pragma unroll
-  for (int j = 0; j < MAXJ; ++j) acc[j] = 0.f;
-  for (int64_t rb = r0; rb < r1; rb += TR) {
-    const int nr = (int)min((int64_t)TR, r1 - rb);
-    __syncthreads();
-    for (int t = threadIdx.x; t < TR * K; t += blockDim.x) {
-      const int r = t / K, k = t % K;
-      float v = 0.f;
-      if (r < nr) v = k < K1 ? ld(A1 + (rb + r) * K1 + k) : bf2f(A2[(rb + r) * K2 + (k - K1)]);
-      As[t] = v;
-    }
-    for (int t = threadIdx.x; t < TR * N; t += blockDim.x) {
-      const int r = t / N, c = t % N;
-      Ds[t] = r < nr ? D[(rb + r) * N + c] : 0.f;
-    }
-    __syncthreads();
-    for (int r = 0; r < nr; ++r) {
-#pragma unroll
-      for (int j = 0; j < MAXJ; ++j) {
-        const int o = threadIdx.x + 256 * j;
-        if (o < nout) {
-          const int k = o / N, c = o % N;
-          const float a = k < K ? As[r * K + k] : 1.f;
-          acc[j] = fmaf(a, Ds[r * N + c], acc[j]);
-        }
+      for (int u = 0; u < 8; ++u) {
+        const int j = __shfl(my, min(q + u, m - 1), 32);
+        v[u] = D2[(WD / 2) * (int64_t)j + c];
       }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (q + u < m) {
+          s0 += v[u].x;
+          s1 += v[u].y;
+        }
     }
   }
+  if (i >= n) return;
+  float2 *o = reinterpret_cast<float2 *>(dH) + (WD / 2) * i + c;
+  *o = float2{o->x + s0, o->y + s1};
+}
+
+// Weight gradients: partial sums over the row chunk of each workgroup, added in
+// order by k_wreduce (deterministic).
+//
+// A message-passing layer: part[blk][k*64 + c] = sum_r A[r][k] dP[r][c] for
+// A = [H, M] (k < 128) and the bias row k = 128 (A = 1), dP as in k_mp_bwd.  A
+// product of 128 x rows by rows x 64 on the FP32 matrix cores: the eight waves
+// of a workgroup take the four 32-column parts of A times two halves of the
+// rows, two 32x32 results each; every load is one line per row.  Registers of
+// A rows in LDS and a scalar loop took 420 us at 43,554 rows; this 18 us.
+constexpr int WU = 8;  // row pairs in flight
+__global__ __launch_bounds__(512) void k_wgrad_mp(int64_t n, int64_t chunk, const uint16_t *H, const uint16_t *M,
+                                                  const uint16_t *Z, const float *dH, float *part) {
+  __shared__ float sh[2 * WD + 1][WD];
+  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
+  const int wave = threadIdx.x >> 6, kt = wave & 3, half = wave >> 2;
+  const int64_t r0 = blockIdx.x * chunk, r1 = min(n, r0 + chunk);
+  const uint16_t *A = (kt < 2 ? H : M) + 32 * (kt & 1) + li;
+  f16v c0, c1;
 #pragma unroll
-  for (int j = 0; j < MAXJ; ++j) {
-    const int o = threadIdx.x + 256 * j;
-    if (o < nout) part[(int64_t)blockIdx.x * nout + o] = acc[j];
+  for (int r = 0; r < 16; ++r) c0[r] = c1[r] = 0.f;
+  float b0 = 0.f, b1 = 0.f;
+  for (int64_t rb = r0 + 2 * half + lh; rb - lh < r1; rb += 4 * WU) {
+    float a[WU], d0[WU], d1[WU];
+#pragma unroll
+    for (int u = 0; u < WU; ++u) {
+      const int64_t r = rb + 4 * u;
+      const bool in = r < r1;
+      const int64_t o = WD * (in ? r : n - 1);
+      const float av = bf2f(A[o]), e0 = dH[o + li], e1 = dH[o + 32 + li];
+      const float z0 = bf2f(Z[o + li]), z1 = bf2f(Z[o + 32 + li]);
+      a[u] = in ? av : 0.f;
+      d0[u] = in && z0 > 0.f ? e0 : 0.f;
+      d1[u] = in && z1 > 0.f ? e1 : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < WU; ++u) {
+      c0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u], d0[u], c0, 0, 0, 0);
+      c1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u], d1[u], c1, 0, 0, 0);
+      b0 += d0[u];
+      b1 += d1[u];
+    }
+  }
+  b0 += __shfl_xor(b0, 32, 64);
+  b1 += __shfl_xor(b1, 32, 64);
+  if (half == 1) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      sh[32 * kt + mf_row(r, lane)][li] = c0[r];
+      sh[32 * kt + mf_row(r, lane)][32 + li] = c1[r];
+    }
+    if (kt == 0 && lh == 0) {
+      sh[2 * WD][li] = b0;
+      sh[2 * WD][32 + li] = b1;
+    }
+  }
+  __syncthreads();
+  if (half == 0) {
+    float *o = part + (int64_t)blockIdx.x * (2 * WD + 1) * WD;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int k = 32 * kt + mf_row(r, lane);
+      o[k * WD + li] = c0[r] + sh[k][li];
+      o[k * WD + 32 + li] = c1[r] + sh[k][32 + li];
+    }
+    if (kt == 0 && lh == 0) {
+      o[2 * WD * WD + li] = b0 + sh[2 * WD][li];
+      o[2 * WD * WD + 32 + li] = b1 + sh[2 * WD][32 + li];
+    }
   }
 }
 
-__global__ void k_wreduce(int nbk, int nout, const float *part, float *out) {
-  const int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= nout) return;
+// The encoder (part[blk][k*64 + c] = sum_r Xn[r][k] dP[r][c], k = 8 the bias,
+// dP masked by h0) and the decoder (part[blk][k*4 + o] = sum_r h3[r][k] dY[r][o],
+// k = 64 the bias): a row per wave and step, lane = column of the wide operand,
+// the narrow one uniform; the four waves' sums added in LDS.  122 us -> 17 us
+// and 113 us -> 6.6 us at 43,554 rows.
+__global__ __launch_bounds__(256) void k_wgrad_enc(int64_t n, int64_t chunk, const float *Xn, const uint16_t *H0,
+                                                   const float *dH, float *part) {
+  __shared__ float sh[4][NF + 1][WD];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t r0 = blockIdx.x * chunk, r1 = min(n, r0 + chunk);
+  float acc[NF + 1];
+#pragma unroll
+  for (int k = 0; k <= NF; ++k) acc[k] = 0.f;
+  for (int64_t rb = r0 + wave; rb < r1; rb += 16) {
+    float d[4], x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t r = min(rb + 4 * u, n - 1);
+      const float e = dH[WD * r + lane];
+      d[u] = rb + 4 * u < r1 && bf2f(H0[WD * r + lane]) > 0.f ? e : 0.f;
+      x[u] = Xn[NF * r + (lane & (NF - 1))];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+      for (int k = 0; k < NF; ++k) acc[k] = fmaf(lanebc(x[u], k), d[u], acc[k]);
+      acc[NF] += d[u];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k <= NF; ++k) sh[wave][k][lane] = acc[k];
+  __syncthreads();
+  for (int o = threadIdx.x; o < (NF + 1) * WD; o += 256) {
+    const int k = o / WD, c = o % WD;
+    part[(int64_t)blockIdx.x * (NF + 1) * WD + o] = sh[0][k][c] + sh[1][k][c] + sh[2][k][c] + sh[3][k][c];
+  }
+}
+__global__ __launch_bounds__(256) void k_wgrad_dec(int64_t n, int64_t chunk, const uint16_t *H, const float *dY,
+                                                   float *part) {
+  __shared__ float sh[4][WD + 1][NO];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t r0 = blockIdx.x * chunk, r1 = min(n, r0 + chunk);
+  float acc[NO] = {0.f, 0.f, 0.f, 0.f}, b = 0.f;
+  for (int64_t rb = r0 + wave; rb < r1; rb += 16) {
+    float h[4], y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t r = min(rb + 4 * u, n - 1);
+      h[u] = bf2f(H[WD * r + lane]);
+      const float e = dY[NO * r + (lane & (NO - 1))];
+      y[u] = rb + 4 * u < r1 ? e : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+      for (int o = 0; o < NO; ++o) acc[o] = fmaf(h[u], lanebc(y[u], o), acc[o]);
+      b += y[u];
+    }
+  }
+#pragma unroll
+  for (int o = 0; o < NO; ++o) sh[wave][lane][o] = acc[o];
+  if (lane < NO) sh[wave][WD][lane] = b;
+  __syncthreads();
+  for (int o = threadIdx.x; o < (WD + 1) * NO; o += 256) {
+    const int k = o / NO, c = o % NO;
+    part[(int64_t)blockIdx.x * (WD + 1) * NO + o] = sh[0][k][c] + sh[1][k][c] + sh[2][k][c] + sh[3][k][c];
+  }
+}
+
+// out[o] = sum over the nbk partial results: 64 outputs a workgroup, its four
+// waves take every fourth partial (one thread for all 256 of them: 62 us for
+// the 8,256 values of a layer; this 4.8 us)
+__global__ __launch_bounds__(256) void k_wreduce(int nbk, int nout, const float *part, float *out) {
+  __shared__ float sh[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int o = blockIdx.x * 64 + lane;
   float s = 0.f;
-  for (int b = 0; b < nbk; ++b) s += part[(int64_t)b * nout + o];
-  out[o] = s;
+  if (o < nout) {
+#pragma unroll 8
+    for (int b = wave; b < nbk; b += 4) s += part[(int64_t)b * nout + o];
+  }
+  sh[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && o < nout) out[o] = sh[0][lane] + sh[1][lane] + sh[2][lane] + sh[3][lane];
 }
 
 __global__ void k_adam(int64_t np, float *p, const float *g, float *m, float *v, float lr, float c1, float c2) {
@@ -439,7 +640,7 @@ struct m3_gnn {
   DBuf<float> prm, norm, grad, adam_m, adam_v;
   int64_t adam_t = 0;
   // activations and work arrays
-  DBuf<float> X, Xn, Y, Tg, dY, dH, dHn, dP, dM, part;
+  DBuf<float> X, Xn, Y, Tg, dY, dH, dHn, dM, part;
   DBuf<uint16_t> H[NL + 1], M[NL + 1], Z[NL + 1];
   DBuf<double> dpart, sc, dU;
   DBuf<float> dloss;
@@ -478,29 +679,20 @@ int gguard(m3_gnn *g, F &&f) {
 }
 
 int wgrid(const m3_gnn *g) { return (int)std::min<int64_t>(256, (g->n + 63) / 64); }
+// workgroups of the matrix-core layers, `rows` rows each per pass
+int mgrid(const m3_gnn *g, int rows) { return (int)std::min<int64_t>(768, (g->n + rows - 1) / rows); }
 
 void forward(m3_gnn *g, const float *X) {
   hipStream_t s = g->stream;
   const int64_t n = g->n;
-  const int gw = (int)std::min<int64_t>(256, (n + 3) / 4);  // 4 waves per block, rows strided
   hipLaunchKernelGGL(k_enc, dim3(nblk(64 * n)), dim3(256), 0, s, n, X, g->norm.p, g->prm.p, g->Xn.p, g->H[0].p);
   for (int l = 1; l <= NL; ++l) {
-    hipLaunchKernelGGL(k_agg, dim3(nblk(64 * n)), dim3(256), 0, s, n, g->ptr.p, g->col.p, g->H[l - 1].p,
+    hipLaunchKernelGGL(k_agg, dim3(nblk(32 * n)), dim3(256), 0, s, n, g->ptr.p, g->col.p, g->H[l - 1].p,
                        g->M[l].p);
-    hipLaunchKernelGGL(k_mp, dim3(gw), dim3(256), 0, s, n, g->H[l - 1].p, g->M[l].p,
+    hipLaunchKernelGGL(k_mp, dim3(mgrid(g, 64)), dim3(256), 0, s, n, g->H[l - 1].p, g->M[l].p,
                        g->prm.p + OFF_L + (l - 1) * LSZ, g->Z[l].p, g->H[l].p);
   }
-  hipLaunchKernelGGL(k_dec, dim3(gw), dim3(256), 0, s, n, g->H[NL].p, g->prm.p, g->Y.p);
-}
-
-template <class TA>
-void wgrad(m3_gnn *g, const TA *A1, int K1, const uint16_t *A2, int K2, const float *D, int N, float *out) {
-  const int nbk = wgrid(g);
-  const int64_t chunk = (g->n + nbk - 1) / nbk;
-  const int nout = (K1 + K2 + 1) * N;
-  hipLaunchKernelGGL((k_wgrad<TA>), dim3(nbk), dim3(256), 0, g->stream, g->n, chunk, A1, K1, A2, K2, D, N,
-                     g->part.p);
-  hipLaunchKernelGGL(k_wreduce, dim3(nblk(nout)), dim3(256), 0, g->stream, nbk, nout, g->part.p, out);
+  hipLaunchKernelGGL(k_dec, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, n, g->H[NL].p, g->prm.p, g->Y.p);
 }
 
 // loss of the current prediction against Tg (raw targets); writes *dloss_slot
@@ -512,20 +704,26 @@ void loss_and_backward(m3_gnn *g, const float *Tg, float *dloss_slot) {
   hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, s, n, g->Y.p, Tg, g->norm.p, scale, g->dY.p, g->dpart.p);
   hipLaunchKernelGGL(k_loss_fin, dim3(1), dim3(256), 0, s, nb, g->dpart.p, (double)ne, dloss_slot);
   float *grad = g->grad.p;
-  wgrad<uint16_t>(g, g->H[NL].p, WD, nullptr, 0, g->dY.p, NO, grad + OFF_WD);
+  const int nbk = wgrid(g);
+  const int64_t chunk = (n + nbk - 1) / nbk;
+  auto reduce = [&](int nout, float *out) {
+    hipLaunchKernelGGL(k_wreduce, dim3((unsigned)((nout + 63) / 64)), dim3(256), 0, s, nbk, nout, g->part.p, out);
+  };
+  hipLaunchKernelGGL(k_wgrad_dec, dim3(nbk), dim3(256), 0, s, n, chunk, g->H[NL].p, g->dY.p, g->part.p);
+  reduce((WD + 1) * NO, grad + OFF_WD);
   hipLaunchKernelGGL(k_dec_bwd, dim3(nblk(64 * n)), dim3(256), 0, s, n, g->dY.p, g->prm.p, g->dH.p);
-  const int gw = (int)std::min<int64_t>(256, (n + 3) / 4);
   float *dH = g->dH.p, *dHn = g->dHn.p;
   for (int l = NL; l >= 1; --l) {
     const float *Wl = g->prm.p + OFF_L + (l - 1) * LSZ;
-    hipLaunchKernelGGL(k_mask, dim3(nblk(WD * n)), dim3(256), 0, s, WD * n, dH, g->Z[l].p, g->dP.p);
-    wgrad<uint16_t>(g, g->H[l - 1].p, WD, g->M[l].p, WD, g->dP.p, WD, grad + OFF_L + (l - 1) * LSZ);
-    hipLaunchKernelGGL(k_mp_bwd, dim3(gw), dim3(256), 0, s, n, g->dP.p, Wl, dH, dHn, g->dM.p);
-    hipLaunchKernelGGL(k_agg_bwd, dim3(nblk(64 * n)), dim3(256), 0, s, n, g->ptr.p, g->col.p, g->dM.p, dHn);
+    hipLaunchKernelGGL(k_wgrad_mp, dim3(nbk), dim3(512), 0, s, n, chunk, g->H[l - 1].p, g->M[l].p, g->Z[l].p, dH,
+                       g->part.p);
+    reduce((2 * WD + 1) * WD, grad + OFF_L + (l - 1) * LSZ);
+    hipLaunchKernelGGL(k_mp_bwd, dim3(mgrid(g, 32)), dim3(256), 0, s, n, g->Z[l].p, Wl, g->ptr.p, dH, dHn, g->dM.p);
+    hipLaunchKernelGGL(k_agg_bwd, dim3(nblk(32 * n)), dim3(256), 0, s, n, g->ptr.p, g->col.p, g->dM.p, dHn);
     std::swap(dH, dHn);
   }
-  hipLaunchKernelGGL(k_mask, dim3(nblk(WD * n)), dim3(256), 0, s, WD * n, dH, g->H[0].p, g->dP.p);
-  wgrad<float>(g, g->Xn.p, NF, nullptr, 0, g->dP.p, WD, grad + OFF_WE);
+  hipLaunchKernelGGL(k_wgrad_enc, dim3(nbk), dim3(256), 0, s, n, chunk, g->Xn.p, g->H[0].p, dH, g->part.p);
+  reduce((NF + 1) * WD, grad + OFF_WE);
 }
 
 void adam_step(m3_gnn *g, float lr) {
@@ -533,6 +731,11 @@ void adam_step(m3_gnn *g, float lr) {
   const float c1 = 1.f - std::pow(0.9f, (float)g->adam_t), c2 = 1.f - std::pow(0.999f, (float)g->adam_t);
   hipLaunchKernelGGL(k_adam, dim3(nblk(NPARAM)), dim3(256), 0, g->stream, (int64_t)NPARAM, g->prm.p, g->grad.p,
                      g->adam_m.p, g->adam_v.p, lr, c1, c2);
+}
+
+void launch_scales(m3_gnn *g) {
+  hipLaunchKernelGGL(k_scales, dim3(SCB), dim3(256), 0, g->stream, g->n, g->Up.p, g->Pp.p, g->T.p, g->Tp.p, g->dpart.p);
+  hipLaunchKernelGGL(k_scales_fin, dim3(1), dim3(64), 0, g->stream, g->n, g->dpart.p, g->sc.p);
 }
 
 void upload_state(m3_gnn *g, const double *T, const double *Tp, const double *Visc, const double *Up,
@@ -547,7 +750,7 @@ void upload_state(m3_gnn *g, const double *T, const double *Tp, const double *Vi
   HIPCHECK(hipMemcpyAsync(g->visc.p, Visc, sizeof(double) * n, hipMemcpyHostToDevice, s));
   HIPCHECK(hipMemcpyAsync(g->Up.p, Up, sizeof(double) * 3 * g->nnod, hipMemcpyHostToDevice, s));
   HIPCHECK(hipMemcpyAsync(g->Pp.p, Pp, sizeof(double) * n, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_scales, dim3(1), dim3(SCB), 0, s, n, g->Up.p, g->Pp.p, g->T.p, g->Tp.p, g->sc.p);
+  launch_scales(g);
 }
 
 void features_to(m3_gnn *g, float *X) {
@@ -609,7 +812,7 @@ void make_base(m3_gnn *g, double t, int order, bool scales = true) {
   hipLaunchKernelGGL(k_lagrange, dim3(nblk(3 * nn)), dim3(256), 0, s, 3 * nn, lu, g->Up.p);
   hipLaunchKernelGGL(k_lagrange, dim3(nblk(n)), dim3(256), 0, s, n, lp, g->Pp.p);
   if (scales)  // needs the new temperature in T
-    hipLaunchKernelGGL(k_scales, dim3(1), dim3(SCB), 0, s, n, g->Up.p, g->Pp.p, g->T.p, g->Tp.p, g->sc.p);
+    launch_scales(g);
 }
 
 // U0 = Up + network change (vertices; edge nodes take the mean of their two
@@ -710,7 +913,7 @@ int m3_gnn_create(m3_gnn **out, int hip_device, const m3_graph_desc *d) {
     g->Y.alloc(NO * n);
     g->Tg.alloc(NO * n);
     g->dY.alloc(NO * n);
-    for (auto *b : {&g->dH, &g->dHn, &g->dP, &g->dM}) b->alloc(WD * n);
+    for (auto *b : {&g->dH, &g->dHn, &g->dM}) b->alloc(WD * n);
     for (int l = 0; l <= NL; ++l) {
       g->H[l].alloc(WD * n);
       if (l) {
