@@ -369,7 +369,7 @@ void diffusion_mesh(m3_ctx *c, const uint32_t *EL2NOD, int64_t nel, int64_t nnod
   const size_t ns = (size_t)D.C.nslot, n = (size_t)nnodT;
   D.M.alloc(ns);
   D.A.alloc(ns);
-  for (auto *b : {&D.ML, &D.Adi, &D.mask, &D.vfix, &D.T, &D.rhs, &D.x, &D.r, &D.rl, &D.d, &D.q, &D.Aq}) b->alloc(n);
+  for (auto *b : {&D.ML, &D.Adi, &D.mask, &D.vfix, &D.T, &D.rhs, &D.x, &D.r, &D.d, &D.q, &D.Aq}) b->alloc(n);
   // padding slots of the value arrays are never read; clear them once anyway
   D.C.val.zero(c->stream);
   D.M.zero(c->stream);
@@ -418,6 +418,18 @@ void diffusion3d(m3_ctx *c, double *T, double kappa, double dt, const int64_t *i
   a.err = c->errflag.p;
   hipLaunchKernelGGL(k_diff_elem, dim3(nblk(D.nel)), dim3(256), 0, s, a);
   HIPCHECK(hipGetLastError());
+  // fixed nodes, while the element kernel runs
+  std::vector<double> mask(n, 1.0), vf(n, 0.0);
+  bool in_range = true;
+  for (int64_t k = 0; k < nfix; ++k) {
+    const int64_t i = ifix[k] - 1;
+    if (i < 0 || i >= n) {
+      in_range = false;
+      continue;
+    }
+    mask[i] = 0.0;
+    vf[i] = vfix[k];
+  }
   int err = 0;
   HIPCHECK(hipMemcpyAsync(&err, c->errflag.p, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHECK(hipStreamSynchronize(s));
@@ -425,14 +437,7 @@ void diffusion3d(m3_ctx *c, double *T, double kappa, double dt, const int64_t *i
   if (err & 2) throw M3Error(M3_E_NUMERIC, "integration point has theta = 0 (det(J_CS) = Inf)");
   D.assembled = true;
   D.have_M = !lumped;
-  // fixed nodes
-  std::vector<double> mask(n, 1.0), vf(n, 0.0);
-  for (int64_t k = 0; k < nfix; ++k) {
-    const int64_t i = ifix[k] - 1;
-    M3_REQUIRE(i >= 0 && i < n, M3_E_ARG, "TBC.ifix out of range");
-    mask[i] = 0.0;
-    vf[i] = vfix[k];
-  }
+  M3_REQUIRE(in_range, M3_E_ARG, "TBC.ifix out of range");
   int64_t nfree = 0;
   for (double m : mask) nfree += m != 0.0;
   D.mask.upload(mask);
@@ -458,8 +463,8 @@ void diffusion3d(m3_ctx *c, double *T, double kappa, double dt, const int64_t *i
     // a zero initial residual is already the solution (the reference would
     // divide 0 / 0 in its first step)
     if (norm_r0 > 0.0 && !(norm_r0 < tol))
-      nit = m3::pcg_diag_run(c, Av, n, D.Adi.p, D.x.p, D.r.p, D.rl.p, D.d.p, D.q.p, D.Aq.p, (double)nfree, tol,
-                             o->itmax, &norm_r);
+      nit = m3::pcg_diag_run(c, Av, n, D.Adi.p, D.x.p, D.r.p, D.d.p, D.q.p, D.Aq.p, (double)nfree, tol, o->itmax,
+                             &norm_r);
   }
   hipLaunchKernelGGL(k_diff_out, dim3(nblk(n)), dim3(256), 0, s, n, D.mask.p, D.x.p, D.vfix.p, D.T.p);
   HIPCHECK(hipGetLastError());

@@ -384,7 +384,7 @@ struct m3_ctx {
     DBuf<uint8_t> cls;
     Sell C;                        // pattern (1 value per slot); val = CC
     DBuf<double> M, A;             // consistent mass and system values on C's slots
-    DBuf<double> ML, Adi, mask, vfix, T, rhs, x, r, rl, d, q, Aq;
+    DBuf<double> ML, Adi, mask, vfix, T, rhs, x, r, d, q, Aq;
   } dif;
   std::vector<double> h_sph;       // finest GCOORD_SPH row per node
   // semi-Lagrangian temperature advection on the finest P1 tetrahedra
@@ -517,8 +517,9 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
 // Jacobi-preconditioned CG on a scalar SELL operator (1 value per slot) whose
 // fixed rows/columns are identity: x and r (initial residual, zero at fixed
 // rows) in place; returns iterations, final RMS residual over nfree in *norm
-int pcg_diag_run(m3_ctx *c, SellView A, int64_t n, const double *Adi, double *x, double *r, double *rl,
-                 double *d, double *q, double *Aq, double nfree, double tol, int itmax, double *norm);
+// (q0, q1, Aq: work space of n values)
+int pcg_diag_run(m3_ctx *c, SellView A, int64_t n, const double *Adi, double *x, double *r, double *q0, double *q1,
+                 double *Aq, double nfree, double tol, int itmax, double *norm);
 void spmv_scalar(hipStream_t s, SellView A, int64_t n, const double *x, double *y);
 // thermal diffusion on linear tetrahedra
 void diffusion_mesh(m3_ctx *c, const uint32_t *EL2NOD, int64_t nel, int64_t nnodT, double theta_cone);

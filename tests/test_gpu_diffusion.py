@@ -178,3 +178,19 @@ def test_thermal_advdiff_step(c0):
     finally:
         del c0._m3ctx
         ctx.close()
+
+
+@pytest.mark.parametrize("itmax", [1, 7, 8, 9, 16, 500])
+def test_iteration_limits_match_the_oracle(c0, ctx0, itmax):
+    """The iterations are queued eight at a time: a limit before, at and after
+    such a group stops after as many iterations, with the same iterate."""
+    from oracle import diffusion as D
+    n = c0.nVnod
+    T0 = np.random.default_rng(9).random(n)
+    ifix, vfix = _fixed(c0, n)
+    T, info = ctx0.diffusion3d(T0, 1e-2, 0.5, ifix, vfix, tol=1e-12, itmax=itmax)
+    To, io = D.diffusion3d_p(T0, 1e-2, c0.GCOORD, c0.GCOORD_SPH, c0.levels[0].EL2NOD[:, :4], ifix, vfix, 0.5,
+                             tol=1e-12, itmax=itmax)
+    assert info["nit"] == io["nit"]
+    assert relerr(info["norm_r"], io["hist"][-1]) < 1e-6
+    assert relerr(T, To) < 1e-10
