@@ -178,84 +178,117 @@ struct AsmArgs {
   int *err;
 };
 
-__global__ __launch_bounds__(64) void k_assemble(AsmArgs a) {
-  const int64_t e = blockIdx.x;
-  const int lane = threadIdx.x;
-  __shared__ int s_nod[10];
-  __shared__ double s_wv[NIP], s_w[NIP], s_wd[NIP], s_wf[NIP], s_rh[NIP][3];
-  __shared__ double s_g[NIP][10][3];  // dN_n/dx_i at each IP (original frame)
-  // the lower node blocks of the element matrix in the KEL layout (block
-  // (na >= nb) at 9 (na (na+1)/2 + nb), entry 3c+d), original frame, then
-  // rotated in place; before the matrix exists the same LDS holds the
-  // per-IP Jacobian products (half the LDS of a full 30x30 copy: more
-  // resident waves)
-  __shared__ double s_Kl[KEL];
-  double(*s_J)[9] = reinterpret_cast<double(*)[9]>(s_Kl);  // [NIP][9]: rows original-frame x_i, cols d xi_k
-  __shared__ double s_RR[10][9];
-  __shared__ double s_Gr[30][4];
-  __shared__ double s_F[30];
-  __shared__ double s_msk[30], s_u0[30];
+// order the LDS accesses of one wave (the waves of a workgroup hold different elements)
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// One wave per element, four elements per workgroup.  The geometry (one lane
+// per integration point) is done by one of the four waves for all of them, 56
+// of its 64 lanes busy (alone, 14 lanes hold a wave through two sincos and three
+// divisions); the spherical coordinates of the nodes are formed before, a lane
+// per node.  K is formed per lane as a 3x3 node block from
+//   S = sum_ip w eta g_a g_b'   ->   K = tr(S) I + S' + C2 S,
+// 12 operations per point instead of 33 for the nine entries one by one, and
+// stays in registers through the rotation.  The lift of prescribed velocities
+// and the removal of fixed dofs run only in elements that have any, G only when
+// it is asked for.  245,760 elements: 1.44 ms -> 1.05 ms (0.22 of it the atomics
+// of Fb and M, 0.13 the store of Kel, 0.97 GB); Kel's bytes alone are 0.17 ms at
+// the copy rate.  Bound by latency: five waves per SIMD, six would spill (slower).
+constexpr int EPB = 4;
+__global__ __launch_bounds__(64 * EPB, 5) void k_assemble(AsmArgs a) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t e_ = (int64_t)blockIdx.x * EPB + wv;
+  const bool live = e_ < a.nel;
+  const int64_t e = live ? e_ : a.nel - 1;
+  __shared__ int s_nodA[EPB][10], s_cls[EPB];
+  __shared__ double s_ipA[EPB][NIP][7];  // w eta, w, w / eta, w Fg, r_hat
+  // gradients at the points [NIP][10][3] and the Jacobian products [NIP][9]
+  // (rows original-frame x_i, columns d xi_k), then the element matrix (KEL
+  // layout: block (na >= nb) at 9 (na (na+1)/2 + nb), entry 3c+d) in their
+  // place; before the gradients, the spherical coordinates of the mapping's
+  // nodes [20][3] and the viscosity and density of the vertices [8]
+  __shared__ double s_buf[EPB][NIP * 39];
+  __shared__ double s_RRA[EPB][10][9];
+  int *s_nod = s_nodA[wv];
+  double(*s_RR)[9] = s_RRA[wv];
+  double(*s_ip)[7] = s_ipA[wv];
+  double(*s_g)[10][3] = reinterpret_cast<double(*)[10][3]>(s_buf[wv]);
+  double(*s_J)[9] = reinterpret_cast<double(*)[9]>(s_buf[wv] + NIP * 30);
+  double *s_Kl = s_buf[wv];
+  double(*s_sph)[3] = reinterpret_cast<double(*)[3]>(s_buf[wv]);
+  static_assert(KEL <= NIP * 39, "element matrix in the gradients' place");
 
   const int cls = a.cls[e];
   if (lane < 10) s_nod[lane] = a.el2nod[e * 10 + lane];
-  __syncthreads();
+  if (lane == 0) s_cls[wv] = cls;
+  wave_sync();
+  // fixed dofs of the element, and whether any of them has a value
+  double msk = 1.0, u0 = 0.0;
   if (lane < 30) {
-    const int n = s_nod[lane / 3];
-    s_msk[lane] = a.mask[3 * (int64_t)n + lane % 3];
-    s_u0[lane] = a.U0[3 * (int64_t)n + lane % 3];
+    const int64_t d = 3 * (int64_t)s_nod[lane / 3] + lane % 3;
+    msk = a.mask[d];
+    u0 = a.U0[d];
   }
+  const unsigned fixed = (unsigned)__ballot(msk == 0.0);
+  const bool lifts = __ballot(u0 != 0.0) != 0;
   for (int t = lane; t < 90; t += 64) s_RR[t / 9][t % 9] = a.frames[(int64_t)s_nod[t / 9] * 9 + t % 9];
+  if (lane >= 32 && lane < 40) {
+    const int n = s_nod[lane & 3];
+    s_buf[wv][60 + lane - 32] = lane < 36 ? a.visc[n] : a.dens[n];
+  }
+  // spherical coordinates of the mapping's nodes in the frame of the class
+  if (lane < (cls == 3 ? 20 : 4)) {
+    double th, ph, rr;
+    if (cls >= 2) {  // 90-degree rotation about X: x'=x, y'=-z, z'=y
+      const double *x = cls == 3 ? a.X20 + (int64_t)a.iso_idx[e] * 60 + 3 * lane : a.X + 3 * (int64_t)s_nod[lane];
+      cart2sph(x[0], -x[2], x[1], th, ph, rr);
+    } else {
+      const double *sv = a.S + 3 * (int64_t)s_nod[lane];
+      th = sv[0];
+      ph = sv[1];
+      rr = sv[2];
+      if (cls == 1) {  // 180-degree rotation about Z
+        ph += M_PI;
+        if (ph > 2.0 * M_PI) ph -= 2.0 * M_PI;
+      }
+    }
+    s_sph[lane][0] = th;
+    s_sph[lane][1] = ph;
+    s_sph[lane][2] = rr;
+  }
+  __syncthreads();
 
-  // ---------------- per-IP geometry (one lane per integration point)
-  if (lane < NIP) {
-    const int ip = lane;
-    // J_SL[k][m] = sum_n dN_n/dxi_k * X_m(n) and the IP's interpolated
-    // coordinates, accumulated node by node as each node's spherical
-    // coordinates are formed (no per-node arrays: fewer registers, more
-    // resident waves)
+  // ---------------- per-IP geometry: one lane per integration point of the
+  // four elements, the workgroups' choice of wave spread over the SIMDs
+  if (wv == (int)(blockIdx.x & (EPB - 1)) && lane < EPB * NIP) {
+    const int el = lane / NIP, ip = lane - NIP * el, cl = s_cls[el];
+    const int64_t ee = (int64_t)blockIdx.x * EPB + el;
+    const bool lv = ee < a.nel;
+    // J_SL[k][m] = sum_n dN_n/dxi_k * X_m(n) and the IP's interpolated coordinates
     double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
     double thi = 0, phi = 0, ri = 0;
-    auto add_node = [&](double th, double ph, double rr, const double *dn, double N) {
+    auto add_node = [&](const double *x, const double *dn, double N) {
       for (int k = 0; k < 3; ++k) {
-        J[k][0] += dn[k] * th;
-        J[k][1] += dn[k] * ph;
-        J[k][2] += dn[k] * rr;
+        J[k][0] += dn[k] * x[0];
+        J[k][1] += dn[k] * x[1];
+        J[k][2] += dn[k] * x[2];
       }
-      thi += N * th;
-      phi += N * ph;
-      ri += N * rr;
+      thi += N * x[0];
+      phi += N * x[1];
+      ri += N * x[2];
     };
-    if (cls == 3) {
-      const double *x20 = a.X20 + (int64_t)a.iso_idx[e] * 60;
-      for (int n = 0; n < 20; ++n) {
-        double th, ph, rr;
-        // 90-degree rotation about X: x'=x, y'=-z, z'=y
-        cart2sph(x20[3 * n], -x20[3 * n + 2], x20[3 * n + 1], th, ph, rr);
-        add_node(th, ph, rr, c_dN20[ip][n], c_N20[ip][n]);
-      }
-    } else if (cls == 2) {
-      for (int n = 0; n < 4; ++n) {
-        const double *x = a.X + 3 * (int64_t)s_nod[n];
-        double th, ph, rr;
-        cart2sph(x[0], -x[2], x[1], th, ph, rr);
-        add_node(th, ph, rr, c_dN4[n], c_N4[ip][n]);
-      }
+    if (cl == 3) {
+      for (int n = 0; n < 20; ++n) add_node(s_buf[el] + 3 * n, c_dN20[ip][n], c_N20[ip][n]);
     } else {
-      for (int n = 0; n < 4; ++n) {
-        const double *sv = a.S + 3 * (int64_t)s_nod[n];
-        double ph = sv[1];
-        if (cls == 1) {  // 180-degree rotation about Z
-          ph += M_PI;
-          if (ph > 2.0 * M_PI) ph -= 2.0 * M_PI;
-        }
-        add_node(sv[0], ph, sv[2], c_dN4[n], c_N4[ip][n]);
-      }
+      for (int n = 0; n < 4; ++n) add_node(s_buf[el] + 3 * n, c_dN4[n], c_N4[ip][n]);
     }
     const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
                        J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
                        J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
-    if (det < 0) atomicOr(a.err, 1);
-    if (thi == 0.0) atomicOr(a.err, 2);
+    if (lv && det < 0) atomicOr(a.err, 1);
+    if (lv && thi == 0.0) atomicOr(a.err, 2);
     const double id = 1.0 / det;
     // inv(J_SL)[m][k] = d xi_k / d sph_m
     double I[3][3];
@@ -269,7 +302,9 @@ __global__ __launch_bounds__(64) void k_assemble(AsmArgs a) {
     I[2][1] = id * (J[0][1] * J[2][0] - J[0][0] * J[2][1]);
     I[2][2] = id * (J[0][0] * J[1][1] - J[0][1] * J[1][0]);
     // note: I is inv of the matrix with rows k; I[m][k] indexes (row m, col k)
-    const double st = sin(thi), ct = cos(thi), sp = sin(phi), cp = cos(phi);
+    double st, ct, sp, cp;
+    sincos(thi, &st, &ct);
+    sincos(phi, &sp, &cp);
     const double dCS = ri * ri * st;
     const double idCS = 1.0 / dCS;
     // J_SC[i][m] = d sph_m / d x_i (class frame)
@@ -283,48 +318,43 @@ __global__ __launch_bounds__(64) void k_assemble(AsmArgs a) {
         for (int m = 0; m < 3; ++m) acc += SC[i][m] * I[m][k];
         D[i][k] = acc;
       }
-    double rh[3] = {st * cp, st * sp, ct};
+    const double rh[3] = {st * cp, st * sp, ct};
     // class frame -> original frame for gradient rows and r_hat
-    double Do[3][3], rho[3];
-    if (cls == 1) {
-      for (int k = 0; k < 3; ++k) { Do[0][k] = -D[0][k]; Do[1][k] = -D[1][k]; Do[2][k] = D[2][k]; }
-      rho[0] = -rh[0]; rho[1] = -rh[1]; rho[2] = rh[2];
-    } else if (cls >= 2) {
-      for (int k = 0; k < 3; ++k) { Do[0][k] = D[0][k]; Do[1][k] = D[2][k]; Do[2][k] = -D[1][k]; }
-      rho[0] = rh[0]; rho[1] = rh[2]; rho[2] = -rh[1];
-    } else {
-      for (int i = 0; i < 3; ++i)
-        for (int k = 0; k < 3; ++k) Do[i][k] = D[i][k];
-      rho[0] = rh[0]; rho[1] = rh[1]; rho[2] = rh[2];
+    double *Jo = s_buf[el] + NIP * 30 + 9 * ip, *po = s_ipA[el][ip];
+    const int r1 = cl >= 2 ? 2 : 1, r2 = cl >= 2 ? 1 : 2;  // source rows of rows 1 and 2
+    const double s01 = cl == 1 ? -1.0 : 1.0, s2 = cl >= 2 ? -1.0 : 1.0;
+    for (int k = 0; k < 3; ++k) {
+      Jo[k] = s01 * D[0][k];
+      Jo[3 + k] = s01 * (r1 == 2 ? D[2][k] : D[1][k]);
+      Jo[6 + k] = s2 * (r2 == 1 ? D[1][k] : D[2][k]);
     }
-    for (int i = 0; i < 3; ++i)
-      for (int k = 0; k < 3; ++k) s_J[ip][3 * i + k] = Do[i][k];
     const double w = dCS * det * c_ipw[ip];
     double vi = 0, di = 0;
     for (int n = 0; n < 4; ++n) {
-      vi += a.visc[s_nod[n]] * c_N4[ip][n];
-      di += a.dens[s_nod[n]] * c_N4[ip][n];
+      vi += s_buf[el][60 + n] * c_N4[ip][n];
+      di += s_buf[el][64 + n] * c_N4[ip][n];
     }
     if (a.hasMin) vi = fmax(vi, a.minV);
     if (a.hasMax) vi = fmin(vi, a.maxV);
-    if (!(vi > 0)) atomicOr(a.err, 4);
+    if (lv && !(vi > 0)) atomicOr(a.err, 4);
     // buoyancy (..._out_cone_no_cross_2pi_opt.m:188-195 and the same branch of
     // the other three class kernels): with a refined region, zero outside it
     // and relative to the element's own reference density inside
     double Fg;
     if (a.ref_in)
-      Fg = a.ref_in[e] ? a.g * a.Bscale * (di - a.ref_d0[e]) : 0.0;
+      Fg = lv && a.ref_in[ee] ? a.g * a.Bscale * (di - a.ref_d0[ee]) : 0.0;
     else
       Fg = a.g * a.Bscale * (di - a.Dens0);
-    s_w[ip] = w;
-    s_wv[ip] = w * vi;
-    s_wd[ip] = w / vi;
-    s_wf[ip] = w * Fg;
-    s_rh[ip][0] = rho[0];
-    s_rh[ip][1] = rho[1];
-    s_rh[ip][2] = rho[2];
+    po[0] = w * vi;
+    po[1] = w;
+    po[2] = w / vi;
+    po[3] = w * Fg;
+    po[4] = s01 * rh[0];
+    po[5] = s01 * (r1 == 2 ? rh[2] : rh[1]);
+    po[6] = s2 * (r2 == 1 ? rh[1] : rh[2]);
   }
   __syncthreads();
+  if (!live) return;  // from here on each wave works alone
   // ---------------- gradients in the original frame
   for (int t = lane; t < NIP * 10; t += 64) {
     const int ip = t / 10, n = t % 10;
@@ -332,158 +362,149 @@ __global__ __launch_bounds__(64) void k_assemble(AsmArgs a) {
       s_g[ip][n][i] = s_J[ip][3 * i] * c_dN10[ip][n][0] + s_J[ip][3 * i + 1] * c_dN10[ip][n][1] +
                       s_J[ip][3 * i + 2] * c_dN10[ip][n][2];
   }
-  __syncthreads();
+  wave_sync();
   // ---------------- K (original frame): K[(a,c)][(b,d)] =
   //   sum_ip w eta [delta_cd g_a.g_b + g_b[c] g_a[d] + C2 g_b[d] g_a[c]]
-  //   one lane per 3x3 node block (na >= nb, 55 blocks): the two gradients of
-  //   an integration point are read once for the block's nine entries
-  const double C2 = a.C2;
+  //   one lane per 3x3 node block (na >= nb, 55 blocks)
+  int na = (int)((sqrtf(8.0f * (float)lane + 1.0f) - 1.0f) * 0.5f);  // lane = na (na+1)/2 + nb
+  if ((na + 1) * (na + 2) / 2 <= lane) ++na;
+  if (na * (na + 1) / 2 > lane) --na;
+  const int nb = lane - na * (na + 1) / 2;
+  double R[3][3];  // the block, rotated to the nodal (theta, phi, r) frames
   if (lane < 55) {
-    int na = 0, nb = lane;
-    while (nb > na) {
-      nb -= na + 1;
-      ++na;
-    }
-    double acc[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+    double S[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
 #pragma unroll 2
     for (int ip = 0; ip < NIP; ++ip) {
-      const double ga[3] = {s_g[ip][na][0], s_g[ip][na][1], s_g[ip][na][2]};
+      const double wv_ = s_ip[ip][0];
+      const double ga[3] = {wv_ * s_g[ip][na][0], wv_ * s_g[ip][na][1], wv_ * s_g[ip][na][2]};
       const double gb[3] = {s_g[ip][nb][0], s_g[ip][nb][1], s_g[ip][nb][2]};
-      const double wv = s_wv[ip];
-      const double dot = ga[0] * gb[0] + ga[1] * gb[1] + ga[2] * gb[2];
 #pragma unroll
       for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          double v = gb[c] * ga[d] + C2 * gb[d] * ga[c];
-          if (c == d) v += dot;
-          acc[c][d] += wv * v;
-        }
+        for (int d = 0; d < 3; ++d) S[c][d] += ga[c] * gb[d];
     }
-    double *blk = s_Kl + 9 * lane;  // lane = na (na+1)/2 + nb
+    const double tr = S[0][0] + S[1][1] + S[2][2];
+    double acc[3][3];
+#pragma unroll
     for (int c = 0; c < 3; ++c)
-      for (int d = 0; d < 3; ++d) {
-        // a diagonal block keeps its lower half (the upper entries mirror it)
-        blk[3 * c + d] = (na == nb && c < d) ? acc[d][c] : acc[c][d];
-        if (na == nb && c < d) continue;
-        const int p = 3 * na + c, q = 3 * nb + d;  // p >= q
-        if (a.dbgK) a.dbgK[e * 465 + (30 * q - q * (q - 1) / 2 + (p - q))] = acc[c][d];
-      }
-  }
-  // ---------------- G (original frame), M, Fb
-  for (int t = lane; t < 120; t += 64) {
-    const int v = t / 30, p = t % 30, na = p / 3, c = p % 3;
-    double acc = 0;
-    for (int ip = 0; ip < NIP; ++ip) acc += s_w[ip] * c_N4[ip][v] * s_g[ip][na][c];
-    s_Gr[p][v] = acc;
-    if (a.dbgG) a.dbgG[e * 120 + t] = acc;
-  }
-  if (lane < 30) {
-    const int na = lane / 3, c = lane % 3;
-    double acc = 0;
-    for (int ip = 0; ip < NIP; ++ip) acc += s_wf[ip] * c_N10[ip][na] * s_rh[ip][c];
-    s_F[lane] = acc;
-    if (a.dbgF) a.dbgF[e * 30 + lane] = acc;
-  }
-  double mval = 0;
-  int mv = 0, mw = 0;
-  if (lane >= 32 && lane < 48) {
-    mv = (lane - 32) / 4;
-    mw = (lane - 32) % 4;
-    for (int ip = 0; ip < NIP; ++ip) mval += s_wd[ip] * c_N4[ip][mv] * c_N4[ip][mw];
-    if (a.dbgM && mv >= mw) {
-      // packed lower column-major: column mw, row mv
-      const int idx = mw * 4 - mw * (mw - 1) / 2 + (mv - mw);
-      a.dbgM[e * 10 + idx] = mval;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) acc[c][d] = S[d][c] + a.C2 * S[c][d] + (c == d ? tr : 0.0);
+    // a diagonal block keeps its lower half (the upper entries mirror it)
+    if (na == nb) {
+      acc[0][1] = acc[1][0];
+      acc[0][2] = acc[2][0];
+      acc[1][2] = acc[2][1];
+    }
+    if (a.dbgK)
+      for (int c = 0; c < 3; ++c)
+        for (int d = 0; d < 3; ++d) {
+          if (na == nb && c < d) continue;
+          const int p = 3 * na + c, q = 3 * nb + d;  // p >= q
+          a.dbgK[e * 465 + (30 * q - q * (q - 1) / 2 + (p - q))] = acc[c][d];
+        }
+    double T1[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int dd = 0; dd < 3; ++dd)
+        T1[i][dd] = acc[i][0] * s_RR[nb][dd] + acc[i][1] * s_RR[nb][3 + dd] + acc[i][2] * s_RR[nb][6 + dd];
+#pragma unroll
+    for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+      for (int dd = 0; dd < 3; ++dd)
+        R[cc][dd] = s_RR[na][cc] * T1[0][dd] + s_RR[na][3 + cc] * T1[1][dd] + s_RR[na][6 + cc] * T1[2][dd];
+    if (na == nb) {
+      R[0][1] = R[1][0];
+      R[0][2] = R[2][0];
+      R[1][2] = R[2][1];
     }
   }
-  __syncthreads();
+  const int32_t *slot = a.slots + e * ASM_SLOTS;  // checked at m3_set_mesh
+  // ---------------- G (original frame; scattered rotated, G_rot[a,:,v] = RR_a'
+  // G[a,:,v]): it depends on the geometry only, so the host asks for it once
+  // per mesh
+  if ((a.scatterG || a.dbgG) && lane < 40) {
+    const int ga = lane / 4, v = lane % 4;
+    double g[3] = {0, 0, 0};
+    for (int ip = 0; ip < NIP; ++ip) {
+      const double wn = s_ip[ip][1] * c_N4[ip][v];
+      for (int c = 0; c < 3; ++c) g[c] += wn * s_g[ip][ga][c];
+    }
+    if (a.dbgG)
+      for (int c = 0; c < 3; ++c) a.dbgG[e * 120 + 30 * v + 3 * ga + c] = g[c];
+    if (a.scatterG && a.write_global) {
+      const int64_t p1 = slot[100 + lane], p2 = slot[140 + lane];
+      for (int cc = 0; cc < 3; ++cc) {
+        const double gr = s_RR[ga][cc] * g[0] + s_RR[ga][3 + cc] * g[1] + s_RR[ga][6 + cc] * g[2];
+        atomicAdd(a.G.val + cc * a.G.nslot + p1, gr);
+        atomicAdd(a.GT.val + cc * a.GT.nslot + p2, gr);
+      }
+    }
+  }
+  // ---------------- Fb (rotated) and M
+  if (lane < 10) {
+    double f[3] = {0, 0, 0};
+    for (int ip = 0; ip < NIP; ++ip) {
+      const double wn = s_ip[ip][3] * c_N10[ip][lane];
+      for (int c = 0; c < 3; ++c) f[c] += wn * s_ip[ip][4 + c];
+    }
+    if (a.dbgF)
+      for (int c = 0; c < 3; ++c) a.dbgF[e * 30 + 3 * lane + c] = f[c];
+    if (a.write_global)
+      for (int cc = 0; cc < 3; ++cc)
+        atomicAdd(&a.Fb[3 * (int64_t)s_nod[lane] + cc],
+                  s_RR[lane][cc] * f[0] + s_RR[lane][3 + cc] * f[1] + s_RR[lane][6 + cc] * f[2]);
+  } else if (lane >= 32 && lane < 48) {
+    const int mv = (lane - 32) / 4, mw = (lane - 32) % 4;
+    double mval = 0;
+    for (int ip = 0; ip < NIP; ++ip) mval += s_ip[ip][2] * c_N4[ip][mv] * c_N4[ip][mw];
+    // packed lower column-major: column mw, row mv
+    if (a.dbgM && mv >= mw) a.dbgM[e * 10 + mw * 4 - mw * (mw - 1) / 2 + (mv - mw)] = mval;
+    if (a.write_global) atomicAdd(a.M.val + slot[180 + (lane - 32)], mval);
+  }
   if (!a.write_global) return;
-  // ---------------- rotate the lower blocks to the nodal (theta, phi, r)
-  // frames, in place: each 3x3 block is read, rotated and written by one
-  // lane; the upper blocks are their transposes
-  if (lane < 55) {
-    int na = 0, nb = lane;
-    while (nb > na) {
-      nb -= na + 1;
-      ++na;
+  auto put = [&] {
+    wave_sync();  // the gradients (or the matrix before) have been read
+    if (lane < 55) {
+      double *blk = s_Kl + 9 * lane;
+      for (int cc = 0; cc < 3; ++cc)
+        for (int dd = 0; dd < 3; ++dd) blk[3 * cc + dd] = R[cc][dd];
     }
-    double *blk = s_Kl + 9 * lane;
-    double Kb[3][3], T1[3][3];
-    for (int i = 0; i < 3; ++i)
-      for (int j = 0; j < 3; ++j) Kb[i][j] = blk[3 * i + j];
-    for (int i = 0; i < 3; ++i)
-      for (int dd = 0; dd < 3; ++dd) {
-        double acc = 0;
-        for (int j = 0; j < 3; ++j) acc += Kb[i][j] * s_RR[nb][3 * j + dd];
-        T1[i][dd] = acc;
+    wave_sync();
+  };
+  // ---------------- BC lift (bc_rhs = K U0)
+  if (lifts) {
+    put();
+    if (lane < 30) {
+      double acc = 0;
+      const int la = lane / 3, cc = lane % 3;
+      for (int lb = 0; lb < 10; ++lb) {
+        // row (la, cc) of block (la, lb): stored block (la, lb), or the
+        // transpose of stored block (lb, la) above the diagonal
+        const bool lo = la >= lb;
+        const double *blk = s_Kl + 9 * (lo ? la * (la + 1) / 2 + lb : lb * (lb + 1) / 2 + la);
+        for (int dd = 0; dd < 3; ++dd) acc += (lo ? blk[3 * cc + dd] : blk[3 * dd + cc]) * a.U0[3 * (int64_t)s_nod[lb] + dd];
       }
-    double R[3][3];
-    for (int cc = 0; cc < 3; ++cc)
-      for (int dd = 0; dd < 3; ++dd) {
-        double acc = 0;
-        for (int i = 0; i < 3; ++i) acc += s_RR[na][3 * i + cc] * T1[i][dd];
-        R[cc][dd] = acc;
-      }
-    for (int cc = 0; cc < 3; ++cc)
-      for (int dd = 0; dd < 3; ++dd) blk[3 * cc + dd] = (na == nb && cc < dd) ? R[dd][cc] : R[cc][dd];
-  }
-  __syncthreads();
-  // ---------------- BC lift (bc_rhs = K U0) and removal of fixed dofs
-  if (lane < 30) {
-    double acc = 0;
-    const int na = lane / 3, cc = lane % 3;
-    for (int nb = 0; nb < 10; ++nb) {
-      // row (na, cc) of block (na, nb): stored block (na, nb), or the
-      // transpose of stored block (nb, na) above the diagonal
-      const bool lo = na >= nb;
-      const double *blk = s_Kl + 9 * (lo ? na * (na + 1) / 2 + nb : nb * (nb + 1) / 2 + na);
-      for (int dd = 0; dd < 3; ++dd) acc += (lo ? blk[3 * cc + dd] : blk[3 * dd + cc]) * s_u0[3 * nb + dd];
+      if (acc != 0.0) atomicAdd(&a.bc_rhs[3 * (int64_t)s_nod[la] + cc], acc);
     }
-    if (acc != 0.0) atomicAdd(&a.bc_rhs[3 * (int64_t)s_nod[lane / 3] + lane % 3], acc);
   }
-  __syncthreads();
-  for (int t = lane; t < KEL; t += 64) {
-    const int pq = c_bq[t], p = pq & 255, q = pq >> 8;
-    s_Kl[t] *= s_msk[p] * s_msk[q];
-  }
-  __syncthreads();
+  // ---------------- removal of fixed dofs
+  if (fixed && lane < 55)
+    for (int cc = 0; cc < 3; ++cc)
+      for (int dd = 0; dd < 3; ++dd)
+        if ((fixed >> (3 * na + cc) | fixed >> (3 * nb + dd)) & 1u) R[cc][dd] *= 0.0;
+  put();
   if (a.Kel)
     for (int t = lane; t < KEL; t += 64) a.Kel[e * KEL + t] = s_Kl[t];
   // ---------------- scatter K blocks (unless the row-owner gather k_gatherK sums them)
-  const int32_t *slot = a.slots + e * ASM_SLOTS;  // checked at m3_set_mesh
   for (int t = lane; t < (a.scatterK ? 100 : 0); t += 64) {
-    const int na = t / 10, nb = t % 10;
+    const int ka = t / 10, kb = t % 10;
     const int64_t pos = slot[t];
-    const bool lo = na >= nb;
-    const double *blk = s_Kl + 9 * (lo ? na * (na + 1) / 2 + nb : nb * (nb + 1) / 2 + na);
+    const bool lo = ka >= kb;
+    const double *blk = s_Kl + 9 * (lo ? ka * (ka + 1) / 2 + kb : kb * (kb + 1) / 2 + ka);
     for (int cc = 0; cc < 3; ++cc)
       for (int dd = 0; dd < 3; ++dd)
         atomicAdd(a.K.val + kval(pos, 3 * cc + dd), lo ? blk[3 * cc + dd] : blk[3 * dd + cc]);
-  }
-  // ---------------- G (rotated): G_rot[a,:,v] = RR_a' G[a,:,v]; it depends
-  // on the geometry only, so the host skips it when the mesh is unchanged
-  if (a.scatterG && lane < 40) {
-    const int na = lane / 4, v = lane % 4;
-    double gr[3];
-    for (int cc = 0; cc < 3; ++cc) {
-      double acc = 0;
-      for (int i = 0; i < 3; ++i) acc += s_RR[na][3 * i + cc] * s_Gr[3 * na + i][v];
-      gr[cc] = acc;
-    }
-    const int64_t p1 = slot[100 + lane], p2 = slot[140 + lane];
-    for (int cc = 0; cc < 3; ++cc) {
-      atomicAdd(a.G.val + cc * a.G.nslot + p1, gr[cc]);
-      atomicAdd(a.GT.val + cc * a.GT.nslot + p2, gr[cc]);
-    }
-  }
-  if (lane >= 32 && lane < 48) atomicAdd(a.M.val + slot[180 + (lane - 32)], mval);
-  // ---------------- Fb (rotated)
-  if (lane < 30) {
-    const int na = lane / 3, cc = lane % 3;
-    double acc = 0;
-    for (int i = 0; i < 3; ++i) acc += s_RR[na][3 * i + cc] * s_F[3 * na + i];
-    atomicAdd(&a.Fb[3 * (int64_t)s_nod[na] + cc], acc);
   }
 }
 
@@ -915,7 +936,7 @@ void launch_assemble(m3_ctx *c, double *dbgK, double *dbgG, double *dbgM, double
   a.scatterK = c->gather_K ? 0 : 1;
   a.scatterG = write_global && !c->g_valid ? 1 : 0;
   a.err = c->errflag.p;
-  hipLaunchKernelGGL(k_assemble, dim3((unsigned)f.nel), dim3(64), 0, c->stream, a);
+  hipLaunchKernelGGL(k_assemble, dim3((unsigned)((f.nel + EPB - 1) / EPB)), dim3(64 * EPB), 0, c->stream, a);
   HIPCHECK(hipGetLastError());
 }
 
