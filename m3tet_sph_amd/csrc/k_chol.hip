@@ -34,6 +34,15 @@ namespace {
 
 constexpr int TS = 64;
 constexpr int TT = TS * TS;
+// The solves take the blocks of the first dissection levels as one, as many
+// whole levels as fit into this many tiles: fewer dependent launches against a
+// longer inversion, once per factorisation.  0 / 16 / 32 / 36 / 48 tiles, us per
+// FP64 iteration of the whole solver and per factorisation:
+//   34 tiles in all   157 / 143 / 142 / 135 / 137 and 546 / 581 / 581 / 637 / 630
+//   130               225 / 222 / 216 / 216 / 212 and 1,097 / 1,093 / 1,156 / 1,156 / 1,197
+//   275             1,429 / 1,422 / 1,406 / 1,403 / 1,355 and 2,667 / 2,662 / 2,675 / 2,740 / 2,728
+// (runs differ by 20 and 15).  A factorisation serves a few hundred iterations.
+constexpr int ROOT_TILES = 36;
 constexpr int LEAF = 80;  // nodes per leaf block (40 / 80 / 160: 309 / 306 / 305 ms per c1 solve)
 
 // ---- host: nested dissection into tile-aligned blocks ----------------------------------
@@ -44,6 +53,7 @@ struct NDState {
   std::vector<int32_t> stamp;
   int cur = 0;
   std::vector<std::vector<int32_t>> blocks;  // node lists in elimination order
+  std::vector<int> depth;                    // dissection depth of each block (0: the first separator)
 };
 
 // Order the nodes of a block along a 3-D Morton (Z-order) curve of their
@@ -218,11 +228,12 @@ void split(NDState &st, std::vector<int32_t> nodes, int ax, std::vector<int32_t>
 
 // Nested dissection: the split across the axis with the smallest separator
 // (ties: the longer extent), both halves recursively, then the separator.
-void nd_rec(NDState &st, std::vector<int32_t> nodes) {
+void nd_rec(NDState &st, std::vector<int32_t> nodes, int depth = 0) {
   if (nodes.empty()) return;
   if (nodes.size() <= (size_t)LEAF) {
     spatial_order(st, nodes);
     st.blocks.push_back(nodes);
+    st.depth.push_back(depth);
     return;
   }
   double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
@@ -247,12 +258,16 @@ void nd_rec(NDState &st, std::vector<int32_t> nodes) {
   }
   if (!have) {  // all nodes at one point: one block
     st.blocks.push_back(nodes);
+    st.depth.push_back(depth);
     return;
   }
   spatial_order(st, bestS);
-  nd_rec(st, bestA);
-  nd_rec(st, bestB);
-  if (!bestS.empty()) st.blocks.push_back(bestS);
+  nd_rec(st, bestA, depth + 1);
+  nd_rec(st, bestB, depth + 1);
+  if (!bestS.empty()) {
+    st.blocks.push_back(bestS);
+    st.depth.push_back(depth);
+  }
 }
 
 // ---- device kernels --------------------------------------------------------------------
@@ -774,15 +789,33 @@ void chol_analyse(m3_ctx *c) {
   for (int64_t n = 0; n < nn; ++n)
     if (mask[3 * n] + mask[3 * n + 1] + mask[3 * n + 2] > 0) nodes.push_back((int32_t)n);
   nd_rec(st, nodes);
+  // dofs of every block; the blocks of the dissection's first levels, as many
+  // whole levels as fit into ROOT_TILES tiles, come last: they are factorised
+  // as blocks of their own but solved as one (below)
+  std::vector<std::vector<int32_t>> bdofs(st.blocks.size());
+  std::vector<int> level_tiles;
+  for (size_t b = 0; b < st.blocks.size(); ++b) {
+    for (int n : st.blocks[b])
+      for (int k = 0; k < 3; ++k)
+        if (mask[3 * (int64_t)n + k] != 0.0) bdofs[b].push_back(3 * n + k);
+    if ((int)level_tiles.size() <= st.depth[b]) level_tiles.resize(st.depth[b] + 1, 0);
+    level_tiles[st.depth[b]] += (int)((bdofs[b].size() + TS - 1) / TS);
+  }
+  int root_depth = 0;
+  for (int t = 0; root_depth < (int)level_tiles.size() && t + level_tiles[root_depth] <= ROOT_TILES; ++root_depth)
+    t += level_tiles[root_depth];
+  std::vector<int> order;
+  for (int root = 0; root < 2; ++root)
+    for (size_t b = 0; b < bdofs.size(); ++b)
+      if ((st.depth[b] < root_depth) == (root == 1)) order.push_back((int)b);
   // positions, padded per block
   std::vector<int32_t> pos2dof, blk_t0, blk_t1;
   int64_t nfree = 0;
-  for (auto &b : st.blocks) {
-    std::vector<int32_t> dofs;
-    for (int n : b)
-      for (int k = 0; k < 3; ++k)
-        if (mask[3 * (int64_t)n + k] != 0.0) dofs.push_back(3 * n + k);
+  int root_blk = -1;  // first block of the root
+  for (int ob : order) {
+    const std::vector<int32_t> &dofs = bdofs[ob];
     if (dofs.empty()) continue;
+    if (root_blk < 0 && st.depth[ob] < root_depth) root_blk = (int)blk_t0.size();
     const int t0 = (int)(pos2dof.size() / TS);
     pos2dof.insert(pos2dof.end(), dofs.begin(), dofs.end());
     nfree += (int64_t)dofs.size();
@@ -891,6 +924,16 @@ void chol_analyse(m3_ctx *c) {
     ch.h_upd_ptr[l + 1] = (int32_t)upd_tile.size();
     ch.h_trsm_ptr[l + 1] = (int32_t)trsm_tile.size();
   }
+  // the solves take the root's blocks as one: its inverse factor is one set of
+  // tiles, and the launches of its blocks' heights go.  The factorisation above
+  // keeps them apart (independent separators run side by side).
+  if (root_blk >= 0 && root_blk + 1 < ch.nblock) {
+    blk_t1[root_blk] = blk_t1.back();
+    blk_t0.resize(root_blk + 1);
+    blk_t1.resize(root_blk + 1);
+    ch.nblock = root_blk + 1;
+    for (int t = blk_t0[root_blk]; t < T; ++t) blk_of[t] = root_blk;
+  }
   // block heights from the structure of L: a block comes after every block
   // that has tiles in its rows
   std::vector<int> hb(ch.nblock, 0);
@@ -926,6 +969,18 @@ void chol_analyse(m3_ctx *c) {
       inv_x.push_back(xidx(b, i, i));
       inv_row.push_back(i);
     }
+  // tiles of X that are not zero: column j of the inverse reaches the rows that
+  // the columns of L reach from j (all of them in a block with a dense factor)
+  std::vector<uint8_t> x_nz((size_t)ch.nX, 0);
+  for (int b = 0; b < ch.nblock; ++b)
+    for (int j = blk_t0[b]; j < blk_t1[b]; ++j) {
+      x_nz[xidx(b, j, j)] = 1;
+      for (int k = j; k < blk_t1[b]; ++k) {
+        if (!x_nz[xidx(b, k, j)]) continue;
+        for (int32_t t = ch.h_colptr[k]; t < ch.h_colptr[k + 1]; ++t)
+          if (ch.h_rowtile[t] < blk_t1[b]) x_nz[xidx(b, ch.h_rowtile[t], j)] = 1;
+      }
+    }
   // Z tiles: for each block S and row tile I below it, Z_Ij = sum_k L_Ik X_kj
   // (k >= j in S); stored after the X tiles in the same pool
   std::vector<int32_t> z_tile, z_pairs;
@@ -942,7 +997,7 @@ void chol_analyse(m3_ctx *c) {
       for (int I : below) {
         const size_t before = z_pairs.size();
         for (int k = j; k < blk_t1[b]; ++k) {
-          const int32_t tl = tile_of(I, k);
+          const int32_t tl = x_nz[xidx(b, k, j)] ? tile_of(I, k) : -1;
           if (tl >= 0) {
             z_pairs.push_back(tl);
             z_pairs.push_back(xidx(b, k, j));
@@ -985,7 +1040,7 @@ void chol_analyse(m3_ctx *c) {
       for (int j = a; j < sp; ++j) {
         InvTask tk;
         for (int k = j; k < sp; ++k) {
-          const int32_t tl = tile_of(i, k);
+          const int32_t tl = x_nz[xidx(b, k, j)] ? tile_of(i, k) : -1;
           if (tl >= 0) {
             tk.pairs.push_back(tl);
             tk.pairs.push_back(xidx(b, k, j));
@@ -998,16 +1053,17 @@ void chol_analyse(m3_ctx *c) {
       }
     for (int i = sp; i < e; ++i)
       for (int j = a; j < sp; ++j) {
+        if (!x_nz[xidx(b, i, j)]) continue;
         InvTask tk;
         tk.out = xidx(b, i, j);
         for (int k = sp; k <= i; ++k) {
           const int32_t tt = tix[(size_t)(k - sp) * na + (j - a)];
-          if (tt >= 0) {
+          if (tt >= 0 && x_nz[xidx(b, i, k)]) {
             tk.pairs.push_back(xidx(b, i, k));
             tk.pairs.push_back(tt);
           }
         }
-        stepX[lv].push_back(std::move(tk));  // written even when zero: the solves read every X_ij
+        stepX[lv].push_back(std::move(tk));
       }
     return lv;
   };
@@ -1034,7 +1090,8 @@ void chol_analyse(m3_ctx *c) {
   for (int h = 0; h < H; ++h) {
     for (int b : blocks_at[h]) {
       for (int i = blk_t0[b]; i < blk_t1[b]; ++i)
-        for (int j = blk_t0[b]; j <= i; ++j) fw.item(i, xidx(b, i, j), j, 0);
+        for (int j = blk_t0[b]; j <= i; ++j)
+          if (x_nz[xidx(b, i, j)]) fw.item(i, xidx(b, i, j), j, 0);
       for (auto &z : zlist[b]) fw.item(z[0], z[2], z[1], 1);
     }
     fw.end_height();
@@ -1042,7 +1099,8 @@ void chol_analyse(m3_ctx *c) {
   for (int h = H - 1; h >= 0; --h) {
     for (int b : blocks_at[h]) {
       for (int j = blk_t0[b]; j < blk_t1[b]; ++j)
-        for (int i = j; i < blk_t1[b]; ++i) bw.item(j, xidx(b, i, j), i, 0);
+        for (int i = j; i < blk_t1[b]; ++i)
+          if (x_nz[xidx(b, i, j)]) bw.item(j, xidx(b, i, j), i, 0);
       for (auto &z : zlist[b]) bw.item(z[1], z[2], z[0], 1);
     }
     bw.end_height();
