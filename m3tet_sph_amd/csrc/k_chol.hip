@@ -715,25 +715,23 @@ __global__ __launch_bounds__(256) void k_gtask(const CholTiles::Item *items, int
   }
 }
 
-// right-hand side into tile order (FP64), and the forward / backward
-// accumulators y and x cleared, in one pass
-template <class T>
-__global__ void k_to_tiles(int64_t npos, const int32_t *pos2dof, const T *rhs, double *w, double *y, double *x) {
+// right-hand side into tile order, and the forward / backward accumulators y
+// and x cleared, in one pass
+__global__ void k_to_tiles(int64_t npos, const int32_t *pos2dof, const double *rhs, double *w, double *y, double *x) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= npos) return;
   const int d = pos2dof[i];
-  w[i] = d >= 0 ? (double)rhs[d] : 0.0;
+  w[i] = d >= 0 ? rhs[d] : 0.0;
   y[i] = 0.0;
   x[i] = 0.0;
 }
 
 // solution back to dof order; fixed dofs (no tile position) get 0
-template <class T>
-__global__ void k_from_tiles(int64_t n, const int32_t *dof2pos, const double *x, T *out) {
+__global__ void k_from_tiles(int64_t n, const int32_t *dof2pos, const double *x, double *out) {
   const int64_t d = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (d >= n) return;
   const int p = dof2pos[d];
-  out[d] = p >= 0 ? (T)x[p] : (T)0;
+  out[d] = p >= 0 ? x[p] : 0.0;
 }
 
 __global__ void k_zero(int64_t n, double *x) {
@@ -1211,38 +1209,31 @@ static void run_phase(m3_ctx *c, hipStream_t s, CholTiles::Phase &p, int h, cons
   }
 }
 
-template <class T>
-static void chol_solve_t(m3_ctx *c, const T *rhs, T *x) {
+void chol_solve_tiles(m3_ctx *c, bool tiles32) {
   CholTiles &ch = c->chol;
-  LevelDev &cl = c->L[c->nmg - 1];
   hipStream_t s = c->stream;
-  const int64_t npos = (int64_t)ch.T * TS;
-  {
-    ProfScope ps(c, 2, true, npos * (4.0 + sizeof(T) + 3 * 8.0));
-    launch_timed(k_to_tiles<T>, dim3(nblk(npos)), dim3(256), s, npos, (const int32_t *)ch.pos2dof.p, rhs, ch.w.p,
-                 ch.y.p, ch.x.p);
-  }
-  // the FP32 solve reads the FP32 copies of the tiles (half the bytes; the
-  // FP32 V-cycle around it carries FP32 values anyway)
-  const bool t32 = std::is_same<T, float>::value;
+  // the FP32 V-cycle reads the FP32 copies of the tiles (half the bytes; the
+  // cycle around it carries FP32 values anyway)
   for (int h = 0; h < ch.H; ++h) {
-    if (t32) run_phase(c, s, ch.fwd, h, (const float *)ch.X32.p, ch.w.p, ch.w.p, ch.y.p, ch.w.p);
+    if (tiles32) run_phase(c, s, ch.fwd, h, (const float *)ch.X32.p, ch.w.p, ch.w.p, ch.y.p, ch.w.p);
     else run_phase(c, s, ch.fwd, h, (const double *)ch.X.p, ch.w.p, ch.w.p, ch.y.p, ch.w.p);
   }
   for (int k = 0; k < ch.H; ++k) {
-    if (t32) run_phase(c, s, ch.bwd, k, (const float *)ch.XT32.p, ch.y.p, ch.x.p, ch.x.p, ch.x.p);
+    if (tiles32) run_phase(c, s, ch.bwd, k, (const float *)ch.XT32.p, ch.y.p, ch.x.p, ch.x.p, ch.x.p);
     else run_phase(c, s, ch.bwd, k, (const double *)ch.XT.p, ch.y.p, ch.x.p, ch.x.p, ch.x.p);
-  }
-  const int64_t n3 = 3 * cl.nnod;
-  {
-    ProfScope ps(c, 2, true, n3 * (4.0 + 8.0 + sizeof(T)));
-    launch_timed(k_from_tiles<T>, dim3(nblk(n3)), dim3(256), s, n3, (const int32_t *)ch.dof2pos.p,
-                 (const double *)ch.x.p, x);
   }
   HIPCHECK(hipGetLastError());
 }
 
-void chol_solve_dev(m3_ctx *c, const double *rhs, double *x) { chol_solve_t<double>(c, rhs, x); }
-void chol_solve_dev32(m3_ctx *c, const float *rhs, float *x) { chol_solve_t<float>(c, rhs, x); }
+void chol_solve_dev(m3_ctx *c, const double *rhs, double *x) {
+  CholTiles &ch = c->chol;
+  LevelDev &cl = c->L[c->nmg - 1];
+  hipStream_t s = c->stream;
+  const int64_t npos = (int64_t)ch.T * TS, n3 = 3 * cl.nnod;
+  hipLaunchKernelGGL(k_to_tiles, dim3(nblk(npos)), dim3(256), 0, s, npos, ch.pos2dof.p, rhs, ch.w.p, ch.y.p, ch.x.p);
+  chol_solve_tiles(c, false);
+  hipLaunchKernelGGL(k_from_tiles, dim3(nblk(n3)), dim3(256), 0, s, n3, ch.dof2pos.p, ch.x.p, x);
+  HIPCHECK(hipGetLastError());
+}
 
 }  // namespace m3

@@ -351,34 +351,53 @@ __global__ void k_spmv_M(SellView M, int64_t nrow, const double *x, double *y) {
   y[row] = a;
 }
 
-// prolongation with the add of the saved defect: df = dd + mask_f * (P dc)
+// prolongation with the add of the saved defect: df = dd + mask_f * (P dc);
+// from the coarsest level (pos not NULL) dc is read where the triangular solves
+// left it, pos[dof] in tile order (-1: fixed, 0)
 template <class VT, class WT>
 __global__ void k_prolong(int64_t nf, const int64_t *ptr, const int32_t *col, const WT *w,
-                          const uint8_t *mask, const VT *dc, const VT *dd, VT *df) {
+                          const uint8_t *mask, const VT *dc, const double *xt, const int32_t *pos, const VT *dd,
+                          VT *df) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= nf) return;
-  VT a0 = 0, a1 = 0, a2 = 0;
+  VT a[3] = {0, 0, 0};
   for (int64_t k = ptr[i]; k < ptr[i + 1]; ++k) {
     const int64_t c3 = 3 * (int64_t)col[k];
     const VT wk = (VT)w[k];
-    a0 += wk * dc[c3];
-    a1 += wk * dc[c3 + 1];
-    a2 += wk * dc[c3 + 2];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      VT v;
+      if (pos) {
+        const int q = pos[c3 + c];
+        v = q >= 0 ? (VT)xt[q] : (VT)0;
+      } else {
+        v = dc[c3 + c];
+      }
+      a[c] += wk * v;
+    }
   }
   const int64_t o = 3 * i;
-  df[o] = (dd ? dd[o] : (VT)0) + (VT)mask[o] * a0;
-  df[o + 1] = (dd ? dd[o + 1] : (VT)0) + (VT)mask[o + 1] * a1;
-  df[o + 2] = (dd ? dd[o + 2] : (VT)0) + (VT)mask[o + 2] * a2;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) df[o + c] = (dd ? dd[o + c] : (VT)0) + (VT)mask[o + c] * a[c];
 }
 
+// what the restriction hands to the coarsest triangular solves: the right-hand
+// side at its place in tile order, and the accumulators cleared there (padding
+// places are zero in all three and stay so)
+struct TileVecs {
+  const int32_t *pos;
+  double *w, *y, *x;
+};
+
 // restriction rc = mask_c * (P' rf); also writes the first smoother iterate
-// d1 = w1 Dinv rc of the coarse level when d1 != nullptr
+// d1 = w1 Dinv rc of the coarse level when d1 != nullptr, or the coarsest
+// solve's vectors instead of rc when t.pos != nullptr
 // 16 lanes cooperate on one coarse row (a coarse node gathers from up to
 // ~100 fine nodes), reduced with cross-lane shuffles.
 template <class VT, class WT>
 __global__ __launch_bounds__(256) void k_restrict(int64_t nc, const int64_t *ptr, const int32_t *col,
                                                   const WT *w, const uint8_t *mask, const VT *rf, VT *rc,
-                                                  const VT *dinv, VT w1, VT *d1) {
+                                                  const VT *dinv, VT w1, VT *d1, TileVecs t) {
   const int64_t j = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 4;
   const int sub = threadIdx.x & 15;
   VT a0 = 0, a1 = 0, a2 = 0;
@@ -396,19 +415,20 @@ __global__ __launch_bounds__(256) void k_restrict(int64_t nc, const int64_t *ptr
     a1 += __shfl_xor(a1, off, 16);
     a2 += __shfl_xor(a2, off, 16);
   }
-  if (j >= nc || sub != 0) return;
-  const int64_t o = 3 * j;
-  a0 *= (VT)mask[o];
-  a1 *= (VT)mask[o + 1];
-  a2 *= (VT)mask[o + 2];
-  rc[o] = a0;
-  rc[o + 1] = a1;
-  rc[o + 2] = a2;
-  if (d1) {
-    d1[o] = w1 * dinv[o] * a0;
-    d1[o + 1] = w1 * dinv[o + 1] * a1;
-    d1[o + 2] = w1 * dinv[o + 2] * a2;
+  if (j >= nc || sub >= 3) return;
+  const int64_t o = 3 * j + sub;
+  const VT a = (sub == 0 ? a0 : sub == 1 ? a1 : a2) * (VT)mask[o];
+  if (t.pos) {
+    const int q = t.pos[o];
+    if (q >= 0) {
+      t.w[q] = (double)a;
+      t.y[q] = 0.0;
+      t.x[q] = 0.0;
+    }
+    return;
   }
+  rc[o] = a;
+  if (d1) d1[o] = w1 * dinv[o] * a;
 }
 
 // V-cycle entry on the finest level: r0 = (VT) r and the first smoother
@@ -445,30 +465,19 @@ __global__ void k_dot(int64_t n, const double *a, const double *b, double *part)
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-// two dot products: s0 = (a - c).b, s1 = a.b
-__global__ void k_dot2(int64_t n, const double *a, const double *c, const double *b, double *part,
-                       int nb) {
-  double s0 = 0, s1 = 0;
-  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
-    const double bb = b[i];
-    s1 += a[i] * bb;
-    if (c) s0 += (a[i] - c[i]) * bb;
-  }
-  __shared__ double sh0[RB], sh1[RB];
-  sh0[threadIdx.x] = s0;
-  sh1[threadIdx.x] = s1;
+// (a - c).b
+__global__ void k_dot_diff(int64_t n, const double *a, const double *c, const double *b, double *part) {
+  double s = 0;
+  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
+    s += (a[i] - c[i]) * b[i];
+  __shared__ double sh[RB];
+  sh[threadIdx.x] = s;
   __syncthreads();
   for (int st = RB / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) {
-      sh0[threadIdx.x] += sh0[threadIdx.x + st];
-      sh1[threadIdx.x] += sh1[threadIdx.x + st];
-    }
+    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    part[blockIdx.x] = sh0[0];
-    part[nb + blockIdx.x] = sh1[0];
-  }
+  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
 __global__ void k_vsum(int64_t n, const double *a, double *part) {
@@ -497,78 +506,89 @@ __global__ void k_sum(const double *part, int nb, double *out) {
   if (threadIdx.x == 0) *out = sh[0];
 }
 
-// ---- CG scalar program ----------------------------------------------------------------
-// scal layout: 0 rd, 1 rdlast, 2 beta, 3 alpha, 4 qKq, 5 rr, 6 tmp0, 7 tmp1
-__global__ void k_cg_beta(const double *part, int nb, double *scal, int first) {
+// ---- CG vector kernels: three per iteration besides the V-cycle and K q ---------------
+// A kernel that needs a dot product adds the partial sums of the kernel before
+// it itself (every workgroup in the same order, so all hold the same value); the
+// residual's partial sums go to the host's memory, which adds them.  With eight
+// vector kernels, two conversions and a copy per iteration the whole of it took
+// 135 / 1,403 us at 5,778 / 337,986 rows (FP64) and 106 / 682 us (mixed), so
+// 129 / 1,357 and 101 / 673 us.
+// scal: 0 r.d of the current direction, 3 alpha, 4 + parity: r.d by iteration
+constexpr int CGB = 512;  // workgroups (and partial sums) of these kernels, at most
+__device__ inline double cg_total(const double *part, int nb, double *sh) {
+  double s = 0;
+  for (int i = threadIdx.x; i < nb; i += RB) s += part[i];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+__device__ inline double cg_block(double s, double *sh) {
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+// partial sums of (r - rlast).d = -alpha Kq.d (0 in the first iteration) and
+// r.d, with d as the V-cycle leaves it
+template <class VT>
+__global__ __launch_bounds__(RB) void k_cg_dots(int64_t n, const double *r, const double *Kq, const VT *d,
+                                                const double *scal, double *part, int first) {
+  __shared__ double sh[4];
   double s0 = 0, s1 = 0;
-  for (int i = threadIdx.x; i < nb; i += RB) {
-    s0 += part[i];
-    s1 += part[nb + i];
+  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
+    const double di = (double)d[i];
+    s1 += r[i] * di;
+    if (!first) s0 += Kq[i] * di;
   }
-  __shared__ double sh0[RB], sh1[RB];
-  sh0[threadIdx.x] = s0;
-  sh1[threadIdx.x] = s1;
-  __syncthreads();
-  for (int st = RB / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) {
-      sh0[threadIdx.x] += sh0[threadIdx.x + st];
-      sh1[threadIdx.x] += sh1[threadIdx.x + st];
-    }
-    __syncthreads();
-  }
+  s0 = cg_block(s0, sh);
+  s1 = cg_block(s1, sh);
   if (threadIdx.x == 0) {
-    // beta = ((r - rlast) . d) / rdlast  (mgpcg_solver_p.m:161), rd = r.d (:166)
-    scal[1] = scal[0];
-    scal[2] = first ? 0.0 : sh0[0] / scal[1];
-    scal[0] = sh1[0];
+    part[blockIdx.x] = first ? 0.0 : -scal[3] * s0;
+    part[gridDim.x + blockIdx.x] = s1;
   }
 }
-
+// beta = ((r - rlast) . d) / rdlast (mgpcg_solver_p.m:161), rd = r.d (:166),
 // q = d + beta q
-__global__ void k_cg_dir(int64_t n, const double *d, double *q, const double *scal) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) q[i] = d[i] + scal[2] * q[i];
-}
-
-// alpha = rd / qKq from the SpMV's partial sums (every block reduces them in
-// the same order, so all blocks hold the same alpha; block 0 records it),
-// then x += alpha q; rlast = r; r -= alpha Kq; partial |r|^2
-__global__ void k_cg_alpha_update(int64_t n, double *x, const double *q, double *r, double *rlast,
-                                  const double *Kq, const double *qpart, int nq, double *scal, double *part) {
-  __shared__ double sh[RB];
-  {
-    double s = 0;
-    for (int i = threadIdx.x; i < nq; i += RB) s += qpart[i];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = RB / 2; st > 0; st >>= 1) {
-      if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-      __syncthreads();
+template <class VT>
+__global__ __launch_bounds__(RB) void k_cg_dir(int64_t n, const VT *d, double *q, const double *part, int nb,
+                                               double *scal, int it) {
+  __shared__ double sh[4];
+  const double rdlast = scal[4 + (it & 1)];
+  const double s0 = it == 1 ? 0.0 : cg_total(part, nb, sh);
+  if (blockIdx.x == 0) {
+    const double rd = cg_total(part + nb, nb, sh);
+    if (threadIdx.x == 0) {
+      scal[0] = rd;
+      scal[4 + ((it + 1) & 1)] = rd;
     }
   }
-  const double qKq = sh[0];
-  const double alpha = scal[0] / qKq;  // alpha = rd / qKq (:173)
-  __syncthreads();
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    scal[4] = qKq;
-    scal[3] = alpha;
+  if (it == 1) {
+    for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) q[i] = (double)d[i];
+  } else {
+    const double beta = s0 / rdlast;
+    for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
+      q[i] = (double)d[i] + beta * q[i];
   }
+}
+
+// alpha = rd / qKq (:173), x += alpha q, r -= alpha Kq; partial |r|^2 to the host
+__global__ __launch_bounds__(RB) void k_cg_update(int64_t n, double *x, const double *q, double *r, const double *Kq,
+                                                  const double *qpart, int nq, double *scal, double *part) {
+  __shared__ double sh[4];
+  const double alpha = scal[0] / cg_total(qpart, nq, sh);
+  if (blockIdx.x == 0 && threadIdx.x == 0) scal[3] = alpha;
   double s = 0;
   for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
     x[i] += alpha * q[i];
-    const double ri = r[i];
-    rlast[i] = ri;
-    const double rn = ri - alpha * Kq[i];
+    const double rn = r[i] - alpha * Kq[i];
     r[i] = rn;
     s += rn * rn;
   }
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int st = RB / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+  s = cg_block(s, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 __global__ void k_axpy(int64_t n, double a, const double *x, double *y) {
@@ -770,6 +790,11 @@ __global__ void k_pack16(int64_t ns, const double *val, uint32_t *out) {
   out[p16_v8(p)] = __float_as_uint((float)val[kval(p, 8)]);
 }
 
+__global__ void k_zero3(int64_t n, double *a, double *b, double *c) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < n) a[i] = b[i] = c[i] = 0.0;
+}
+
 __global__ void k_zero64(int64_t n, double *x) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) x[i] = 0.0;
@@ -864,12 +889,13 @@ void spmv_M(hipStream_t s, Sell &M, const double *x, double *y) {
 }
 void prolong(hipStream_t s, LevelDev &fine, const double *dc, const double *dd, double *df) {
   hipLaunchKernelGGL((k_prolong<double, double>), dim3(nblk(fine.nnod)), dim3(256), 0, s, fine.nnod,
-                     fine.P_ptr.p, fine.P_col.p, fine.P_val.p, fine.vmask.p, dc, dd, df);
+                     fine.P_ptr.p, fine.P_col.p, fine.P_val.p, fine.vmask.p, dc, (const double *)nullptr,
+                     (const int32_t *)nullptr, dd, df);
 }
 void restrict_(hipStream_t s, LevelDev &fine, LevelDev &coarse, const double *rf, double *rc) {
   hipLaunchKernelGGL((k_restrict<double, double>), dim3(nblk(16 * coarse.nnod)), dim3(256), 0, s,
                      coarse.nnod, fine.R_ptr.p, fine.R_col.p, fine.R_val.p, coarse.vmask.p, rf, rc,
-                     (const double *)nullptr, 0.0, (double *)nullptr);
+                     (const double *)nullptr, 0.0, (double *)nullptr, TileVecs{});
 }
 
 static void add_scalar_impl(hipStream_t s, double *a, double v, int64_t n) {
@@ -944,6 +970,7 @@ static void vcycle_impl(m3_ctx *c, VecSet<VT> (*vs)(LevelDev &)) {
     LevelDev &cl = c->L[l + 1];
     VecSet<VT> vc = vs(cl);
     const bool coarsest = (l + 1 == nm - 1);
+    const TileVecs tv = coarsest ? TileVecs{c->chol.dof2pos.p, c->chol.w.p, c->chol.y.p, c->chol.x.p} : TileVecs{};
     const double rb = (double)lv.R_col.n * (sv + 4.0) + (cl.nnod + 1.0) * sizeof(*lv.R_ptr.p) +
                       3.0 * cl.nnod + 3.0 * lv.nnod * sv + 3.0 * cl.nnod * sv * (coarsest ? 1 : 3);
     ProfScope ps(c, 2, true, rb);
@@ -951,26 +978,25 @@ static void vcycle_impl(m3_ctx *c, VecSet<VT> (*vs)(LevelDev &)) {
       launch_timed(k_restrict<double, double>, dim3(nblk(16 * cl.nnod)), dim3(256), s, (int64_t)cl.nnod,
                    (const int64_t *)lv.R_ptr.p, (const int32_t *)lv.R_col.p, (const double *)lv.R_val.p,
                    (const uint8_t *)cl.vmask.p, (const double *)v.r1, vc.r0,
-                   coarsest ? (const double *)nullptr : vc.dinv, WDOWN[0], coarsest ? (double *)nullptr : vc.d);
+                   coarsest ? (const double *)nullptr : vc.dinv, WDOWN[0], coarsest ? (double *)nullptr : vc.d, tv);
     else
       launch_timed(k_restrict<float, float>, dim3(nblk(16 * cl.nnod)), dim3(256), s, (int64_t)cl.nnod,
                    (const int64_t *)lv.R_ptr.p, (const int32_t *)lv.R_col.p, (const float *)lv.R_val32.p,
                    (const uint8_t *)cl.vmask.p, (const float *)v.r1, vc.r0,
-                   coarsest ? (const float *)nullptr : vc.dinv, (float)WDOWN[0], coarsest ? (float *)nullptr : vc.d);
+                   coarsest ? (const float *)nullptr : vc.dinv, (float)WDOWN[0], coarsest ? (float *)nullptr : vc.d, tv);
   }
-  // coarsest: FP64 Cholesky
-  {
-    LevelDev &cl = c->L[nm - 1];
-    const int64_t n3 = 3 * cl.nnod;
-    if constexpr (std::is_same<VT, double>::value) chol_solve_dev(c, cl.r0.p, cl.d.p);
-    else chol_solve_dev32(c, cl.r0f.p, cl.df.p);  // FP64 inside, FP32 at the boundary
-  }
+  // coarsest: FP64 Cholesky, from the tile-ordered right-hand side that the
+  // restriction wrote to the tile-ordered x that the prolongation reads
+  chol_solve_tiles(c, !std::is_same<VT, double>::value);
   for (int l = nm - 2; l >= 0; --l) {
     LevelDev &lv = c->L[l];
     LevelDev &cl = c->L[l + 1];
     VecSet<VT> v = vs(lv);
     VecSet<VT> vc = vs(cl);
     const double *wu = l == 0 ? WUP1 : WUP;
+    const bool coarsest = (l + 1 == nm - 1);
+    const double *xt = coarsest ? c->chol.x.p : nullptr;
+    const int32_t *pos = coarsest ? c->chol.dof2pos.p : nullptr;
     // prolongated correction into dn; three sweeps dn -> d -> dn -> d leave
     // the level's result in d
     {
@@ -980,11 +1006,11 @@ static void vcycle_impl(m3_ctx *c, VecSet<VT> (*vs)(LevelDev &)) {
       if constexpr (std::is_same<VT, double>::value)
         launch_timed(k_prolong<double, double>, dim3(nblk(lv.nnod)), dim3(256), s, (int64_t)lv.nnod,
                      (const int64_t *)lv.P_ptr.p, (const int32_t *)lv.P_col.p, (const double *)lv.P_val.p,
-                     (const uint8_t *)lv.vmask.p, (const double *)vc.d, (const double *)v.dd, v.dn);
+                     (const uint8_t *)lv.vmask.p, (const double *)vc.d, xt, pos, (const double *)v.dd, v.dn);
       else
         launch_timed(k_prolong<float, float>, dim3(nblk(lv.nnod)), dim3(256), s, (int64_t)lv.nnod,
                      (const int64_t *)lv.P_ptr.p, (const int32_t *)lv.P_col.p, (const float *)lv.P_val32.p,
-                     (const uint8_t *)lv.vmask.p, (const float *)vc.d, (const float *)v.dd, v.dn);
+                     (const uint8_t *)lv.vmask.p, (const float *)vc.d, xt, pos, (const float *)v.dd, v.dn);
     }
     const int kind = l == 0 ? pk : 2;
     const double b6 = sweep_bytes<MT>(lv, 4, sv);
@@ -994,7 +1020,9 @@ static void vcycle_impl(m3_ctx *c, VecSet<VT> (*vs)(LevelDev &)) {
   }
 }
 
-void vcycle(m3_ctx *c, const double *r, double *d, int precision) {
+// the cycle on r; the result is left in the finest level's d (df in the mixed
+// form)
+void vcycle(m3_ctx *c, const double *r, int precision) {
   hipStream_t s = c->stream;
   LevelDev &f = c->L[0];
   const int64_t n3 = 3 * f.nnod;
@@ -1005,8 +1033,6 @@ void vcycle(m3_ctx *c, const double *r, double *d, int precision) {
                    f.r0.p, f.d.p);
     }
     vcycle_impl<double, double>(c, vecs64);
-    ProfScope ps(c, 2, true, n3 * 16.0);
-    launch_timed(k_copy, dim3(nblk(n3)), dim3(256), s, n3, (const double *)f.d.p, d);
   } else {
     {
       ProfScope ps(c, 2, true, n3 * (8.0 + 3 * 4.0));
@@ -1014,12 +1040,9 @@ void vcycle(m3_ctx *c, const double *r, double *d, int precision) {
                    (float)WDOWN1[0], f.r0f.p, f.df.p);
     }
     vcycle_impl<B16P, float>(c, vecs32);
-    ProfScope ps(c, 2, true, n3 * 12.0);
-    launch_timed(k_convert<float, double>, dim3(nblk(n3)), dim3(256), s, n3, (const float *)f.df.p, d);
   }
   HIPCHECK(hipGetLastError());
 }
-
 
 // FP32 / BF16 copies of the operators for the mixed-precision V-cycle
 void build_mixed(m3_ctx *c) {
@@ -1069,7 +1092,7 @@ double dot(m3_ctx *c, const double *a, const double *b, int64_t n) {
 
 double dot_diff(m3_ctx *c, const double *a, const double *cvec, const double *b, int64_t n) {
   const int nb = red_blocks(n);
-  hipLaunchKernelGGL(k_dot2, dim3(nb), dim3(RB), 0, c->stream, n, a, cvec, b, c->partial.p, nb);
+  hipLaunchKernelGGL(k_dot_diff, dim3(nb), dim3(RB), 0, c->stream, n, a, cvec, b, c->partial.p);
   hipLaunchKernelGGL(k_sum, dim3(1), dim3(RB), 0, c->stream, c->partial.p, nb, c->scal.p + 8);
   HIPCHECK(hipMemcpyAsync(c->h_scal + 8, c->scal.p + 8, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHECK(hipStreamSynchronize(c->stream));
@@ -1119,8 +1142,19 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
   LevelDev &f = c->L[0];
   const int64_t n3 = 3 * f.nnod;
   const double nfree = (double)f.nfree;
-  double *r = c->cg_r.p, *rl = c->cg_rlast.p, *d = c->cg_d.p, *q = c->cg_q.p, *Kq = c->cg_Kq.p;
-  const int nb = red_blocks(n3);
+  double *r = c->cg_r.p, *q = c->cg_q.p, *Kq = c->cg_Kq.p;
+  const int nb = (int)std::min<int64_t>(CGB, (n3 + RB - 1) / RB);
+  // |r|^2 / nfree from the partial sums in the host's memory
+  auto rms = [&]() {
+    HIPCHECK(hipStreamSynchronize(s));
+    double t = 0;
+    for (int i = 0; i < nb; ++i) t += c->h_part[i];
+    return std::sqrt(t / nfree);
+  };
+  // the coarsest solve's vectors, padding places included (a failed solve may
+  // have left a NaN there)
+  CholTiles &ch = c->chol;
+  hipLaunchKernelGGL(k_zero3, dim3(nblk(ch.w.n)), dim3(256), 0, s, (int64_t)ch.w.n, ch.w.p, ch.y.p, ch.x.p);
   const int32_t *perm = f.K.vperm_p();
   double *xi = perm ? c->cg_x.p : x;  // the iterate in vector order
   // r = b - K x  (masked: fixed entries of b are zeroed); a caller that
@@ -1134,32 +1168,27 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
     SweepVec<double> v{xi, c->cg_b.p, nullptr, 0.0, nullptr, r, nullptr, nullptr};
     launch_sweep<double, double, 2>(s, f.K, f.K.val.p, v);
   }
-  hipLaunchKernelGGL(k_dot, dim3(nb), dim3(RB), 0, s, n3, r, r, c->partial.p);
-  hipLaunchKernelGGL(k_sum, dim3(1), dim3(RB), 0, s, c->partial.p, nb, c->scal.p + 5);
-  HIPCHECK(hipMemcpyAsync(c->h_scal + 5, c->scal.p + 5, sizeof(double), hipMemcpyDeviceToHost, s));
-  HIPCHECK(hipStreamSynchronize(s));
-  double rrms = std::sqrt(c->h_scal[5] / nfree);
+  hipLaunchKernelGGL(k_dot, dim3(nb), dim3(RB), 0, s, n3, r, r, c->h_part);
+  double rrms = rms();
   if (std::isnan(rrms)) throw M3Error(M3_E_NUMERIC, "RHS vector contains NaNs");
   if (!is_abs) tol = tol * rrms;
   if (hist) hist->push_back(rrms);
   int it = 0;
   const int gK = sweep_grid<double>(f.K);  // partial sums of the K q product, one per workgroup of its launch
-  hipLaunchKernelGGL(k_zero64, dim3(nblk(n3)), dim3(256), 0, s, n3, q);  // q = d + 0 q on the first step
+  double *qpart = c->partial.p, *dpart = c->partial.p + c->partial.n / 2;
+  auto iterate = [&](const auto *d) {
+    using VT = std::remove_const_t<std::remove_pointer_t<decltype(d)>>;
+    hipLaunchKernelGGL(k_cg_dots<VT>, dim3(nb), dim3(RB), 0, s, n3, r, Kq, d, c->scal.p, dpart, it == 1 ? 1 : 0);
+    hipLaunchKernelGGL(k_cg_dir<VT>, dim3(nb), dim3(RB), 0, s, n3, d, q, dpart, nb, c->scal.p, it);
+  };
   for (it = 1; it <= itmax; ++it) {
-    vcycle(c, r, d, precision);
-    hipLaunchKernelGGL(k_dot2, dim3(nb), dim3(RB), 0, s, n3, r, it == 1 ? (const double *)nullptr : rl, d,
-                       c->partial.p, nb);
-    hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(RB), 0, s, c->partial.p, nb, c->scal.p, it == 1 ? 1 : 0);
-    hipLaunchKernelGGL(k_cg_dir, dim3(nblk(n3)), dim3(256), 0, s, n3, d, q, c->scal.p);
-    SweepVec<double> v{q, nullptr, nullptr, 0.0, Kq, nullptr, nullptr, c->partial.p};
+    vcycle(c, r, precision);
+    if (precision == M3_PREC_FP64) iterate((const double *)f.d.p);
+    else iterate((const float *)f.df.p);
+    SweepVec<double> v{q, nullptr, nullptr, 0.0, Kq, nullptr, nullptr, qpart};
     launch_sweep<double, double, 9>(s, f.K, f.K.val.p, v);
-    double *upart = c->partial.p + c->partial.n / 2;  // the SpMV's partials stay readable
-    hipLaunchKernelGGL(k_cg_alpha_update, dim3(nb), dim3(RB), 0, s, n3, xi, q, r, rl, Kq, c->partial.p, gK,
-                       c->scal.p, upart);
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(RB), 0, s, upart, nb, c->scal.p + 5);
-    HIPCHECK(hipMemcpyAsync(c->h_scal + 5, c->scal.p + 5, sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHECK(hipStreamSynchronize(s));
-    rrms = std::sqrt(c->h_scal[5] / nfree);
+    hipLaunchKernelGGL(k_cg_update, dim3(nb), dim3(RB), 0, s, n3, xi, q, r, Kq, qpart, gK, c->scal.p, c->h_part);
+    rrms = rms();
     if (hist) hist->push_back(rrms);
     if (std::isnan(rrms)) throw M3Error(M3_E_NUMERIC, "NaN in CG residual");
     if (rrms < tol) break;

@@ -305,6 +305,7 @@ int m3_create(m3_ctx **ctx, int hip_device) {
     HIPCHECK(hipSetDevice(hip_device));
     HIPCHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIPCHECK(hipHostMalloc(&c->h_scal, 64 * sizeof(double)));
+    HIPCHECK(hipHostMalloc(&c->h_part, 512 * sizeof(double)));
     c->scal.alloc(64);
     c->errflag.alloc(1);
     m3::upload_sf_tables();
@@ -327,6 +328,7 @@ void m3_destroy(m3_ctx *c) {
     std::swap(tmp.L, c->L);
   }
   if (c->h_scal) (void)hipHostFree(c->h_scal);
+  if (c->h_part) (void)hipHostFree(c->h_part);
   if (c->ev_start) (void)hipEventDestroy(c->ev_start);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -620,7 +622,7 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
       lv.mask.alloc(n3);
     }
     const size_t n3 = 3 * f.nnod;
-    for (auto *b : {&c->cg_r, &c->cg_rlast, &c->cg_d, &c->cg_q, &c->cg_Kq, &c->cg_x, &c->cg_b, &c->Uv,
+    for (auto *b : {&c->cg_r, &c->cg_q, &c->cg_Kq, &c->cg_x, &c->cg_b, &c->Uv,
                     &c->Zv, &c->Yv, &c->Rhs, &c->Fb, &c->bc_rhs, &c->U0, &c->fbbc, &c->Usol})
       b->alloc(n3);
     for (auto *b : {&c->pr, &c->prlast, &c->pd, &c->pq, &c->pSq, &c->pP, &c->pMd, &c->LiMM, &c->gU0, &c->Psol})

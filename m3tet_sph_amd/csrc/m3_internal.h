@@ -348,8 +348,9 @@ struct m3_ctx {
   DBuf<double> partial;            // per-block partial sums
   DBuf<double> scal;               // device scalars
   double *h_scal = nullptr;        // pinned host mirror
+  double *h_part = nullptr;        // pinned: partial sums that the host adds (512)
   // CG / Patera vectors (3*nnod or nV)
-  DBuf<double> cg_r, cg_rlast, cg_d, cg_q, cg_Kq, cg_x, cg_b;
+  DBuf<double> cg_r, cg_q, cg_Kq, cg_x, cg_b;
   DBuf<double> Uv, Zv, Yv, Rhs;
   DBuf<double> pr, prlast, pd, pq, pSq, pP, pMd;
   DBuf<double> fbbc, gU0;  // Patera: mask (Fb - bc_rhs) and GG' U0, per solve
@@ -490,10 +491,12 @@ void prolong(hipStream_t s, LevelDev &fine, const double *dc, const double *dd, 
 void restrict_(hipStream_t s, LevelDev &fine, LevelDev &coarse, const double *rf, double *rc);
 
 // V-cycle building blocks (templated on FP64 / FP32 vectors in k_sparse.hip)
-void vcycle(m3_ctx *c, const double *r, double *d, int precision);
+void vcycle(m3_ctx *c, const double *r, int precision);
 void chol_factor(m3_ctx *c);
 void chol_solve_dev(m3_ctx *c, const double *rhs, double *x);  // device vectors, coarse level
-void chol_solve_dev32(m3_ctx *c, const float *rhs, float *x);   // the same, FP32 in and out
+// the triangular solves alone, from chol.w to chol.x in tile order (chol.y and
+// chol.x cleared by the caller); tiles32: on the FP32 copies of the tiles
+void chol_solve_tiles(m3_ctx *c, bool tiles32);
 
 // vector helpers
 double dot(m3_ctx *c, const double *a, const double *b, int64_t n);
