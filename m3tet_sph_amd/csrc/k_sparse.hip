@@ -94,15 +94,27 @@ struct SweepVec {
   VT *y, *r_out, *d_out;
   double *part;
 };
+template <class VT>
+struct SweepIn {
+  VT r0 = 0, dinv = 0, x = 0;
+};
 template <class VT, int MODE>
-__device__ inline void sweep_out(const SweepVec<VT> &v, int64_t o, VT kx, double &dot) {
+__device__ inline SweepIn<VT> sweep_in(const SweepVec<VT> &v, int64_t o) {
+  SweepIn<VT> t;
+  if (MODE & 2) t.r0 = v.r0[o];
+  if (MODE & 4) t.dinv = v.dinv[o];
+  if (MODE & 12) t.x = v.x[o];
+  return t;
+}
+template <class VT, int MODE>
+__device__ inline void sweep_out(const SweepVec<VT> &v, const SweepIn<VT> &t, int64_t o, VT kx, double &dot) {
   if (MODE & 1) v.y[o] = kx;
   if (MODE & 2) {
-    const VT q = v.r0[o] - kx;
+    const VT q = t.r0 - kx;
     if (v.r_out) v.r_out[o] = q;
-    if (MODE & 4) v.d_out[o] = v.x[o] + v.w * v.dinv[o] * q;
+    if (MODE & 4) v.d_out[o] = t.x + v.w * t.dinv * q;
   }
-  if (MODE & 8) dot += (double)v.x[o] * (double)kx;
+  if (MODE & 8) dot += (double)t.x * (double)kx;
 }
 // sum of s over the workgroup's NW waves, in order, to part[blockIdx.x]
 template <int NW>
@@ -121,10 +133,15 @@ __device__ inline void block_part(double s, double *sh, double *part) {
 // stored blocks dealt to W waves (wave w takes blocks w, w + W, ...: every load
 // still one contiguous stretch per wave), partial sums added in LDS.  These
 // levels are latency-bound: a vertex row of 65 blocks is a chain of dependent
-// column and vector loads, and one wave per slice leaves the chip empty.  5,778
-// rows, FP64 / BF16: four lanes per row 22.7 us, W = 4 / 8 / 16: 9.5 / 7.8 /
-// 7.9 us and 5.7 / 4.8 / 4.7 us; 43,554 rows: four lanes per row 37.6 and 15.3
-// us, W = 4 / 8 / 16: 26.8 / 23.6 / 20.5 us and 10.3 / 9.3 / 8.6 us.
+// column and vector loads, and one wave per slice leaves the chip empty.  So a
+// lane's blocks, the last ones too, go UNR at a time with all their loads in
+// flight, and the row's own vectors are read first.  One whole iteration,
+// FP64 / mixed, with the remainder block by block and after it (2 16): 5,778
+// rows 121 / 92 us, 23,058 rows 206 / 143; UNR and W 4 16: 107 / 92 and 176 / 127,
+// 2 16: 106 / 91 and 175 / 125, 4 8: 107 / 93 and 181 / 134, 3 8: 108 / 99 and
+// 182 / 136 (43,554 rows below a swept window level: alike).  One wave per
+// slice took 22.7 us per FP64 sweep at 5,778 rows, this 8.8.
+constexpr int SD_UNR = 2, SD_W = 16;
 template <class MT, class VT, int MODE, int W, int UNR>
 __global__ __launch_bounds__(64 * W) void k_sweep(SweepPat K, const MT *__restrict__ val, SweepVec<VT> v) {
   __shared__ VT sh[W][192];
@@ -132,27 +149,30 @@ __global__ __launch_bounds__(64 * W) void k_sweep(SweepPat K, const MT *__restri
   const int64_t q = (int64_t)blockIdx.x * 64 + lane;
   const int64_t g0 = K.slice_ptr[blockIdx.x] >> 6;
   const int len = q < K.n ? K.len[q] : 0;
+  // the row's own vectors, ahead of the long chain
+  const int64_t o = 192 * (int64_t)blockIdx.x + threadIdx.x;
+  SweepIn<VT> in;
+  if (threadIdx.x < 192 && o < 3 * K.n) in = sweep_in<VT, MODE>(v, o);
   VT y0 = 0, y1 = 0, y2 = 0;
-  auto blocks = [&](int k0, auto cnt) {
-    constexpr int N = decltype(cnt)::value;
-    int cc[N];
-    VT x[N][3];
-    Blk<MT, false> b[N];
+  for (int k = w; k < len; k += UNR * W) {
+    int cc[UNR];
+    VT x[UNR][3];
+    Blk<MT, false> b[UNR];
 #pragma unroll
-    for (int u = 0; u < N; ++u) {
-      cc[u] = lds_<false>(K.col + (g0 + k0 + u * W) * 64 + lane);
-      b[u].load(val, g0 + k0 + u * W, lane);
-    }
+    for (int u = 0; u < UNR; ++u)
+      if (k + u * W < len) {
+        cc[u] = lds_<false>(K.col + (g0 + k + u * W) * 64 + lane);
+        b[u].load(val, g0 + k + u * W, lane);
+      }
 #pragma unroll
-    for (int u = 0; u < N; ++u)
+    for (int u = 0; u < UNR; ++u)
+      if (k + u * W < len)
 #pragma unroll
-      for (int j = 0; j < 3; ++j) x[u][j] = v.x[3 * (int64_t)cc[u] + j];
+        for (int j = 0; j < 3; ++j) x[u][j] = v.x[3 * (int64_t)cc[u] + j];
 #pragma unroll
-    for (int u = 0; u < N; ++u) b[u].apply(x[u][0], x[u][1], x[u][2], y0, y1, y2);
-  };
-  int k = w;
-  for (; k + (UNR - 1) * W < len; k += UNR * W) blocks(k, std::integral_constant<int, UNR>{});
-  for (; k < len; k += W) blocks(k, std::integral_constant<int, 1>{});
+    for (int u = 0; u < UNR; ++u)
+      if (k + u * W < len) b[u].apply(x[u][0], x[u][1], x[u][2], y0, y1, y2);
+  }
   sh[w][3 * lane] = y0;
   sh[w][3 * lane + 1] = y1;
   sh[w][3 * lane + 2] = y2;
@@ -162,8 +182,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep(SweepPat K, const MT *__restri
     VT s = sh[0][threadIdx.x];
 #pragma unroll
     for (int j = 1; j < W; ++j) s += sh[j][threadIdx.x];
-    const int64_t o = 192 * (int64_t)blockIdx.x + threadIdx.x;
-    if (o < 3 * K.n) sweep_out<VT, MODE>(v, o, s, dot);
+    if (o < 3 * K.n) sweep_out<VT, MODE>(v, in, o, s, dot);
   }
   if (MODE & 8) {
     __shared__ double ds[W];
@@ -253,7 +272,7 @@ __global__ __launch_bounds__(64 * SW_NW, (std::is_same<MT, double>::value ? 4 : 
     }
     const int64_t o0 = 3 * (int64_t)b * SW_WIN;
     for (int t = threadIdx.x; t < 3 * SW_WIN && o0 + t < 3 * K.n; t += 64 * SW_NW)
-      sweep_out<VT, MODE>(v, o0 + t, ys[t], dot);
+      sweep_out<VT, MODE>(v, sweep_in<VT, MODE>(v, o0 + t), o0 + t, ys[t], dot);
   }
   if (MODE & 8) {
     __shared__ double ds[SW_NW];
@@ -351,34 +370,68 @@ __global__ void k_spmv_M(SellView M, int64_t nrow, const double *x, double *y) {
   y[row] = a;
 }
 
+constexpr int TR_UNR = 4;  // transfer weights per lane in flight
+
 // prolongation with the add of the saved defect: df = dd + mask_f * (P dc);
 // from the coarsest level (pos not NULL) dc is read where the triangular solves
-// left it, pos[dof] in tile order (-1: fixed, 0)
+// left it, pos[dof] in tile order (-1: fixed, 0).  Four lanes per node: the
+// chain of row pointer, column, place and value is the time (one lane per node
+// 11.0 us at 5,778 rows FP64, this 4.2; 337,986 rows FP32 18 -> 13).
 template <class VT, class WT>
 __global__ void k_prolong(int64_t nf, const int64_t *ptr, const int32_t *col, const WT *w,
                           const uint8_t *mask, const VT *dc, const double *xt, const int32_t *pos, const VT *dd,
                           VT *df) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= nf) return;
-  VT a[3] = {0, 0, 0};
-  for (int64_t k = ptr[i]; k < ptr[i + 1]; ++k) {
-    const int64_t c3 = 3 * (int64_t)col[k];
-    const VT wk = (VT)w[k];
+  const int64_t i = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 2;
+  const int sub = threadIdx.x & 3;
+  VT a[3] = {0, 0, 0}, old = 0, m = 0;
+  const int64_t o = 3 * i + sub;
+  if (i < nf) {
+    const int64_t end = ptr[i + 1];
+    int64_t k = ptr[i] + sub;
+    if (sub < 3) {
+      old = dd ? dd[o] : (VT)0;
+      m = (VT)mask[o];
+    }
+    for (; k < end; k += 4 * TR_UNR) {
+      int64_t c3[TR_UNR];
+      VT wk[TR_UNR], v[TR_UNR][3];
+      int q[TR_UNR][3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      VT v;
+      for (int u = 0; u < TR_UNR; ++u)
+        if (k + 4 * u < end) {
+          c3[u] = 3 * (int64_t)col[k + 4 * u];
+          wk[u] = (VT)w[k + 4 * u];
+        }
       if (pos) {
-        const int q = pos[c3 + c];
-        v = q >= 0 ? (VT)xt[q] : (VT)0;
+#pragma unroll
+        for (int u = 0; u < TR_UNR; ++u)
+          if (k + 4 * u < end)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) q[u][c] = pos[c3[u] + c];
+#pragma unroll
+        for (int u = 0; u < TR_UNR; ++u)
+          if (k + 4 * u < end)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) v[u][c] = q[u][c] >= 0 ? (VT)xt[q[u][c]] : (VT)0;
       } else {
-        v = dc[c3 + c];
+#pragma unroll
+        for (int u = 0; u < TR_UNR; ++u)
+          if (k + 4 * u < end)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) v[u][c] = dc[c3[u] + c];
       }
-      a[c] += wk * v;
+#pragma unroll
+      for (int u = 0; u < TR_UNR; ++u)
+        if (k + 4 * u < end)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) a[c] += wk[u] * v[u][c];
     }
   }
-  const int64_t o = 3 * i;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) df[o + c] = (dd ? dd[o + c] : (VT)0) + (VT)mask[o + c] * a[c];
+  for (int off = 2; off > 0; off >>= 1)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) a[c] += __shfl_xor(a[c], off, 4);
+  if (i < nf && sub < 3) df[o] = old + m * (sub == 0 ? a[0] : sub == 1 ? a[1] : a[2]);
 }
 
 // what the restriction hands to the coarsest triangular solves: the right-hand
@@ -393,7 +446,8 @@ struct TileVecs {
 // d1 = w1 Dinv rc of the coarse level when d1 != nullptr, or the coarsest
 // solve's vectors instead of rc when t.pos != nullptr
 // 16 lanes cooperate on one coarse row (a coarse node gathers from up to
-// ~100 fine nodes), reduced with cross-lane shuffles.
+// ~100 fine nodes), reduced with cross-lane shuffles, TR_UNR entries of a lane
+// in flight (5,778 rows FP64 6.8 -> 5.2 us).
 template <class VT, class WT>
 __global__ __launch_bounds__(256) void k_restrict(int64_t nc, const int64_t *ptr, const int32_t *col,
                                                   const WT *w, const uint8_t *mask, const VT *rf, VT *rc,
@@ -402,12 +456,28 @@ __global__ __launch_bounds__(256) void k_restrict(int64_t nc, const int64_t *ptr
   const int sub = threadIdx.x & 15;
   VT a0 = 0, a1 = 0, a2 = 0;
   if (j < nc) {
-    for (int64_t k = ptr[j] + sub; k < ptr[j + 1]; k += 16) {
-      const int64_t f3 = 3 * (int64_t)col[k];
-      const VT wk = (VT)w[k];
-      a0 += wk * rf[f3];
-      a1 += wk * rf[f3 + 1];
-      a2 += wk * rf[f3 + 2];
+    const int64_t end = ptr[j + 1];
+    for (int64_t k = ptr[j] + sub; k < end; k += 16 * TR_UNR) {
+      int64_t f3[TR_UNR];
+      VT wk[TR_UNR], x[TR_UNR][3];
+#pragma unroll
+      for (int u = 0; u < TR_UNR; ++u)
+        if (k + 16 * u < end) {
+          f3[u] = 3 * (int64_t)col[k + 16 * u];
+          wk[u] = (VT)w[k + 16 * u];
+        }
+#pragma unroll
+      for (int u = 0; u < TR_UNR; ++u)
+        if (k + 16 * u < end)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) x[u][c] = rf[f3[u] + c];
+#pragma unroll
+      for (int u = 0; u < TR_UNR; ++u)
+        if (k + 16 * u < end) {
+          a0 += wk[u] * x[u][0];
+          a1 += wk[u] * x[u][1];
+          a2 += wk[u] * x[u][2];
+        }
     }
   }
   for (int off = 8; off > 0; off >>= 1) {
@@ -844,7 +914,7 @@ static void launch_sweep(hipStream_t s, const Sell &K, const MT *val, const Swee
     if (sweep_resident<MT>(K)) go(k_sweep_win<MT, VT, MODE, UNR, true>);
     else go(k_sweep_win<MT, VT, MODE, UNR, false>);
   } else {
-    launch_timed(k_sweep<MT, VT, MODE, 16, 2>, dim3((unsigned)P.nsl), dim3(64 * 16), s, P, val, v);
+    launch_timed(k_sweep<MT, VT, MODE, SD_W, SD_UNR>, dim3((unsigned)P.nsl), dim3(64 * SD_W), s, P, val, v);
   }
 }
 void to_places(hipStream_t s, const LevelDev &lv, const double *x, double *y) {
@@ -888,7 +958,7 @@ void spmv_M(hipStream_t s, Sell &M, const double *x, double *y) {
   hipLaunchKernelGGL(k_spmv_M, dim3(nblk(M.nrow)), dim3(256), 0, s, M.view(), M.nrow, x, y);
 }
 void prolong(hipStream_t s, LevelDev &fine, const double *dc, const double *dd, double *df) {
-  hipLaunchKernelGGL((k_prolong<double, double>), dim3(nblk(fine.nnod)), dim3(256), 0, s, fine.nnod,
+  hipLaunchKernelGGL((k_prolong<double, double>), dim3(nblk(4 * fine.nnod)), dim3(256), 0, s, fine.nnod,
                      fine.P_ptr.p, fine.P_col.p, fine.P_val.p, fine.vmask.p, dc, (const double *)nullptr,
                      (const int32_t *)nullptr, dd, df);
 }
@@ -1004,11 +1074,11 @@ static void vcycle_impl(m3_ctx *c, VecSet<VT> (*vs)(LevelDev &)) {
                         3.0 * lv.nnod + 3.0 * cl.nnod * sv + 3.0 * lv.nnod * sv * 2;
       ProfScope ps(c, 2, true, pb);
       if constexpr (std::is_same<VT, double>::value)
-        launch_timed(k_prolong<double, double>, dim3(nblk(lv.nnod)), dim3(256), s, (int64_t)lv.nnod,
+        launch_timed(k_prolong<double, double>, dim3(nblk(4 * lv.nnod)), dim3(256), s, (int64_t)lv.nnod,
                      (const int64_t *)lv.P_ptr.p, (const int32_t *)lv.P_col.p, (const double *)lv.P_val.p,
                      (const uint8_t *)lv.vmask.p, (const double *)vc.d, xt, pos, (const double *)v.dd, v.dn);
       else
-        launch_timed(k_prolong<float, float>, dim3(nblk(lv.nnod)), dim3(256), s, (int64_t)lv.nnod,
+        launch_timed(k_prolong<float, float>, dim3(nblk(4 * lv.nnod)), dim3(256), s, (int64_t)lv.nnod,
                      (const int64_t *)lv.P_ptr.p, (const int32_t *)lv.P_col.p, (const float *)lv.P_val32.p,
                      (const uint8_t *)lv.vmask.p, (const float *)vc.d, xt, pos, (const float *)v.dd, v.dn);
     }
