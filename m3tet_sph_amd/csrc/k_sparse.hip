@@ -306,24 +306,54 @@ __global__ void k_rhs_in(int64_t n3, const int32_t *perm, const uint8_t *vmask, 
 // G:  y[3*row+c] = mask * sum_k val[c][p] * x[col]        (3x1 blocks)
 // GT: y[row]     = sum_k sum_c val[c][p] * x[3*col+c]     (1x3 blocks)
 // M:  y[row]     = sum_k val[p] * x[col]
-__global__ void k_spmv_G(SellView G, int64_t nrow, const double *x, double *y, const double *mask) {
-  const int64_t row = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (row >= nrow) return;
-  const int64_t base = sell_base(G, row);
-  const int len = G.rowlen[row];
+// Slices of 64 rows with their blocks dealt to a workgroup's waves, SG_UNR blocks
+// of a lane in flight, sums added in LDS: one thread per row is a chain of
+// dependent loads (G: 5,778 rows 10.2 -> 5.3 us, 337,986 rows 30.4 -> 23.5 us).
+// G: y = mask * (G x) (+ add)
+constexpr int SG_W = 4, SG_UNR = 4;
+__global__ __launch_bounds__(64 * SG_W) void k_spmv_G(SellView G, int64_t nrow, const double *x, double *y,
+                                                      const double *mask, const double *add) {
+  __shared__ double sh[SG_W][192];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t row = 64 * (int64_t)blockIdx.x + lane;
   double a0 = 0, a1 = 0, a2 = 0;
-  for (int k = 0; k < len; ++k) {
-    const int64_t p = base + (int64_t)k * 64;
-    const double xv = x[G.col[p]];
-    a0 += G.val[p] * xv;
-    a1 += G.val[G.nslot + p] * xv;
-    a2 += G.val[2 * G.nslot + p] * xv;
+  if (row < nrow) {
+    const int64_t base = sell_base(G, row);
+    const int len = G.rowlen[row];
+    for (int k = w; k < len; k += SG_W * SG_UNR) {
+      int cc[SG_UNR];
+      double g[SG_UNR][3], xv[SG_UNR];
+#pragma unroll
+      for (int u = 0; u < SG_UNR; ++u)
+        if (k + u * SG_W < len) {
+          const int64_t p = base + (int64_t)(k + u * SG_W) * 64;
+          cc[u] = G.col[p];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) g[u][c] = G.val[c * G.nslot + p];
+        }
+#pragma unroll
+      for (int u = 0; u < SG_UNR; ++u)
+        if (k + u * SG_W < len) xv[u] = x[cc[u]];
+#pragma unroll
+      for (int u = 0; u < SG_UNR; ++u)
+        if (k + u * SG_W < len) {
+          a0 += g[u][0] * xv[u];
+          a1 += g[u][1] * xv[u];
+          a2 += g[u][2] * xv[u];
+        }
+    }
   }
-  const int64_t o = 3 * row;
-  if (mask) { a0 *= mask[o]; a1 *= mask[o + 1]; a2 *= mask[o + 2]; }
-  y[o] = a0;
-  y[o + 1] = a1;
-  y[o + 2] = a2;
+  sh[w][3 * lane] = a0;
+  sh[w][3 * lane + 1] = a1;
+  sh[w][3 * lane + 2] = a2;
+  __syncthreads();
+  const int64_t o = 192 * (int64_t)blockIdx.x + threadIdx.x;
+  if (threadIdx.x >= 192 || o >= 3 * nrow) return;
+  double s = sh[0][threadIdx.x];
+#pragma unroll
+  for (int j = 1; j < SG_W; ++j) s += sh[j][threadIdx.x];
+  if (mask) s *= mask[o];
+  y[o] = add ? s + add[o] : s;
 }
 
 // GT with the blocks of each slice split over GTW waves: wave w of a
@@ -332,42 +362,48 @@ __global__ void k_spmv_G(SellView G, int64_t nrow, const double *x, double *y, c
 // LDS.  The pressure rows are few (nVnod) and long: one thread per row left
 // the c1 product at 170 workgroups for 256 CUs.
 constexpr int GTW = 8;
-__global__ __launch_bounds__(64 * GTW) void k_spmv_GT_split(SellView G, int64_t nrow, const double *x,
-                                                            double *y) {
+__device__ inline double spmv_GT_row(const SellView &G, int64_t q, int64_t nrow, const double *x,
+                                     double (*sh)[64]) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t q = (int64_t)blockIdx.x * 64 + lane;  // position in the slices
   double a = 0;
   if (q < nrow) {
     const int64_t row = G.perm ? (int64_t)G.perm[q] : q;
     const int64_t base = G.slice_ptr[q >> 6] + (q & 63);
     const int len = G.rowlen[row];
-    for (int k = w; k < len; k += GTW) {
-      const int64_t p = base + (int64_t)k * 64;
-      const int64_t c3 = 3 * (int64_t)G.col[p];
-      a += G.val[p] * x[c3] + G.val[G.nslot + p] * x[c3 + 1] + G.val[2 * G.nslot + p] * x[c3 + 2];
+    for (int k = w; k < len; k += GTW * SG_UNR) {
+      int cc[SG_UNR];
+      double g[SG_UNR][3], xv[SG_UNR][3];
+#pragma unroll
+      for (int u = 0; u < SG_UNR; ++u)
+        if (k + u * GTW < len) {
+          const int64_t p = base + (int64_t)(k + u * GTW) * 64;
+          cc[u] = G.col[p];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) g[u][c] = G.val[c * G.nslot + p];
+        }
+#pragma unroll
+      for (int u = 0; u < SG_UNR; ++u)
+        if (k + u * GTW < len)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) xv[u][c] = x[3 * (int64_t)cc[u] + c];
+#pragma unroll
+      for (int u = 0; u < SG_UNR; ++u)
+        if (k + u * GTW < len) a += g[u][0] * xv[u][0] + g[u][1] * xv[u][1] + g[u][2] * xv[u][2];
     }
   }
-  __shared__ double sh[GTW][64];
   sh[w][lane] = a;
   __syncthreads();
-  if (w == 0 && q < nrow) {
-    double t = sh[0][lane];
-    for (int j = 1; j < GTW; ++j) t += sh[j][lane];
-    y[G.perm ? (int64_t)G.perm[q] : q] = t;
-  }
+  double t = sh[0][lane];
+#pragma unroll
+  for (int j = 1; j < GTW; ++j) t += sh[j][lane];
+  return t;
 }
-
-__global__ void k_spmv_M(SellView M, int64_t nrow, const double *x, double *y) {
-  const int64_t row = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (row >= nrow) return;
-  const int64_t base = sell_base(M, row);
-  const int len = M.rowlen[row];
-  double a = 0;
-  for (int k = 0; k < len; ++k) {
-    const int64_t p = base + (int64_t)k * 64;
-    a += M.val[p] * x[M.col[p]];
-  }
-  y[row] = a;
+__global__ __launch_bounds__(64 * GTW) void k_spmv_GT_split(SellView G, int64_t nrow, const double *x,
+                                                            double *y) {
+  __shared__ double sh[GTW][64];
+  const int64_t q = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);  // position in the slices
+  const double t = spmv_GT_row(G, q, nrow, x, sh);
+  if (threadIdx.x < 64 && q < nrow) y[G.perm ? (int64_t)G.perm[q] : q] = t;
 }
 
 constexpr int TR_UNR = 4;  // transfer weights per lane in flight
@@ -518,62 +554,29 @@ __global__ void k_convert(int64_t n, const A *x, B *y) {
   if (i < n) y[i] = (B)x[i];
 }
 
-// ---- reductions (deterministic two-stage) -----------------------------------------
+// ---- reductions: partial sums on the device, added by the host or by the kernel that
+// needs them, in a fixed order --------------------------------------------------------
 constexpr int RB = 256;
-
-__global__ void k_dot(int64_t n, const double *a, const double *b, double *part) {
-  double s = 0;
-  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
-    s += a[i] * b[i];
-  __shared__ double sh[RB];
-  sh[threadIdx.x] = s;
+__device__ inline double rb_block(double s, double *sh) {
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
   __syncthreads();
-  for (int st = RB / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-// (a - c).b
-__global__ void k_dot_diff(int64_t n, const double *a, const double *c, const double *b, double *part) {
-  double s = 0;
-  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
-    s += (a[i] - c[i]) * b[i];
-  __shared__ double sh[RB];
-  sh[threadIdx.x] = s;
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
   __syncthreads();
-  for (int st = RB / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
-
-__global__ void k_vsum(int64_t n, const double *a, double *part) {
-  double s = 0;
-  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) s += a[i];
-  __shared__ double sh[RB];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int st = RB / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-__global__ void k_sum(const double *part, int nb, double *out) {
+__device__ inline double rb_total(const double *part, int nb, double *sh) {
   double s = 0;
   for (int i = threadIdx.x; i < nb; i += RB) s += part[i];
-  __shared__ double sh[RB];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int st = RB / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = sh[0];
+  return rb_block(s, sh);
+}
+// a.b, or the sum of a when b is NULL
+__global__ __launch_bounds__(RB) void k_dot(int64_t n, const double *a, const double *b, double *part) {
+  __shared__ double sh[4];
+  double s = 0;
+  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
+    s += b ? a[i] * b[i] : a[i];
+  s = rb_block(s, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 // ---- CG vector kernels: three per iteration besides the V-cycle and K q ---------------
@@ -585,22 +588,6 @@ __global__ void k_sum(const double *part, int nb, double *out) {
 // 129 / 1,357 and 101 / 673 us.
 // scal: 0 r.d of the current direction, 3 alpha, 4 + parity: r.d by iteration
 constexpr int CGB = 512;  // workgroups (and partial sums) of these kernels, at most
-__device__ inline double cg_total(const double *part, int nb, double *sh) {
-  double s = 0;
-  for (int i = threadIdx.x; i < nb; i += RB) s += part[i];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-  __syncthreads();
-  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
-}
-__device__ inline double cg_block(double s, double *sh) {
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-  __syncthreads();
-  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
-}
 // partial sums of (r - rlast).d = -alpha Kq.d (0 in the first iteration) and
 // r.d, with d as the V-cycle leaves it
 template <class VT>
@@ -613,8 +600,8 @@ __global__ __launch_bounds__(RB) void k_cg_dots(int64_t n, const double *r, cons
     s1 += r[i] * di;
     if (!first) s0 += Kq[i] * di;
   }
-  s0 = cg_block(s0, sh);
-  s1 = cg_block(s1, sh);
+  s0 = rb_block(s0, sh);
+  s1 = rb_block(s1, sh);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = first ? 0.0 : -scal[3] * s0;
     part[gridDim.x + blockIdx.x] = s1;
@@ -627,9 +614,9 @@ __global__ __launch_bounds__(RB) void k_cg_dir(int64_t n, const VT *d, double *q
                                                double *scal, int it) {
   __shared__ double sh[4];
   const double rdlast = scal[4 + (it & 1)];
-  const double s0 = it == 1 ? 0.0 : cg_total(part, nb, sh);
+  const double s0 = it == 1 ? 0.0 : rb_total(part, nb, sh);
   if (blockIdx.x == 0) {
-    const double rd = cg_total(part + nb, nb, sh);
+    const double rd = rb_total(part + nb, nb, sh);
     if (threadIdx.x == 0) {
       scal[0] = rd;
       scal[4 + ((it + 1) & 1)] = rd;
@@ -648,7 +635,7 @@ __global__ __launch_bounds__(RB) void k_cg_dir(int64_t n, const VT *d, double *q
 __global__ __launch_bounds__(RB) void k_cg_update(int64_t n, double *x, const double *q, double *r, const double *Kq,
                                                   const double *qpart, int nq, double *scal, double *part) {
   __shared__ double sh[4];
-  const double alpha = scal[0] / cg_total(qpart, nq, sh);
+  const double alpha = scal[0] / rb_total(qpart, nq, sh);
   if (blockIdx.x == 0 && threadIdx.x == 0) scal[3] = alpha;
   double s = 0;
   for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) {
@@ -657,7 +644,7 @@ __global__ __launch_bounds__(RB) void k_cg_update(int64_t n, double *x, const do
     r[i] = rn;
     s += rn * rn;
   }
-  s = cg_block(s, sh);
+  s = rb_block(s, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
@@ -711,6 +698,123 @@ __global__ __launch_bounds__(64 * SP_W) void k_spmv1(SellView A, int64_t nrow, c
   if (w == 0 && q < nrow) y[q] = a;
 }
 
+// ---- Patera pressure iteration (flow3d_patera_mg_sph_p.m:476-560) ----------------------
+// Four launches besides G q and the velocity solve, and one read by the host, the
+// norm at the end: a launch that needs a dot product or a mean adds the partial
+// sums of the launch before it, and the mean that is taken out of a sum comes from
+// the sums of its terms.  Against 17 vector launches with six blocking reads, 27
+// iterations within a whole solve at 5,778 nodes: 24.0 -> 20.7 ms; at 337,986
+// nodes, 18 iterations of a time step: idle time 13.0 -> 6.0 ms.
+// scal: PP_RD + parity: r.d by iteration
+constexpr int PP_RD = 24, PP_BLOCKS = 1024;
+// d = p + w LiMM (r - M p), p = LiMM r (precondition_P); per-workgroup sums of
+// (r - rlast).d, r.d, d and the last direction q (the first and last 0 in a restart)
+__global__ __launch_bounds__(64 * SP_W) void k_pp_prec(SellView M, int64_t n, const double *r, const double *rl,
+                                                       const double *LiMM, const double *q, double wm, double *d,
+                                                       double *part, int restart) {
+  __shared__ double sh[SP_W][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double s[4] = {0, 0, 0, 0};
+  for (int64_t b = blockIdx.x; 64 * b < n; b += gridDim.x) {
+    const int64_t i = 64 * b + lane;
+    double a = 0;
+    if (i < n) {
+      const int64_t base = sell_base(M, i);
+      const int len = M.rowlen[i];
+#pragma unroll 4
+      for (int k = w; k < len; k += SP_W) {
+        const int64_t p = base + (int64_t)k * 64;
+        const int64_t j = M.col[p];
+        a += M.val[p] * (LiMM[j] * r[j]);
+      }
+    }
+    __syncthreads();
+    sh[w][lane] = a;
+    __syncthreads();
+    if (w == 0 && i < n) {
+      const double Mp = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
+      const double ri = r[i], l = LiMM[i], di = l * ri + wm * (l * (ri - Mp));
+      d[i] = di;
+      if (!restart) {
+        s[0] += (ri - rl[i]) * di;
+        s[3] += q[i];
+      }
+      s[1] += ri * di;
+      s[2] += di;
+    }
+  }
+  if (w != 0) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    for (int off = 32; off > 0; off >>= 1) s[j] += __shfl_xor(s[j], off, 64);
+    if (lane == 0) part[j * gridDim.x + blockIdx.x] = s[j];
+  }
+}
+// q = d + beta q less its mean; beta = (r - rlast).d / rdlast
+__global__ __launch_bounds__(RB) void k_pp_dir(int64_t n, const double *d, double *q, const double *part, int nb,
+                                               double *scal, int ip, int restart) {
+  __shared__ double sh[4];
+  const double rdlast = scal[PP_RD + ((ip + 1) & 1)];
+  double t[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) t[j] = rb_total(part + j * nb, nb, sh);
+  if (blockIdx.x == 0 && threadIdx.x == 0) scal[PP_RD + (ip & 1)] = t[1];
+  const double beta = restart ? 0.0 : t[0] / rdlast;
+  const double m = (t[2] + beta * t[3]) / (double)n;
+  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
+    q[i] = (restart ? d[i] : d[i] + beta * q[i]) - m;
+}
+// Sq = G' z; per-workgroup sums of q.Sq, Sq and r
+__global__ __launch_bounds__(64 * GTW) void k_pp_S(SellView G, int64_t n, const double *z, const double *q,
+                                                   const double *r, double *Sq, double *part) {
+  __shared__ double sh[GTW][64];
+  double s[3] = {0, 0, 0};
+  for (int64_t b = blockIdx.x; 64 * b < n; b += gridDim.x) {
+    const int64_t k = 64 * b + (threadIdx.x & 63);
+    __syncthreads();
+    const double t = spmv_GT_row(G, k, n, z, sh);
+    if (threadIdx.x < 64 && k < n) {
+      const int64_t i = G.perm ? (int64_t)G.perm[k] : k;
+      Sq[i] = t;
+      s[0] += q[i] * t;
+      s[1] += t;
+      s[2] += r[i];
+    }
+  }
+  if (threadIdx.x >= 64) return;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    for (int off = 32; off > 0; off >>= 1) s[j] += __shfl_xor(s[j], off, 64);
+    if (threadIdx.x == 0) part[j * gridDim.x + blockIdx.x] = s[j];
+  }
+}
+// alpha = rd / q.Sq; P += alpha q, U += alpha Z, r -= alpha Sq and r's mean;
+// partial |r|^2 to the host
+__global__ __launch_bounds__(RB) void k_pp_update(int64_t n, int64_t n3, double *P, const double *q, double *U,
+                                                  const double *Z, double *r, double *rl, const double *Sq,
+                                                  const double *part, int nb, const double *scal, int ip,
+                                                  double *out) {
+  __shared__ double sh[4];
+  double t[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) t[j] = rb_total(part + j * nb, nb, sh);
+  const double alpha = scal[PP_RD + (ip & 1)] / t[0];
+  const double m = (t[2] - alpha * t[1]) / (double)n;
+  double s = 0;
+  for (int64_t i = blockIdx.x * (int64_t)RB + threadIdx.x; i < n3; i += (int64_t)gridDim.x * RB) {
+    U[i] += alpha * Z[i];
+    if (i < n) {
+      P[i] += alpha * q[i];
+      const double ri = r[i], rn = ri - alpha * Sq[i] - m;
+      rl[i] = ri;
+      r[i] = rn;
+      s += rn * rn;
+    }
+  }
+  s = rb_block(s, sh);
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
+}
+
 // ---- Jacobi-preconditioned CG on a scalar matrix (pcg_solver_p.m:49-186) --------------
 // Two launches per iteration and no host in between: the direction and the
 // product, then the update.  A workgroup that needs a dot product adds the
@@ -721,22 +825,10 @@ __global__ __launch_bounds__(64 * SP_W) void k_spmv1(SellView A, int64_t nrow, c
 // and a blocking read per iteration took 55 us at 43,554 rows, this 20.
 // state: 0 r.d of the current direction, 1 |r|^2, 2 iterations done,
 // 3 stopped (1 converged, 2 NaN)
-constexpr int PC_T = 256;
-__device__ inline double pc_total(const double *part, int nb, double *sh) {
-  double s = 0;
-  for (int i = threadIdx.x; i < nb; i += PC_T) s += part[i];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-  __syncthreads();
-  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
-}
+constexpr int PC_T = RB;
 __device__ inline void pc_part(double s, double *part, double *sh) {
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  s = rb_block(s, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 // partial sums: |r|^2 at up, (r - rlast).d at up + nu, r.d at up + 2 nu
 __global__ __launch_bounds__(PC_T) void k_pcg_start(int64_t n, const double *r, const double *Adi, double *up, int nu) {
@@ -819,7 +911,7 @@ __global__ __launch_bounds__(PC_T) void k_pcg_update(int64_t n, const double *q,
                                                      int nu, double *state, int it) {
   __shared__ double sh[4];
   if (state[3] != 0.0) return;
-  const double alpha = state[0] / pc_total(qp, nq, sh);
+  const double alpha = state[0] / rb_total(qp, nq, sh);
   if (blockIdx.x == 0 && threadIdx.x == 0) state[2] = it;
   double rr = 0, s0 = 0, s1 = 0;
   for (int64_t i = blockIdx.x * (int64_t)PC_T + threadIdx.x; i < n; i += (int64_t)gridDim.x * PC_T) {
@@ -838,7 +930,7 @@ __global__ __launch_bounds__(PC_T) void k_pcg_update(int64_t n, const double *q,
 __global__ __launch_bounds__(PC_T) void k_pcg_look(const double *up, int nu, double *state, double rr_stop) {
   __shared__ double sh[4];
   if (state[3] != 0.0) return;
-  const double rr = pc_total(up, nu, sh);
+  const double rr = rb_total(up, nu, sh);
   if (threadIdx.x == 0) {
     state[1] = rr;
     if (state[2] > 0.0 && !(rr >= rr_stop)) state[3] = rr < rr_stop ? 1.0 : 2.0;
@@ -947,16 +1039,15 @@ void spmv_K(hipStream_t s, LevelDev &lv, const double *x, double *y) {
   to_nodes(s, lv, lv.r1.p, y);
 }
 
-void spmv_G(hipStream_t s, Sell &G, const double *q, double *y, const double *mask) {
-  hipLaunchKernelGGL(k_spmv_G, dim3(nblk(G.nrow)), dim3(256), 0, s, G.view(), G.nrow, q, y, mask);
+void spmv_G(hipStream_t s, Sell &G, const double *q, double *y, const double *mask, const double *add) {
+  hipLaunchKernelGGL(k_spmv_G, dim3((unsigned)((G.nrow + 63) / 64)), dim3(64 * SG_W), 0, s, G.view(), G.nrow, q, y,
+                     mask, add);
 }
 void spmv_GT(hipStream_t s, Sell &GT, const double *z, double *y) {
   hipLaunchKernelGGL(k_spmv_GT_split, dim3((unsigned)((GT.nrow + 63) / 64)), dim3(64 * GTW), 0, s, GT.view(),
                      GT.nrow, z, y);
 }
-void spmv_M(hipStream_t s, Sell &M, const double *x, double *y) {
-  hipLaunchKernelGGL(k_spmv_M, dim3(nblk(M.nrow)), dim3(256), 0, s, M.view(), M.nrow, x, y);
-}
+void spmv_M(hipStream_t s, Sell &M, const double *x, double *y) { spmv_scalar(s, M.view(), M.nrow, x, y); }
 void prolong(hipStream_t s, LevelDev &fine, const double *dc, const double *dd, double *df) {
   hipLaunchKernelGGL((k_prolong<double, double>), dim3(nblk(4 * fine.nnod)), dim3(256), 0, s, fine.nnod,
                      fine.P_ptr.p, fine.P_col.p, fine.P_val.p, fine.vmask.p, dc, (const double *)nullptr,
@@ -1144,39 +1235,22 @@ void build_mixed(m3_ctx *c) {
 }
 
 // ---- dot products and vector helpers ----------------------------------------------------
-static int red_blocks(int64_t n) {
-  int64_t b = (n + RB - 1) / RB;
-  if (b > 1024) b = 1024;
-  if (b < 1) b = 1;
-  return (int)b;
+static int red_blocks(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(CGB, (n + RB - 1) / RB)); }
+// the sum of the nb partial sums that the stream's last kernels leave in h_part
+static double host_sum(m3_ctx *c, int nb) {
+  HIPCHECK(hipStreamSynchronize(c->stream));
+  double t = 0;
+  for (int i = 0; i < nb; ++i) t += c->h_part[i];
+  return t;
 }
 
 double dot(m3_ctx *c, const double *a, const double *b, int64_t n) {
   const int nb = red_blocks(n);
-  hipLaunchKernelGGL(k_dot, dim3(nb), dim3(RB), 0, c->stream, n, a, b, c->partial.p);
-  hipLaunchKernelGGL(k_sum, dim3(1), dim3(RB), 0, c->stream, c->partial.p, nb, c->scal.p + 8);
-  HIPCHECK(hipMemcpyAsync(c->h_scal + 8, c->scal.p + 8, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(hipStreamSynchronize(c->stream));
-  return c->h_scal[8];
+  hipLaunchKernelGGL(k_dot, dim3(nb), dim3(RB), 0, c->stream, n, a, b, c->h_part);
+  return host_sum(c, nb);
 }
 
-double dot_diff(m3_ctx *c, const double *a, const double *cvec, const double *b, int64_t n) {
-  const int nb = red_blocks(n);
-  hipLaunchKernelGGL(k_dot_diff, dim3(nb), dim3(RB), 0, c->stream, n, a, cvec, b, c->partial.p);
-  hipLaunchKernelGGL(k_sum, dim3(1), dim3(RB), 0, c->stream, c->partial.p, nb, c->scal.p + 8);
-  HIPCHECK(hipMemcpyAsync(c->h_scal + 8, c->scal.p + 8, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(hipStreamSynchronize(c->stream));
-  return c->h_scal[8];
-}
-
-double mean(m3_ctx *c, const double *a, int64_t n) {
-  const int nb = red_blocks(n);
-  hipLaunchKernelGGL(k_vsum, dim3(nb), dim3(RB), 0, c->stream, n, a, c->partial.p);
-  hipLaunchKernelGGL(k_sum, dim3(1), dim3(RB), 0, c->stream, c->partial.p, nb, c->scal.p + 8);
-  HIPCHECK(hipMemcpyAsync(c->h_scal + 8, c->scal.p + 8, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHECK(hipStreamSynchronize(c->stream));
-  return c->h_scal[8] / (double)n;
-}
+double mean(m3_ctx *c, const double *a, int64_t n) { return dot(c, a, nullptr, n) / (double)n; }
 
 // bit 32 of flag when x holds a NaN
 __global__ void k_nan_flag(int64_t n, const double *x, int *flag) {
@@ -1213,14 +1287,8 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
   const int64_t n3 = 3 * f.nnod;
   const double nfree = (double)f.nfree;
   double *r = c->cg_r.p, *q = c->cg_q.p, *Kq = c->cg_Kq.p;
-  const int nb = (int)std::min<int64_t>(CGB, (n3 + RB - 1) / RB);
-  // |r|^2 / nfree from the partial sums in the host's memory
-  auto rms = [&]() {
-    HIPCHECK(hipStreamSynchronize(s));
-    double t = 0;
-    for (int i = 0; i < nb; ++i) t += c->h_part[i];
-    return std::sqrt(t / nfree);
-  };
+  const int nb = red_blocks(n3);
+  auto rms = [&]() { return std::sqrt(host_sum(c, nb) / nfree); };
   // the coarsest solve's vectors, padding places included (a failed solve may
   // have left a NaN there)
   CholTiles &ch = c->chol;
@@ -1271,6 +1339,26 @@ int mgpcg_run(m3_ctx *c, double *x, const double *b, double tol, bool is_abs, in
 void spmv_scalar(hipStream_t s, SellView A, int64_t n, const double *x, double *y) {
   hipLaunchKernelGGL(k_spmv1, dim3((unsigned)((n + 63) / 64)), dim3(64 * SP_W), 0, s, A, n, x, y);
   HIPCHECK(hipGetLastError());
+}
+
+// the next direction of the pressure iteration, of the ip-th iteration
+void patera_direction(m3_ctx *c, int64_t n, double wm, bool restart, int ip) {
+  hipStream_t s = c->stream;
+  const int nb = (int)std::min<int64_t>(PP_BLOCKS, (n + 63) / 64);
+  hipLaunchKernelGGL(k_pp_prec, dim3(nb), dim3(64 * SP_W), 0, s, c->M.view(), n, c->pr.p, c->prlast.p, c->LiMM.p,
+                     c->pq.p, wm, c->pd.p, c->partial.p, restart ? 1 : 0);
+  hipLaunchKernelGGL(k_pp_dir, dim3(red_blocks(n)), dim3(RB), 0, s, n, c->pd.p, c->pq.p, c->partial.p, nb, c->scal.p,
+                     ip, restart ? 1 : 0);
+}
+// the step along it with z = K^-1 G q: P, U, the residual; returns |r|
+double patera_step(m3_ctx *c, int64_t n, int64_t n3, double *U, const double *z, int ip) {
+  hipStream_t s = c->stream;
+  const int nb = (int)std::min<int64_t>(PP_BLOCKS, (n + 63) / 64), ng = red_blocks(n3);
+  hipLaunchKernelGGL(k_pp_S, dim3(nb), dim3(64 * GTW), 0, s, c->GT.view(), n, z, c->pq.p, c->pr.p, c->pSq.p,
+                     c->partial.p);
+  hipLaunchKernelGGL(k_pp_update, dim3(ng), dim3(RB), 0, s, n, n3, c->pP.p, c->pq.p, U, z, c->pr.p, c->prlast.p,
+                     c->pSq.p, c->partial.p, nb, c->scal.p, ip, c->h_part);
+  return std::sqrt(host_sum(c, ng));
 }
 
 // pcg_solver_p.m:49-186 with the 'diag' preconditioner (Polak-Ribiere beta,

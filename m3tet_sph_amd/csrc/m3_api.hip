@@ -625,7 +625,7 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
     for (auto *b : {&c->cg_r, &c->cg_q, &c->cg_Kq, &c->cg_x, &c->cg_b, &c->Uv,
                     &c->Zv, &c->Yv, &c->Rhs, &c->Fb, &c->bc_rhs, &c->U0, &c->fbbc, &c->Usol})
       b->alloc(n3);
-    for (auto *b : {&c->pr, &c->prlast, &c->pd, &c->pq, &c->pSq, &c->pP, &c->pMd, &c->LiMM, &c->gU0, &c->Psol})
+    for (auto *b : {&c->pr, &c->prlast, &c->pd, &c->pq, &c->pSq, &c->pP, &c->LiMM, &c->gU0, &c->Psol})
       b->alloc(f.nV);
     c->visc.alloc(f.nnod);
     c->dens.alloc(f.nnod);
@@ -877,8 +877,7 @@ static void do_patera(m3_ctx *c, double *U, double *P, const m3_patera_opts *o, 
   double t_vel = 0, t_pres = 0;
   auto t_start = clk::now();
   double *Uf = c->Uv.p, *Z = c->Zv.p, *Y = c->Yv.p, *Rhs = c->Rhs.p;
-  double *r = c->pr.p, *rl = c->prlast.p, *d = c->pd.p, *q = c->pq.p, *Sq = c->pSq.p, *Pd = c->pP.p,
-         *Md = c->pMd.p;
+  double *r = c->pr.p, *q = c->pq.p, *Pd = c->pP.p;
   DBuf<double> &fbbc = c->fbbc, &gU0 = c->gU0;
   // fbbc = mask (Fb - bc_rhs); gU0 = GG' U0
   m3::copy(s, c->Fb.p, fbbc.p, n3);
@@ -902,8 +901,7 @@ static void do_patera(m3_ctx *c, double *U, double *P, const m3_patera_opts *o, 
     c->Uv.zero(s);
   }
   auto rhs_of_P = [&]() {  // Rhs = mask (Fb + GG P - bc_rhs)
-    m3::spmv_G(s, c->G, Pd, Rhs, f.mask.p);
-    m3::axpy(s, 1.0, fbbc.p, Rhs, n3);
+    m3::spmv_G(s, c->G, Pd, Rhs, f.mask.p, fbbc.p);
   };
   auto pres_res = [&](bool rm0) {  // r = -GG' U (U = Uf + U0), mean removed
     m3::spmv_GT(s, c->GT, Uf, r);
@@ -940,45 +938,26 @@ static void do_patera(m3_ctx *c, double *U, double *P, const m3_patera_opts *o, 
   const double tol_U_abs = rtol_U * tol_Pat;
   int nitZ = 0, itPat = 0;
   bool restart = true, conv_problem = false;
-  double rd = 0, norm_rP0 = norm_rP, tolZ = 0;
-  int it0 = 1;
+  double norm_rP0 = norm_rP, tolZ = 0;
+  int it0 = 1, ip = 0;
   for (int pass_out = 0;; ++pass_out) {
   for (itPat = it0; itPat <= o->itmax_Pat; ++itPat) {
     auto tp = clk::now();
-    // d = r ./ LMM; d += w LiMM (r - MM d)   (precondition_P, pc_Pat = 3)
-    m3::scale_mask(s, r, c->LiMM.p, d, nV);
-    m3::spmv_M(s, c->M, d, Md);
-    m3::copy(s, r, Sq, nV);
-    m3::axpy(s, -1.0, Md, Sq, nV);
-    m3::scale_mask(s, Sq, c->LiMM.p, Sq, nV);
-    m3::axpy(s, wMM, Sq, d, nV);
+    // d = r ./ LMM; d += w LiMM (r - MM d)   (precondition_P, pc_Pat = 3); the
+    // search direction q, its mean removed
     if (restart) {
-      m3::copy(s, d, q, nV);
-      restart = false;
       norm_rP0 = norm_rP;
       tolZ = rtol_U * std::max(rtol_restart * norm_rP0, tol_Pat);
-    } else {
-      const double rdlast = rd;
-      const double beta = m3::dot_diff(c, r, rl, d, nV) / rdlast;
-      m3::xpby(s, d, beta, q, nV);
     }
-    m3::add_scalar(s, q, -m3::mean(c, q, nV), nV);
-    rd = m3::dot(c, r, d, nV);
+    m3::patera_direction(c, nV, wMM, restart, ++ip);
+    restart = false;
     m3::spmv_G(s, c->G, q, Y, f.mask.p);
     c->Zv.zero(s);
     t_pres += secs(tp, clk::now());
     nitZ += vel_solve(Z, Y, tolZ, true, true);
     tp = clk::now();
-    m3::spmv_GT(s, c->GT, Z, Sq);
-    const double qSq = m3::dot(c, q, Sq, nV);
-    m3::copy(s, r, rl, nV);
-    const double alpha = rd / qSq;
-    m3::axpy(s, alpha, q, Pd, nV);
-    m3::axpy(s, alpha, Z, Uf, n3);
-    m3::axpy(s, -alpha, Sq, r, nV);
-    m3::add_scalar(s, r, -m3::mean(c, r, nV), nV);
     const double norm_rP_last = norm_rP;
-    norm_rP = normdf(r, nV, (double)nV);
+    norm_rP = m3::patera_step(c, nV, n3, Uf, Z, ip) / std::sqrt((double)nV);
     const double norm_rP_min = std::min(norm_rP_last, norm_rP);
     t_pres += secs(tp, clk::now());
     if (norm_rP < tol_Pat && itPat >= o->itmin_Pat) break;

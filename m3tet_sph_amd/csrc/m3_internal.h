@@ -352,7 +352,7 @@ struct m3_ctx {
   // CG / Patera vectors (3*nnod or nV)
   DBuf<double> cg_r, cg_q, cg_Kq, cg_x, cg_b;
   DBuf<double> Uv, Zv, Yv, Rhs;
-  DBuf<double> pr, prlast, pd, pq, pSq, pP, pMd;
+  DBuf<double> pr, prlast, pd, pq, pSq, pP;
   DBuf<double> fbbc, gU0;  // Patera: mask (Fb - bc_rhs) and GG' U0, per solve
   // solution of the last Stokes solve, kept on the device (U with the BC
   // values, rotated frame; P)
@@ -484,7 +484,7 @@ void spmv_K(hipStream_t s, LevelDev &lv, const double *x, double *y);  // node o
 // vectors of a level between the node order and K's vector order
 void to_places(hipStream_t s, const LevelDev &lv, const double *x, double *y);
 void to_nodes(hipStream_t s, const LevelDev &lv, const double *x, double *y);
-void spmv_G(hipStream_t s, Sell &G, const double *q, double *y, const double *mask);
+void spmv_G(hipStream_t s, Sell &G, const double *q, double *y, const double *mask, const double *add = nullptr);
 void spmv_GT(hipStream_t s, Sell &GT, const double *z, double *y);
 void spmv_M(hipStream_t s, Sell &M, const double *x, double *y);
 void prolong(hipStream_t s, LevelDev &fine, const double *dc, const double *dd, double *df);
@@ -500,7 +500,6 @@ void chol_solve_tiles(m3_ctx *c, bool tiles32);
 
 // vector helpers
 double dot(m3_ctx *c, const double *a, const double *b, int64_t n);
-double dot_diff(m3_ctx *c, const double *a, const double *b, const double *d, int64_t n);
 void axpy(hipStream_t s, double a, const double *x, double *y, int64_t n);
 void slm_advect(m3_ctx *c, const double *Ux, const double *Uy, const double *Uz, double *T, double dt,
                 const m3_slm_opts *opts, m3_slm_info *info);
@@ -512,6 +511,8 @@ void xpby(hipStream_t s, const double *x, double b, double *y, int64_t n);  // y
 void copy(hipStream_t s, const double *x, double *y, int64_t n);
 void scale_mask(hipStream_t s, const double *x, const double *m, double *y, int64_t n);
 double mean(m3_ctx *c, const double *a, int64_t n);
+void patera_direction(m3_ctx *c, int64_t n, double wm, bool restart, int ip);
+double patera_step(m3_ctx *c, int64_t n, int64_t n3, double *U, const double *z, int ip);
 void add_scalar(hipStream_t s, double *a, double v, int64_t n);
 void scal(hipStream_t s, double a, double *y, int64_t n);
 void build_mixed(m3_ctx *c);
