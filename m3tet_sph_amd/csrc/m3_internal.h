@@ -213,7 +213,8 @@ struct CholTiles {
   DBuf<int32_t> diagtile;        // T: tile index of (J,J)
   // factorisation: tile tasks by dependency level
   int nlev = 0;
-  std::vector<int32_t> h_lev_ptr, h_upd_ptr, h_trsm_ptr;
+  std::vector<int32_t> h_lev_ptr, h_trsm_ptr;
+  std::vector<int32_t> h_upd_ptr;             // per level: chunks by levels before the last, by the last one
   DBuf<int32_t> lev_cols, upd_tile, upd_pairs, trsm_tile, trsm_col;
   DBuf<int64_t> upd_pair_ptr, upd_pair_end;  // per update chunk: pair range
   // supernodes: explicit inverse of each block's diagonal part
