@@ -328,80 +328,80 @@ __device__ inline void tile_mm_mf(const double *A, const double *B, bool transB,
   __syncthreads();
   mf_lds(sA, sB, m, threadIdx.x >> 6);
 }
-// sum_p A_p op(B_p) over the tile pairs p0 <= p < p1 (op(B) = B' when
-// transB), 512 threads in two groups of four waves that take turns: in phase
-// s group s&1 loads pair s into its own LDS buffers while the other group
-// multiplies pair s-1, so the loads of one pair overlap the matrix-core
-// products of the previous one (the products of a 64x64 tile pair take
-// 64 v_mfma_f64_16x16x4 per wave, about as long as the loads).  Each group
-// accumulates its own pairs; on return sA[0][r][c] holds the whole sum, with
-// every thread past the final barrier.
-__device__ inline void pair_sum_2g(const double *Abase, const double *Bbase, const int32_t *pairs, int64_t p0,
-                                   int64_t p1, bool transB, double (*sA)[TS][TS + 1], double (*sB)[TS][TS + 1]) {
-  const int g = threadIdx.x >> 8, lt = threadIdx.x & 255, w = (threadIdx.x >> 6) & 3;
+// sum_p A_p op(B_p) over the tile pairs p0 <= p < p1 (op(B) = B' when transB);
+// the loads of a pair are in flight during the products of the one before it
+// (64 v_mfma_f64_16x16x4 per wave, 1.7 us).  66 KB of LDS, so that two
+// workgroups share a CU and one's first loads and last stores overlap the
+// other's products: one workgroup of two groups of four waves that took turns
+// (133 KB) left the matrix cores idle half of a chunk of four pairs.  1,844 tile
+// columns: updates 13.2 -> 11.2 ms, Z 2.42 -> 1.96 ms, the factorisation 18.16 ->
+// 15.7 ms (two groups with the loads a pair further ahead: 20.1 ms; chunks that
+// share a tile dealt to one XCD: 19.2 ms).
+// On return sA[r][c] holds the sum, with every thread past the final barrier.
+struct PairLds {
+  double A[TS][TS + 1], B[TS][TS + 1];
+};
+__device__ inline void pair_sum(const double *Abase, const double *Bbase, const int32_t *pairs, int64_t p0,
+                                int64_t p1, bool transB, PairLds &lds) {
+  auto &sA = lds.A;
+  auto &sB = lds.B;
   MfAcc m;
   mf_zero(m);
-  const int64_t n = p1 - p0;
-  for (int64_t st = 0; st <= n; ++st) {
-    if ((st & 1) == g && st < n) {
-      const double *A = Abase + (int64_t)pairs[2 * (p0 + st)] * TT;
-      const double *B = Bbase + (int64_t)pairs[2 * (p0 + st) + 1] * TT;
-      double va[TT / 256], vb[TT / 256];
+  double va[TT / 256], vb[TT / 256];
+  auto fetch = [&](int64_t p) {
+    const double *A = Abase + (int64_t)pairs[2 * p] * TT;
+    const double *B = Bbase + (int64_t)pairs[2 * p + 1] * TT;
 #pragma unroll
-      for (int q = 0; q < TT / 256; ++q) {
-        va[q] = A[lt + 256 * q];
-        vb[q] = B[lt + 256 * q];
-      }
-#pragma unroll
-      for (int q = 0; q < TT / 256; ++q) {
-        const int t = lt + 256 * q, r = t & 63, c = t >> 6;
-        sA[g][r][c] = va[q];
-        if (transB) sB[g][r][c] = vb[q];
-        else sB[g][c][r] = vb[q];
-      }
+    for (int q = 0; q < TT / 256; ++q) {
+      va[q] = A[threadIdx.x + 256 * q];
+      vb[q] = B[threadIdx.x + 256 * q];
     }
-    if (st >= 1 && ((st - 1) & 1) == g) mf_lds(sA[g], sB[g], m, w);
+  };
+  if (p0 < p1) fetch(p0);
+  for (int64_t p = p0; p < p1; ++p) {
+    if (p > p0) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < TT / 256; ++q) {
+      const int t = threadIdx.x + 256 * q, r = t & 63, c = t >> 6;
+      sA[r][c] = va[q];
+      if (transB) sB[r][c] = vb[q];
+      else sB[c][r] = vb[q];
+    }
+    if (p + 1 < p1) fetch(p + 1);
     __syncthreads();
+    mf_lds(sA, sB, m, threadIdx.x >> 6);
   }
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int r0 = 32 * (w >> 1), c0 = 32 * (w & 1), li = lane & 15, lq = lane >> 4;
-  if (g == 1)
-    for (int bi = 0; bi < 2; ++bi)
-      for (int bj = 0; bj < 2; ++bj)
-        for (int r = 0; r < 4; ++r) sA[1][r0 + 16 * bi + lq + 4 * r][c0 + 16 * bj + li] = m.d[bi][bj][r];
   __syncthreads();
-  if (g == 0)
-    for (int bi = 0; bi < 2; ++bi)
-      for (int bj = 0; bj < 2; ++bj)
-        for (int r = 0; r < 4; ++r) {
-          double &o = sA[0][r0 + 16 * bi + lq + 4 * r][c0 + 16 * bj + li];
-          o = m.d[bi][bj][r] + sA[1][r0 + 16 * bi + lq + 4 * r][c0 + 16 * bj + li];
-        }
+  for (int bi = 0; bi < 2; ++bi)
+    for (int bj = 0; bj < 2; ++bj)
+      for (int r = 0; r < 4; ++r) sA[r0 + 16 * bi + lq + 4 * r][c0 + 16 * bj + li] = m.d[bi][bj][r];
   __syncthreads();
 }
 
 // C_IJ -= sum_pairs L_IK L_JK'  (one workgroup per chunk of at most UCH pairs
-// of a target tile; chunks of one tile subtract atomically).  c1 coarse
-// factorisation with 8 / 4 / 2 pairs per chunk: 3.09 / 2.98 / 3.11 ms
-constexpr int UCH = 4;
+// of a target tile; chunks of one tile subtract atomically).  Factorisation of
+// 34 / 275 / 1,844 tile columns with 3, 4, 6 and 8 pairs per chunk: 635 / 2,370 /
+// 15,655, 635 / 2,350 / 15,690, 625 / 2,340 / 15,406 and 681 / 2,555 / 15,833 us.
+constexpr int UCH = 6;
 struct UpdArgs {
   const int32_t *tile;         // per chunk: target tile
   const int64_t *pbeg, *pend;  // per chunk: range of its pairs
   const int32_t *pairs;
   double *tiles;
 };
-using UpdLds = double[2][2][TS][TS + 1];
-__device__ inline void update_chunk(const UpdArgs &u, int ck, UpdLds &lds) {
+__device__ inline void update_chunk(const UpdArgs &u, int ck, PairLds &lds) {
   double *C = u.tiles + (int64_t)u.tile[ck] * TT;
-  pair_sum_2g(u.tiles, u.tiles, u.pairs, u.pbeg[ck], u.pend[ck], true, lds[0], lds[1]);
+  pair_sum(u.tiles, u.tiles, u.pairs, u.pbeg[ck], u.pend[ck], true, lds);
 #pragma unroll
-  for (int q = 0; q < TT / 512; ++q) {
-    const int t = threadIdx.x + 512 * q;
-    atomicAdd(C + t, -lds[0][0][t & 63][t >> 6]);
+  for (int q = 0; q < TT / 256; ++q) {
+    const int t = threadIdx.x + 256 * q;
+    atomicAdd(C + t, -lds.A[t & 63][t >> 6]);
   }
 }
-__global__ __launch_bounds__(512) void k_update(UpdArgs u, int chunk0) {
-  __shared__ UpdLds lds;
+__global__ __launch_bounds__(256) void k_update(UpdArgs u, int chunk0) {
+  __shared__ PairLds lds;
   update_chunk(u, chunk0 + blockIdx.x, lds);
 }
 
@@ -440,9 +440,11 @@ constexpr int PB = 8, PW = 4;  // panel width, waves per tile
 
 struct PotrfLds {
   double S[TS][TS + 2];   // L, row-major, rows 16-byte aligned
-  double P[PW][TS][PB];   // each wave's copy of the factored panel, row c = L[c][kb..kb+7]
+  union {                 // P is done with before X is begun
+    double P[PW][TS][PB];   // each wave's copy of the factored panel, row c = L[c][kb..kb+7]
+    double X[TS][TS + 1];   // inv(L), row-major
+  };
   double RD[PW][TS];      // each wave's copy of 1 / L[c][c]
-  double X[TS][TS + 1];   // inv(L), row-major
   double Tf[1024];        // B X_AA of the doubling steps
 };
 __device__ inline void potrf_tile(int J, double *A, const int32_t *pos2dof, double *dinv, double *dinvT, int *err,
@@ -601,22 +603,19 @@ __device__ inline void potrf_tile(int J, double *A, const int32_t *pos2dof, doub
 // wait for this level: the chunks of columns from the levels before it.  A level
 // is a chain update, potrf, trsm of 25, 19 and 8 us (275 tile columns in 43
 // levels) and the diagonal tiles leave nearly all CUs idle; now the chain holds
-// only the update by the level just finished.  Factorisation of 275 tile columns
-// 2.74 -> 2.40 ms, of 1,844 (99 levels, bound by the products) 18.59 -> 18.16,
-// of 34 columns 0.64 -> 0.63.
-__global__ __launch_bounds__(512) void k_potrf_update(const int32_t *cols, int ncol, const int32_t *diagtile,
+// only the update by the level just finished.  With the updates as they were then,
+// factorisation of 275 tile columns 2.74 -> 2.40 ms, of 1,844 (99 levels, bound by
+// the products) 18.59 -> 18.16, of 34 columns 0.64 -> 0.63.
+__global__ __launch_bounds__(64 * PW) void k_potrf_update(const int32_t *cols, int ncol, const int32_t *diagtile,
                                                       const int32_t *pos2dof, double *dinv, double *dinvT, int *err,
                                                       UpdArgs u, int chunk0) {
   __shared__ union Lds {
-    UpdLds upd;
+    PairLds upd;
     PotrfLds potrf;
     __device__ Lds() {}
   } lds;
   const int b = blockIdx.x;
   if (b < ncol) {
-    // the tile is the work of PW waves; the others end here, and the barriers
-    // wait for the waves that are left
-    if (threadIdx.x >= 64 * PW) return;
     const int J = cols[b];
     potrf_tile(J, u.tiles + (int64_t)diagtile[J] * TT, pos2dof, dinv, dinvT, err, lds.potrf);
   } else {
@@ -673,24 +672,24 @@ __global__ __launch_bounds__(256) void k_inv(const int32_t *inv_x, const int32_t
 // out = sign * sum_p A_p P_p, A_p from Abase (the L tiles for T = B X_AA, the
 // pool for X_CA = -X_CC T), P_p from the pool.  neg: the X step, which also
 // writes the transposed copy and the FP32 copies.  No pairs: the tile is zero.
-__global__ __launch_bounds__(512) void k_invp(const int32_t *out, const int64_t *pair_ptr, const int32_t *pairs,
+__global__ __launch_bounds__(256) void k_invp(const int32_t *out, const int64_t *pair_ptr, const int32_t *pairs,
                                               int task0, const double *Abase, double *X, double *XT, float *X32,
                                               float *XT32, int neg) {
   const int task = task0 + blockIdx.x;
-  __shared__ double sA[2][TS][TS + 1];
-  __shared__ double sB[2][TS][TS + 1];
-  pair_sum_2g(Abase, X, pairs, pair_ptr[task], pair_ptr[task + 1], false, sA, sB);
+  __shared__ PairLds lds;
+  auto &sA = lds.A;
+  pair_sum(Abase, X, pairs, pair_ptr[task], pair_ptr[task + 1], false, lds);
   double *O = X + (int64_t)out[task] * TT;
   double *OT = XT + (int64_t)out[task] * TT;
   const double sg = neg ? -1.0 : 1.0;
   const int64_t o = (int64_t)out[task] * TT;
 #pragma unroll
-  for (int q = 0; q < TT / 512; ++q) {
-    const int t = threadIdx.x + 512 * q, r = t & 63, c = t >> 6;
-    const double v = sg * sA[0][r][c];
+  for (int q = 0; q < TT / 256; ++q) {
+    const int t = threadIdx.x + 256 * q, r = t & 63, c = t >> 6;
+    const double v = sg * sA[r][c];
     O[t] = v;
     if (neg) {
-      const double vt = sg * sA[0][c][r];  // OT[r + 64c] = O[c + 64r]
+      const double vt = sg * sA[c][r];  // OT[r + 64c] = O[c + 64r]
       OT[t] = vt;
       X32[o + t] = (float)v;
       XT32[o + t] = (float)vt;
@@ -699,20 +698,20 @@ __global__ __launch_bounds__(512) void k_invp(const int32_t *out, const int64_t 
 }
 
 // Z_Ij = sum_k L_Ik X_kj over the block's columns k >= j, and its transposed copy
-__global__ __launch_bounds__(512) void k_zprod(const int32_t *z_tile, const int64_t *pair_ptr,
+__global__ __launch_bounds__(256) void k_zprod(const int32_t *z_tile, const int64_t *pair_ptr,
                                                const int32_t *pairs, const double *tiles, double *X,
                                                double *XT, float *X32, float *XT32) {
   const int task = blockIdx.x;
-  __shared__ double sA[2][TS][TS + 1];
-  __shared__ double sB[2][TS][TS + 1];
-  pair_sum_2g(tiles, X, pairs, pair_ptr[task], pair_ptr[task + 1], false, sA, sB);
+  __shared__ PairLds lds;
+  auto &sA = lds.A;
+  pair_sum(tiles, X, pairs, pair_ptr[task], pair_ptr[task + 1], false, lds);
   double *Zo = X + (int64_t)z_tile[task] * TT;
   double *ZTo = XT + (int64_t)z_tile[task] * TT;
   const int64_t o = (int64_t)z_tile[task] * TT;
 #pragma unroll
-  for (int q = 0; q < TT / 512; ++q) {
-    const int t = threadIdx.x + 512 * q, r = t & 63, c = t >> 6;
-    const double v = sA[0][r][c], vt = sA[0][c][r];
+  for (int q = 0; q < TT / 256; ++q) {
+    const int t = threadIdx.x + 256 * q, r = t & 63, c = t >> 6;
+    const double v = sA[r][c], vt = sA[c][r];
     Zo[t] = v;
     ZTo[t] = vt;
     X32[o + t] = (float)v;
@@ -1213,10 +1212,10 @@ void chol_factor(m3_ctx *c) {
   const UpdArgs upd{ch.upd_tile.p, ch.upd_pair_ptr.p, ch.upd_pair_end.p, ch.upd_pairs.p, ch.tiles.p};
   for (int l = 0; l < ch.nlev; ++l) {
     const int u0 = ch.h_upd_ptr[2 * l + 1], u1 = ch.h_upd_ptr[2 * l + 2];
-    if (u1 > u0) hipLaunchKernelGGL(k_update, dim3(u1 - u0), dim3(512), 0, s, upd, u0);
+    if (u1 > u0) hipLaunchKernelGGL(k_update, dim3(u1 - u0), dim3(256), 0, s, upd, u0);
     const int c0 = ch.h_lev_ptr[l], nc = ch.h_lev_ptr[l + 1] - c0;
     const int e1 = l + 1 < ch.nlev ? ch.h_upd_ptr[2 * l + 3] : u1;
-    hipLaunchKernelGGL(k_potrf_update, dim3(nc + (e1 - u1)), dim3(512), 0, s, ch.lev_cols.p + c0, nc, ch.diagtile.p,
+    hipLaunchKernelGGL(k_potrf_update, dim3(nc + (e1 - u1)), dim3(64 * PW), 0, s, ch.lev_cols.p + c0, nc, ch.diagtile.p,
                        ch.pos2dof.p, ch.dinv.p, ch.dinvT.p, c->errflag.p, upd, u1);
     const int t0 = ch.h_trsm_ptr[l], t1 = ch.h_trsm_ptr[l + 1];
     if (t1 > t0)
@@ -1229,11 +1228,11 @@ void chol_factor(m3_ctx *c) {
     const int a = ch.h_invp_ptr[st], b = ch.h_invp_ptr[st + 1];
     const bool xstep = (st & 1) != 0;
     if (b > a)
-      hipLaunchKernelGGL(k_invp, dim3(b - a), dim3(512), 0, s, ch.invp_out.p, ch.invp_pair_ptr.p, ch.invp_pairs.p, a,
+      hipLaunchKernelGGL(k_invp, dim3(b - a), dim3(256), 0, s, ch.invp_out.p, ch.invp_pair_ptr.p, ch.invp_pairs.p, a,
                          xstep ? ch.X.p : ch.tiles.p, ch.X.p, ch.XT.p, ch.X32.p, ch.XT32.p, xstep ? 1 : 0);
   }
   if (ch.nZ > 0)
-    hipLaunchKernelGGL(k_zprod, dim3((unsigned)ch.nZ), dim3(512), 0, s, ch.z_tile.p, ch.z_pair_ptr.p,
+    hipLaunchKernelGGL(k_zprod, dim3((unsigned)ch.nZ), dim3(256), 0, s, ch.z_tile.p, ch.z_pair_ptr.p,
                        ch.z_pairs.p, ch.tiles.p, ch.X.p, ch.XT.p, ch.X32.p, ch.XT32.p);
   HIPCHECK(hipGetLastError());
   c->factored = true;
