@@ -65,9 +65,10 @@ WINDOW_ROWS = 131072  # levels of this many nodes or more are swept in windows (
 # HBM bytes per launch of the dominant kernel, measured with two rocprofv3
 # counter passes (FETCH_SIZE x 2.0000 + WRITE_SIZE x 1.0000, factors from the
 # 1 GiB copy kernel of m3_copy_rate profiled in the same runs); recorded in
-# profiles/c1_k_smooth_hbm_traffic.md.  Keyed by (config, kernel); other
+# profiles/c1_sweep_hbm_traffic.md.  Keyed by (config, kernel); other
 # configs and kernels report null.
 MEASURED_TRAFFIC = {
+    ("c1", "k_sweep_win<B16P,float,6>"): 246303000,
 }
 
 

@@ -101,8 +101,8 @@ typedef struct {
 /* Precision of the multigrid V-cycle (the outer CG, dot products, Patera
  * update and coarse Cholesky are FP64 in every mode).  M3_PREC_MIXED: FP32
  * vectors and accumulation, BF16 matrix values on the finest and middle
- * levels (the finest keeps v8 of each 3x3 block in FP32), coarse triangular
- * solves on FP32 copies of the factor's inverse tiles. */
+ * levels (v8 of each 3x3 block in FP32), coarse triangular solves on FP32
+ * copies of the factor's inverse tiles. */
 enum { M3_PREC_FP64 = 0, M3_PREC_MIXED = 1 };
 
 /* Solver parameters: flow3d_patera_mg_sph_p.m:70-98, mgpcg_solver_p.m:674-682. */
