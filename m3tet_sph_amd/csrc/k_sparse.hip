@@ -25,6 +25,9 @@
 
 #include <hip/hip_bf16.h>
 
+#include <cstdint>
+#include <cstring>
+
 namespace {
 
 // BF16 values in packed groups (kval's counterpart p16_words / p16_v8): eight
@@ -1361,9 +1364,29 @@ double patera_step(m3_ctx *c, int64_t n, int64_t n3, double *U, const double *z,
   return std::sqrt(host_sum(c, ng));
 }
 
+// The smallest rr >= 0 that does not meet sqrt(rr / nfree) < tol, so that the
+// kernels' comparison rr < rr_stop is that test for every rr, also where tol^2
+// underflows; 0 (never met) for a tol <= 0 or NaN.  The test is monotone in rr,
+// and non-negative doubles are ordered as their bits.
+static double pcg_stop(double tol, double nfree) {
+  const auto met = [&](uint64_t bits) {
+    double rr;
+    std::memcpy(&rr, &bits, sizeof rr);
+    return std::sqrt(rr / nfree) < tol;
+  };
+  uint64_t lo = 0, hi = 0x7ff0000000000000ull;  // +0 and +inf, which never meets it
+  while (lo < hi) {
+    const uint64_t mid = lo + (hi - lo) / 2;
+    if (met(mid)) lo = mid + 1;
+    else hi = mid;
+  }
+  double rr;
+  std::memcpy(&rr, &lo, sizeof rr);
+  return rr;
+}
+
 // pcg_solver_p.m:49-186 with the 'diag' preconditioner (Polak-Ribiere beta,
-// alpha = r.d / q.Aq), k_pcg_dir and k_pcg_update.  The norms are compared as
-// squares: |r| / sqrt(nfree) < tol.
+// alpha = r.d / q.Aq), k_pcg_dir and k_pcg_update; the norm is |r| / sqrt(nfree)
 int pcg_diag_run(m3_ctx *c, SellView A, int64_t n, const double *Adi, double *x, double *r, double *q0, double *q1,
                  double *Aq, double nfree, double tol, int itmax, double *norm) {
   hipStream_t s = c->stream;
@@ -1371,7 +1394,7 @@ int pcg_diag_run(m3_ctx *c, SellView A, int64_t n, const double *Adi, double *x,
   const int nu = (int)std::min<int64_t>(256, (n + PC_T - 1) / PC_T), nq = (int)((n + 63) / 64);
   double *up = c->partial.p, *qp = c->partial.p + 3 * nu;
   M3_REQUIRE((size_t)(3 * nu + nq) <= c->partial.n, M3_E_STATE, "partial sums do not fit");
-  const double rr_stop = tol > 0 ? tol * tol * nfree : -1.0;  // -1: never met
+  const double rr_stop = pcg_stop(tol, nfree);
   hipLaunchKernelGGL(k_zero64, dim3(1), dim3(256), 0, s, (int64_t)6, state);
   hipLaunchKernelGGL(k_zero64, dim3(nblk(n)), dim3(256), 0, s, n, q0);
   hipLaunchKernelGGL(k_pcg_start, dim3(nu), dim3(PC_T), 0, s, n, r, Adi, up, nu);

@@ -194,3 +194,20 @@ def test_iteration_limits_match_the_oracle(c0, ctx0, itmax):
     assert info["nit"] == io["nit"]
     assert relerr(info["norm_r"], io["hist"][-1]) < 1e-6
     assert relerr(T, To) < 1e-10
+
+
+def test_tolerance_whose_square_underflows(c0, ctx0):
+    """An absolute tolerance of 1e-170 is met by the residual that underflows to
+    zero (the oracle after 25 iterations), as any tolerance is met by zero."""
+    from oracle import diffusion as D
+    n = c0.nVnod
+    T0 = np.random.default_rng(9).random(n)
+    ifix, _ = _fixed(c0, n)
+    o = dict(tol=1e-170, is_abs_tol=True, itmax=200)
+    T, info = ctx0.diffusion3d(T0, 1.0, 1e-12, ifix, T0[ifix], **o)
+    To, io = D.diffusion3d_p(T0, 1.0, c0.GCOORD, c0.GCOORD_SPH, c0.levels[0].EL2NOD[:, :4], ifix, T0[ifix], 1e-12, **o)
+    log("underflow", info, io["nit"])
+    assert io["hist"][-1] == 0.0 and info["norm_r"] == 0.0
+    # sums in another order, each iteration 1e-6 of the one before: a few more or fewer
+    assert abs(info["nit"] - io["nit"]) <= 5
+    assert relerr(T, To) < 1e-10
