@@ -826,8 +826,11 @@ __global__ __launch_bounds__(RB) void k_pp_update(int64_t n, int64_t n3, double 
 // tolerance, so the host can queue several iterations and read the state after
 // them; the iterates are those of a loop that looks every time.  Seven launches
 // and a blocking read per iteration took 55 us at 43,554 rows, this 20.
-// state: 0 r.d of the current direction, 1 |r|^2, 2 iterations done,
-// 3 stopped (1 converged, 2 NaN)
+// state: 0 r.d of the current direction, 1 |r|^2, 2 iterations done, 3 stopped
+// (1 converged, 2 NaN) as the direction's launches read it, 4 + parity: r.d by
+// iteration, 6 stopped as a direction's launch finds it.  No launch of several
+// workgroups reads a value that it writes: k_pcg_dir reads 3 and writes 6, the
+// update after it reads 6 and writes 3.
 constexpr int PC_T = RB;
 __device__ inline void pc_part(double s, double *part, double *sh) {
   s = rb_block(s, sh);
@@ -888,7 +891,7 @@ __global__ __launch_bounds__(64 * SP_W) void k_pcg_dir(SellView A, int64_t n, co
   if (blockIdx.x == 0 && t == 0) {
     state[1] = s[0];
     if (stop) {
-      state[3] = s[0] < rr_stop ? 1.0 : 2.0;
+      state[6] = s[0] < rr_stop ? 1.0 : 2.0;
     } else {
       state[0] = s[2];
       state[4 + ((it + 1) & 1)] = s[2];
@@ -913,7 +916,10 @@ __global__ __launch_bounds__(PC_T) void k_pcg_update(int64_t n, const double *q,
                                                      const double *qp, int nq, double *x, double *r, double *up,
                                                      int nu, double *state, int it) {
   __shared__ double sh[4];
-  if (state[3] != 0.0) return;
+  if (state[6] != 0.0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) state[3] = state[6];
+    return;
+  }
   const double alpha = state[0] / rb_total(qp, nq, sh);
   if (blockIdx.x == 0 && threadIdx.x == 0) state[2] = it;
   double rr = 0, s0 = 0, s1 = 0;
@@ -932,7 +938,7 @@ __global__ __launch_bounds__(PC_T) void k_pcg_update(int64_t n, const double *q,
 // |r|^2 after the last queued iteration
 __global__ __launch_bounds__(PC_T) void k_pcg_look(const double *up, int nu, double *state, double rr_stop) {
   __shared__ double sh[4];
-  if (state[3] != 0.0) return;
+  if (state[3] != 0.0) return;  // one workgroup, and it writes behind rb_total's barriers
   const double rr = rb_total(up, nu, sh);
   if (threadIdx.x == 0) {
     state[1] = rr;
@@ -1390,12 +1396,12 @@ static double pcg_stop(double tol, double nfree) {
 int pcg_diag_run(m3_ctx *c, SellView A, int64_t n, const double *Adi, double *x, double *r, double *q0, double *q1,
                  double *Aq, double nfree, double tol, int itmax, double *norm) {
   hipStream_t s = c->stream;
-  double *state = c->scal.p + 16;  // 6 values
+  double *state = c->scal.p + 16;  // 7 values
   const int nu = (int)std::min<int64_t>(256, (n + PC_T - 1) / PC_T), nq = (int)((n + 63) / 64);
   double *up = c->partial.p, *qp = c->partial.p + 3 * nu;
   M3_REQUIRE((size_t)(3 * nu + nq) <= c->partial.n, M3_E_STATE, "partial sums do not fit");
   const double rr_stop = pcg_stop(tol, nfree);
-  hipLaunchKernelGGL(k_zero64, dim3(1), dim3(256), 0, s, (int64_t)6, state);
+  hipLaunchKernelGGL(k_zero64, dim3(1), dim3(256), 0, s, (int64_t)7, state);
   hipLaunchKernelGGL(k_zero64, dim3(nblk(n)), dim3(256), 0, s, n, q0);
   hipLaunchKernelGGL(k_pcg_start, dim3(nu), dim3(PC_T), 0, s, n, r, Adi, up, nu);
   // iterations queued before the host looks: a few launches that end at once
