@@ -1214,6 +1214,7 @@ int m3_get_vector(m3_ctx *c, int32_t which, int32_t level, double *out) {
       case 0: c->Fb.download(out, 3 * c->nnod); break;
       case 1: c->bc_rhs.download(out, 3 * c->nnod); break;
       case 2: {
+        M3_REQUIRE(lv.dinv.n == (size_t)(3 * lv.nnod), M3_E_STATE, "m3_set_mesh has not been completed");
         const std::vector<double> di = lv.dinv.to_host();
         for (int64_t q = 0; q < lv.nnod; ++q) {
           const int64_t r = lv.K.h_vperm.empty() ? q : (int64_t)lv.K.h_vperm[q];

@@ -57,3 +57,21 @@ def test_level_operators(shape):
         assert relerr(x16, x64) < 1e-4 and abs(n64 - n16) <= 3
     finally:
         ctx.close()
+
+
+def test_vectors_of_an_unfinished_mesh(tiny):
+    """A mesh that is refused at its second level leaves the first one without
+    its vectors: reading the diagonal of K raises."""
+    import copy
+    from m3tet_sph_amd import api
+    ctx = api.StokesContext(tiny)
+    try:
+        bad = copy.copy(tiny)
+        bad.levels = [copy.copy(L) for L in tiny.levels]
+        bad.levels[1].EL2NOD = tiny.levels[1].EL2NOD + tiny.levels[1].nnod
+        with pytest.raises(api.M3Error, match="EL2NOD entry out of range"):
+            ctx._set_mesh(bad)
+        with pytest.raises(api.M3Error):
+            ctx.get_vector(2, 0)
+    finally:
+        ctx.close()
