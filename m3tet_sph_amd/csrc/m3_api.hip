@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <map>
+#include <memory>
 #include <numeric>
 #include <unordered_map>
 
@@ -61,58 +62,117 @@ void Sell::build(int64_t nrow_, int64_t ncol_, const std::vector<int64_t> &ptr,
   val.alloc((size_t)nslot * bs);
 }
 
+namespace {
+
+// Host array whose pages the threads that fill it touch first (a vector clears
+// them one after the other: half the time of a large one's whole use)
+template <class T>
+struct HostArr {
+  std::unique_ptr<T[]> p;
+  size_t n;
+  explicit HostArr(size_t count) : p(new T[count]), n(count) {}
+  T &operator[](size_t i) { return p[i]; }
+};
+
+// The different vector places that a window of rows gathers: an open-addressed
+// table of SIZE entries (at most half of them taken), so that a thread needs
+// 128 KB whatever the mesh, and a look-up stays in its L2.
+struct WindowTable {
+  static constexpr int SIZE = 16384, FULL = SIZE / 2;
+  std::vector<int32_t> key = std::vector<int32_t>(SIZE, -1), rank = std::vector<int32_t>(SIZE);
+  std::vector<int32_t> list;  // the places, in the order of their first look-up
+  WindowTable() { list.reserve(FULL + 1); }
+  void clear() {
+    std::fill(key.begin(), key.end(), -1);
+    list.clear();
+  }
+  // entry of place i, added if it is new; no more than FULL places
+  int at(int32_t i) {
+    uint32_t h = ((uint32_t)i * 2654435761u) >> 18;
+    while (key[h] != i) {
+      if (key[h] < 0) {
+        key[h] = i;
+        list.push_back(i);
+        break;
+      }
+      h = (h + 1) & (SIZE - 1);
+    }
+    return (int)h;
+  }
+  // list ascending, rank of every entry in it
+  void number() {
+    std::sort(list.begin(), list.end());
+    for (size_t r = 0; r < list.size(); ++r) rank[at(list[r])] = (int32_t)r;
+  }
+};
+
+}  // namespace
+
 bool Sell::build_windows(const std::vector<int32_t> &order, int w, int cap) {
   const int64_t nw = (nrow + w - 1) / w;
   std::vector<std::vector<int32_t>> lists(nw);
-  std::vector<uint16_t> h_idx((size_t)nslot, 0);
-  std::vector<int32_t> h_plen(nrow), pos(nrow);
-  std::vector<uint16_t> h_lrow(nrow);
+  HostArr<uint16_t> h_idx((size_t)nslot), h_lrow(nrow);
+  HostArr<int32_t> h_plen(nrow);
+  std::vector<int32_t> pos(nrow);
+#pragma omp parallel for schedule(static)
   for (int64_t i = 0; i < nrow; ++i) pos[order[i]] = (int32_t)i;
-  bool fits = true;
-#pragma omp parallel reduction(&& : fits)
-  {
-    std::vector<int32_t> seen(ncol, -1), at(ncol);  // last window that holds an entry, its place there
-#pragma omp for schedule(dynamic, 4)
-    for (int64_t b = 0; b < nw; ++b) {
-      std::vector<int32_t> &L = lists[b];
-      const int64_t q0 = b * w, q1 = std::min(nrow, q0 + w);
-      auto each = [&](auto fn) {
-        for (int64_t q = q0; q < q1; ++q) {
-          const int len = h_rowlen[h_perm[q]];
-          const int64_t base = h_slice_ptr[q >> 6] + (q & 63);
-          h_plen[q] = len;
-          h_lrow[q] = (uint16_t)(pos[h_perm[q]] - q0);
-          for (int k = 0; k < len; ++k) fn(base + 64 * (int64_t)k, pos[h_col[base + 64 * (int64_t)k]]);
-        }
-      };
-      each([&](int64_t, int32_t i) {
-        if (seen[i] != (int32_t)b) {
-          seen[i] = (int32_t)b;
-          L.push_back(i);
-        }
-      });
-      std::sort(L.begin(), L.end());
-      for (size_t i = 0; i < L.size(); ++i) at[L[i]] = (int32_t)i;
-      if ((int64_t)L.size() > cap) fits = false;
-      else each([&](int64_t slot, int32_t i) { h_idx[slot] = (uint16_t)at[i]; });
+  cap = std::min(cap, WindowTable::FULL);
+  bool fits = true, memory = true;  // an exception must not leave a parallel region
+  std::vector<WindowTable> tables(omp_get_max_threads());
+#pragma omp parallel for schedule(dynamic, 4) reduction(&& : fits, memory)
+  for (int64_t b = 0; b < nw; ++b) {
+    WindowTable &t = tables[omp_get_thread_num()];
+    t.clear();
+    const int64_t q0 = b * w, q1 = std::min(nrow, q0 + w);
+    // padding slots are never read; they hold the window's first place
+    std::fill(&h_idx[h_slice_ptr[q0 >> 6]], &h_idx[0] + h_slice_ptr[(q1 + 63) >> 6], (uint16_t)0);
+    bool ok = true;
+    for (int64_t q = q0; q < q1 && ok; ++q) {
+      const int len = h_rowlen[h_perm[q]];
+      const int64_t base = h_slice_ptr[q >> 6] + (q & 63);
+      h_plen[q] = len;
+      h_lrow[q] = (uint16_t)(pos[h_perm[q]] - q0);
+      for (int k = 0; k < len && ok; ++k) {
+        h_idx[base + 64 * (int64_t)k] = (uint16_t)t.at(pos[h_col[base + 64 * (int64_t)k]]);
+        ok = (int)t.list.size() <= cap;
+      }
+    }
+    if (!ok) {
+      fits = false;
+      continue;
+    }
+    t.number();
+    for (int64_t q = q0; q < q1; ++q) {
+      const int64_t base = h_slice_ptr[q >> 6] + (q & 63);
+      for (int k = 0; k < h_plen[q]; ++k) {
+        uint16_t &e = h_idx[base + 64 * (int64_t)k];
+        e = (uint16_t)t.rank[e];
+      }
+    }
+    try {
+      lists[b] = t.list;
+    } catch (const std::bad_alloc &) {
+      memory = false;
     }
   }
+  if (!memory) throw std::bad_alloc();
   if (!fits) return false;
-  std::vector<int32_t> h_lptr(nw + 1, 0), h_list;
+  std::vector<int32_t> h_lptr(nw + 1, 0);
   umax = 0;
   for (int64_t b = 0; b < nw; ++b) {
     umax = std::max(umax, (int)lists[b].size());
     h_lptr[b + 1] = h_lptr[b] + (int32_t)lists[b].size();
   }
-  h_list.reserve(h_lptr[nw]);
-  for (const auto &L : lists) h_list.insert(h_list.end(), L.begin(), L.end());
+  HostArr<int32_t> h_list(h_lptr[nw]);
+#pragma omp parallel for schedule(static)
+  for (int64_t b = 0; b < nw; ++b) std::copy(lists[b].begin(), lists[b].end(), &h_list[h_lptr[b]]);
   win = w;
   nwin = (int)nw;
-  plen.upload(h_plen);
+  plen.upload(h_plen.p.get(), h_plen.n);
   lptr.upload(h_lptr);
-  list.upload(h_list);
-  idx.upload(h_idx);
-  lrow.upload(h_lrow);
+  list.upload(h_list.p.get(), h_list.n);
+  idx.upload(h_idx.p.get(), h_idx.n);
+  lrow.upload(h_lrow.p.get(), h_lrow.n);
   h_vperm = order;
   h_vpos.swap(pos);
   vperm.upload(h_vperm);
@@ -388,6 +448,7 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
       if (w) {
         M3_REQUIRE(m->GCOORD, M3_E_ARG, "missing GCOORD");
         const std::vector<int32_t> order = hilbert_order(m->GCOORD, lv.nnod), place = window_placement(order, w, ptr);
+        mark("space-filling order");
         lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9, &place);
         mark("level connectivity + K pattern");
         if (!lv.K.build_windows(order, w, m3::SWEEP_CAP)) lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
@@ -519,11 +580,10 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
       LevelDev &fl = c->L[l];
       LevelDev &cl = c->L[l + 1];
       M3_REQUIRE(m->Ic2f_ptr[l] && m->Ic2f_col[l] && m->Ic2f_val[l], M3_E_ARG, "missing Ic2f");
-      const int64_t *pp = m->Ic2f_ptr[l];
-      std::vector<int64_t> P_ptr(pp, pp + fl.nnod + 1);
+      const int64_t *P_ptr = m->Ic2f_ptr[l];
       const int64_t nnzP = P_ptr[fl.nnod];
-      std::vector<int32_t> P_col(m->Ic2f_col[l], m->Ic2f_col[l] + nnzP);
-      std::vector<double> P_val(m->Ic2f_val[l], m->Ic2f_val[l] + nnzP);
+      const int32_t *P_col = m->Ic2f_col[l];
+      const double *P_val = m->Ic2f_val[l];
       for (int64_t k = 0; k < nnzP; ++k)
         M3_REQUIRE(P_col[k] >= 0 && P_col[k] < cl.nnod, M3_E_MESH, "Ic2f column out of range");
       // both directions in the levels' vector orders: row q of P is the node at
@@ -531,30 +591,47 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
       const std::vector<int32_t> &fperm = fl.K.h_vperm, &cipos = cl.K.h_vpos;
       auto fnode = [&](int64_t q) { return fperm.empty() ? q : (int64_t)fperm[q]; };
       std::vector<int64_t> PP(fl.nnod + 1, 0), R_ptr(cl.nnod + 1, 0);
-      for (int64_t q = 0; q < fl.nnod; ++q) PP[q + 1] = PP[q] + P_ptr[fnode(q) + 1] - P_ptr[fnode(q)];
-      std::vector<int32_t> PC(nnzP), R_col(nnzP);
-      std::vector<double> PV(nnzP), R_val(nnzP);
+#pragma omp parallel for schedule(static)
+      for (int64_t q = 0; q < fl.nnod; ++q) PP[q + 1] = P_ptr[fnode(q) + 1] - P_ptr[fnode(q)];
+      for (int64_t q = 0; q < fl.nnod; ++q) PP[q + 1] += PP[q];
+      HostArr<int32_t> PC(nnzP), R_col(nnzP);
+      HostArr<double> PV(nnzP), R_val(nnzP);
 #pragma omp parallel for schedule(static)
       for (int64_t q = 0; q < fl.nnod; ++q)
         for (int64_t k = P_ptr[fnode(q)], o = PP[q]; k < P_ptr[fnode(q) + 1]; ++k, ++o) {
           PC[o] = cipos.empty() ? P_col[k] : cipos[P_col[k]];
           PV[o] = P_val[k];
         }
-      for (int64_t k = 0; k < nnzP; ++k) R_ptr[PC[k] + 1]++;
+      // the transpose: every thread reads all of P and keeps the entries of its
+      // own range of coarse rows (fine rows ascending in each)
+      const int nt = omp_get_max_threads();
+      auto first = [&](int t) { return (int32_t)(cl.nnod * t / nt); };
+#pragma omp parallel for schedule(static, 1)
+      for (int t = 0; t < nt; ++t) {
+        const int32_t j0 = first(t), j1 = first(t + 1);
+        for (int64_t k = 0; k < nnzP; ++k)
+          if (PC[k] >= j0 && PC[k] < j1) R_ptr[PC[k] + 1]++;
+      }
       for (int64_t j = 0; j < cl.nnod; ++j) R_ptr[j + 1] += R_ptr[j];
       std::vector<int64_t> fill(R_ptr.begin(), R_ptr.end() - 1);
-      for (int64_t i = 0; i < fl.nnod; ++i)
-        for (int64_t k = PP[i]; k < PP[i + 1]; ++k) {
-          const int64_t q = fill[PC[k]]++;
-          R_col[q] = (int32_t)i;
-          R_val[q] = PV[k];
-        }
+#pragma omp parallel for schedule(static, 1)
+      for (int t = 0; t < nt; ++t) {
+        const int32_t j0 = first(t), j1 = first(t + 1);
+        for (int64_t i = 0; i < fl.nnod; ++i)
+          for (int64_t k = PP[i]; k < PP[i + 1]; ++k) {
+            if (PC[k] < j0 || PC[k] >= j1) continue;
+            const int64_t q = fill[PC[k]]++;
+            R_col[q] = (int32_t)i;
+            R_val[q] = PV[k];
+          }
+      }
+      mark("transfers");
       fl.P_ptr.upload(PP);
-      fl.P_col.upload(PC);
-      fl.P_val.upload(PV);
+      fl.P_col.upload(PC.p.get(), PC.n);
+      fl.P_val.upload(PV.p.get(), PV.n);
       fl.R_ptr.upload(R_ptr);
-      fl.R_col.upload(R_col);
-      fl.R_val.upload(R_val);
+      fl.R_col.upload(R_col.p.get(), R_col.n);
+      fl.R_val.upload(R_val.p.get(), R_val.n);
       // Q_e[i][a] = Ic2f(node_e(i), node_parent(a)); every nonzero of the
       // rows of a child must lie on its parent's nodes (nesting invariant).
       // Distinct tables are numbered in order of first appearance: a 64-bit
