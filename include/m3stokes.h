@@ -156,6 +156,12 @@ void m3_destroy(m3_ctx *ctx);
 const char *m3_last_error(const m3_ctx *ctx);
 
 int m3_set_mesh(m3_ctx *ctx, const m3_mesh_desc *mesh);
+/* Which multigrid levels the m3_set_mesh calls from now on sweep in windows: the
+ * fewest rows of such a level, and the most vector entries that a window of more
+ * than 64 rows / one of 64 rows gathers (at most 6300; larger windows are split,
+ * and a level whose 64 rows gather more has no windows).  0: the library's own
+ * choice.  It moves work, not results.  No reference counterpart. */
+int m3_sweep_windows(m3_ctx *ctx, int64_t rows, int32_t split, int32_t limit);
 /* ifix: 1-based rotated-frame dofs, vfix: values (UBC.ifix / UBC.vfix). */
 int m3_set_bc(m3_ctx *ctx, const int64_t *ifix, const double *vfix, int64_t nfix);
 
@@ -292,7 +298,9 @@ int m3_apply(m3_ctx *ctx, int32_t which, int32_t level, const double *x, double 
 int m3_get_vector(m3_ctx *ctx, int32_t which, int32_t level, double *out);
 
 /* Sizes: n[0]=levels, n[1..] per-level block nonzeros of K, then coarse factor
- * statistics (free dofs, tiles, stored tiles, levels). */
+ * statistics (free dofs, tiles, stored tiles, levels, solve levels), then per
+ * level the stored block slots of K, the windows of its sweeps (0: swept
+ * without) and the most vector entries that one of them gathers. */
 int m3_stats(m3_ctx *ctx, int64_t *out, int32_t nout);
 
 /* Residuals of (U, P) for the assembled problem, RMS norms (normdf.m:22):

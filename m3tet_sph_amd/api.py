@@ -105,6 +105,7 @@ LIB.m3_set_fields.argtypes = [C.c_void_p, D, D]
 LIB.m3_apply.argtypes = [C.c_void_p, C.c_int32, C.c_int32, D, D]
 LIB.m3_get_vector.argtypes = [C.c_void_p, C.c_int32, C.c_int32, D]
 LIB.m3_stats.argtypes = [C.c_void_p, I64, C.c_int32]
+LIB.m3_sweep_windows.argtypes = [C.c_void_p, C.c_int64, C.c_int32, C.c_int32]
 LIB.m3_sl_advect.argtypes = [C.c_void_p, D, D, C.c_double, C.c_double, C.c_double, D]
 
 
@@ -295,7 +296,7 @@ LIB.m3_calculate_dt.restype = C.c_int
 for _f in ("m3_create", "m3_set_mesh", "m3_set_bc", "m3_assemble", "m3_element_matrices",
            "m3_restrict_stiffmat", "m3_cholesky_factorization", "m3_cholesky_solve", "m3_mgpcg",
            "m3_patera", "m3_flow3d_patera_sph", "m3_flow3d_patera_sph_dstart", "m3_apply", "m3_get_vector",
-           "m3_stats", "m3_sl_advect", "m3_solution_device", "m3_get_solution", "m3_set_fields"):
+           "m3_stats", "m3_sweep_windows", "m3_sl_advect", "m3_solution_device", "m3_get_solution", "m3_set_fields"):
     getattr(LIB, _f).restype = C.c_int
 
 
@@ -399,7 +400,8 @@ def export_case(path, m, inputs):
 class StokesContext:
     """Device state of one mesh (patterns, operators, hierarchy, factor)."""
 
-    def __init__(self, mesh: meshmod.ShellMesh, device=0):
+    def __init__(self, mesh: meshmod.ShellMesh, device=0, sweep_windows=None):
+        """sweep_windows: (rows, split, limit) of m3_sweep_windows."""
         self._h = C.c_void_p()
         rc = LIB.m3_create(C.byref(self._h), device)
         if rc:
@@ -410,6 +412,8 @@ class StokesContext:
             raise M3Error(rc, msg)
         self.mesh = mesh
         self._keep = []
+        if sweep_windows is not None:
+            self._check(LIB.m3_sweep_windows(self._h, *sweep_windows))
         self._set_mesh(mesh)
 
     def close(self):
@@ -653,13 +657,15 @@ class StokesContext:
         return out
 
     def stats(self):
-        out = np.zeros(32, dtype=np.int64)
-        self._check(LIB.m3_stats(self._h, _p(out, I64), 32))
+        out = np.zeros(64, dtype=np.int64)
+        self._check(LIB.m3_stats(self._h, _p(out, I64), 64))
         nmg = int(out[0])
         return dict(nmg=nmg, nnzb=[int(v) for v in out[1:1 + nmg]],
                     chol_n=int(out[1 + nmg]), chol_T=int(out[2 + nmg]), chol_tiles=int(out[3 + nmg]),
                     chol_levels=int(out[4 + nmg]), chol_heights=int(out[5 + nmg]),
-                    nslot=[int(v) for v in out[6 + nmg:6 + 2 * nmg]])
+                    nslot=[int(v) for v in out[6 + nmg:6 + 2 * nmg]],
+                    windows=[int(v) for v in out[6 + 2 * nmg:6 + 3 * nmg]],
+                    window_entries=[int(v) for v in out[6 + 3 * nmg:6 + 4 * nmg]])
 
 
 # ---------------------------------------------------------------------------

@@ -211,6 +211,7 @@ __global__ __launch_bounds__(64 * W) void k_sweep(SweepPat K, const MT *__restri
 // values of 337,986 rows, which take 210 MB); streaming loads otherwise (FP64
 // there 149 us with cached loads).
 constexpr int SW_WIN = 512, SW_NW = 8, SW_W = 2, SW_TEAMS = SW_NW / SW_W;
+static_assert(24 * (m3::SWEEP_LIMIT + SW_WIN) + 8 * SW_NW <= 160 * 1024, "LDS of a window");
 template <class MT, class VT, int MODE, int UNR, bool RES>
 __global__ __launch_bounds__(64 * SW_NW, (std::is_same<MT, double>::value ? 4 : 8)) void k_sweep_win(
     SweepPat K, int nwin, int umax, const MT *__restrict__ val, SweepVec<VT> v) {
@@ -225,7 +226,8 @@ __global__ __launch_bounds__(64 * SW_NW, (std::is_same<MT, double>::value ? 4 : 
   }
   double dot = 0;
   if (b >= 0) {
-    const int l0 = K.lptr[b], nl = K.lptr[b + 1] - l0;
+    const int2 w0 = K.win[b], w1 = K.win[b + 1];
+    const int l0 = w0.y, nl = w1.y - l0, nr = w1.x - w0.x;
     for (int t = threadIdx.x; t < 3 * nl; t += 64 * SW_NW) {
       const int i = t / 3;
       xs[t] = v.x[3 * (int64_t)K.list[l0 + i] + (t - 3 * i)];
@@ -233,12 +235,12 @@ __global__ __launch_bounds__(64 * SW_NW, (std::is_same<MT, double>::value ? 4 : 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, w = wave % SW_W, team = wave / SW_W;
     __syncthreads();
 #pragma unroll 1
-    for (int rd = 0; rd < SW_WIN / (64 * SW_TEAMS); ++rd) {
-      const int64_t sl = (int64_t)b * (SW_WIN / 64) + rd * SW_TEAMS + team;
-      const int64_t q = sl * 64 + lane;
+    for (int rd = 0; 64 * SW_TEAMS * rd < nr; ++rd) {
+      const int sl = (w0.x >> 6) + rd * SW_TEAMS + team;
+      const int q = sl * 64 + lane;
       VT y0 = 0, y1 = 0, y2 = 0;
       VT *yr = ys;
-      if (q < K.n) {
+      if (q < w1.x) {
         const int64_t g0 = K.slice_ptr[sl] >> 6;
         const int len = K.len[q];
         yr += 3 * K.lrow[q];
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(64 * SW_NW, (std::is_same<MT, double>::value ? 4 : 
       // the slice's waves add their sums in turn (a row belongs to one lane of each)
 #pragma unroll
       for (int j = 0; j < SW_W; ++j) {
-        if (w == j && q < K.n) {
+        if (w == j && q < w1.x) {
           yr[0] = j == 0 ? y0 : yr[0] + y0;
           yr[1] = j == 0 ? y1 : yr[1] + y1;
           yr[2] = j == 0 ? y2 : yr[2] + y2;
@@ -273,8 +275,8 @@ __global__ __launch_bounds__(64 * SW_NW, (std::is_same<MT, double>::value ? 4 : 
         __syncthreads();
       }
     }
-    const int64_t o0 = 3 * (int64_t)b * SW_WIN;
-    for (int t = threadIdx.x; t < 3 * SW_WIN && o0 + t < 3 * K.n; t += 64 * SW_NW)
+    const int64_t o0 = 3 * (int64_t)w0.x;
+    for (int t = threadIdx.x; t < 3 * nr; t += 64 * SW_NW)
       sweep_out<VT, MODE>(v, sweep_in<VT, MODE>(v, o0 + t), o0 + t, ys[t], dot);
   }
   if (MODE & 8) {
@@ -985,7 +987,7 @@ thread_local hipEvent_t prof_start = nullptr, prof_stop = nullptr;
 // 42.9 us, 174,114 rows 27.1 / 74.5 against 30.3 / 89.7 us, 256,050 rows 33.9 /
 // 93.3 against 44.8 / 130 us).  Windows of 256 rows: 25.4 / 82.3 us on 174,114
 // rows, 34.1 / 102 us on 256,050.
-int sweep_window(int64_t n) { return n >= 131072 ? SW_WIN : 0; }
+int sweep_window(const SweepRule &r, int64_t n) { return n >= r.rows ? SW_WIN : 0; }
 
 // do the values stay in the last-level cache (256 MB) between sweeps?
 template <class MT>
@@ -995,7 +997,7 @@ static bool sweep_resident(const Sell &K) {
 // workgroups of a sweep, each with its partial sum (MODE bit 8)
 template <class MT>
 static int sweep_grid(const Sell &K) {
-  if (!K.win) return (int)((K.nrow + 63) / 64);
+  if (!K.nwin) return (int)((K.nrow + 63) / 64);
   return sweep_resident<MT>(K) ? (K.nwin + 7) / 8 * 8 : K.nwin;
 }
 
@@ -1003,7 +1005,7 @@ static int sweep_grid(const Sell &K) {
 template <class MT, class VT, int MODE>
 static void launch_sweep(hipStream_t s, const Sell &K, const MT *val, const SweepVec<VT> &v) {
   const SweepPat P = K.sweep();
-  if (K.win) {
+  if (K.nwin) {
     constexpr int UNR = std::is_same<MT, double>::value ? 2 : 3;
     const unsigned lds = (unsigned)(3 * ((size_t)K.umax + SW_WIN) * sizeof(VT));
     auto go = [&](auto kern) {
@@ -1115,7 +1117,7 @@ static void sweep(hipStream_t s, const LevelDev &lv, const VT *x, const VT *r0, 
 //          the mask, the gathered vector once and the vectors read / written.
 template <class MT>
 static double sweep_bytes(const LevelDev &lv, int nvec, size_t vt) {
-  return (double)lv.K.nnz * (block_value_bytes<MT>() + (lv.K.win ? 2.0 : 4.0)) + 4.0 * lv.nnod +
+  return (double)lv.K.nnz * (block_value_bytes<MT>() + (lv.K.nwin ? 2.0 : 4.0)) + 4.0 * lv.nnod +
          3.0 * lv.nnod * nvec * vt;
 }
 

@@ -33,7 +33,7 @@ void Sell::build(int64_t nrow_, int64_t ncol_, const std::vector<int64_t> &ptr,
   h_ipos.clear();
   h_vperm.clear();
   h_vpos.clear();
-  win = 0;
+  nwin = 0;
   if (place) {
     h_perm = *place;
     h_ipos.resize(nrow);
@@ -108,22 +108,23 @@ struct WindowTable {
 
 }  // namespace
 
-bool Sell::build_windows(const std::vector<int32_t> &order, int w, int cap) {
-  const int64_t nw = (nrow + w - 1) / w;
+bool Sell::build_windows(const std::vector<int32_t> &order, const std::vector<int32_t> &first,
+                         const m3::SweepRule &rule) {
+  const int64_t nw = (int64_t)first.size() - 1;
   std::vector<std::vector<int32_t>> lists(nw);
   HostArr<uint16_t> h_idx((size_t)nslot), h_lrow(nrow);
   HostArr<int32_t> h_plen(nrow);
   std::vector<int32_t> pos(nrow);
 #pragma omp parallel for schedule(static)
   for (int64_t i = 0; i < nrow; ++i) pos[order[i]] = (int32_t)i;
-  cap = std::min(cap, WindowTable::FULL);
   bool fits = true, memory = true;  // an exception must not leave a parallel region
   std::vector<WindowTable> tables(omp_get_max_threads());
 #pragma omp parallel for schedule(dynamic, 4) reduction(&& : fits, memory)
   for (int64_t b = 0; b < nw; ++b) {
     WindowTable &t = tables[omp_get_thread_num()];
     t.clear();
-    const int64_t q0 = b * w, q1 = std::min(nrow, q0 + w);
+    const int64_t q0 = first[b], q1 = first[b + 1];
+    const int cap = rule.most(q1 - q0);
     // padding slots are never read; they hold the window's first place
     std::fill(&h_idx[h_slice_ptr[q0 >> 6]], &h_idx[0] + h_slice_ptr[(q1 + 63) >> 6], (uint16_t)0);
     bool ok = true;
@@ -157,19 +158,18 @@ bool Sell::build_windows(const std::vector<int32_t> &order, int w, int cap) {
   }
   if (!memory) throw std::bad_alloc();
   if (!fits) return false;
-  std::vector<int32_t> h_lptr(nw + 1, 0);
+  std::vector<int2> h_win(nw + 1, int2{0, 0});
   umax = 0;
   for (int64_t b = 0; b < nw; ++b) {
     umax = std::max(umax, (int)lists[b].size());
-    h_lptr[b + 1] = h_lptr[b] + (int32_t)lists[b].size();
+    h_win[b + 1] = int2{first[b + 1], h_win[b].y + (int32_t)lists[b].size()};
   }
-  HostArr<int32_t> h_list(h_lptr[nw]);
+  HostArr<int32_t> h_list(h_win[nw].y);
 #pragma omp parallel for schedule(static)
-  for (int64_t b = 0; b < nw; ++b) std::copy(lists[b].begin(), lists[b].end(), &h_list[h_lptr[b]]);
-  win = w;
+  for (int64_t b = 0; b < nw; ++b) std::copy(lists[b].begin(), lists[b].end(), &h_list[h_win[b].y]);
   nwin = (int)nw;
   plen.upload(h_plen.p.get(), h_plen.n);
-  lptr.upload(h_lptr);
+  win.upload(h_win);
   list.upload(h_list.p.get(), h_list.n);
   idx.upload(h_idx.p.get(), h_idx.n);
   lrow.upload(h_lrow.p.get(), h_lrow.n);
@@ -236,16 +236,51 @@ std::vector<int32_t> hilbert_order(const double *X, int64_t n) {
   return order;
 }
 
-// Placement of a level whose sweeps run on windows of w rows: the Hilbert order
-// of the nodes, longest rows first inside every window.
-std::vector<int32_t> window_placement(const std::vector<int32_t> &order, int w, const std::vector<int64_t> &ptr) {
+// Placement of a level whose sweeps run on windows: the Hilbert order of the
+// nodes, longest rows first inside every window.
+std::vector<int32_t> window_placement(const std::vector<int32_t> &order, const std::vector<int32_t> &first,
+                                      const std::vector<int64_t> &ptr) {
   std::vector<int32_t> p = order;
-  const int64_t n = (int64_t)p.size();
 #pragma omp parallel for schedule(static)
-  for (int64_t a = 0; a < n; a += w)
-    std::stable_sort(p.begin() + a, p.begin() + std::min<int64_t>(n, a + w),
+  for (size_t b = 0; b < first.size() - 1; ++b)
+    std::stable_sort(p.begin() + first[b], p.begin() + first[b + 1],
                      [&](int32_t i, int32_t j) { return ptr[i + 1] - ptr[i] > ptr[j + 1] - ptr[j]; });
   return p;
+}
+
+// The windows again, those that gather too much halved (at a slice) until they
+// do not; empty if a slice alone does
+std::vector<int32_t> split_windows(const std::vector<int32_t> &order, const std::vector<int32_t> &first,
+                                   const std::vector<int64_t> &ptr, const std::vector<int32_t> &cols,
+                                   const m3::SweepRule &rule) {
+  std::vector<int32_t> pos(order.size());
+  for (size_t i = 0; i < order.size(); ++i) pos[order[i]] = (int32_t)i;
+  WindowTable t;
+  auto fits = [&](int32_t q0, int32_t q1) {
+    t.clear();
+    for (int32_t q = q0; q < q1; ++q)
+      for (int64_t k = ptr[order[q]]; k < ptr[order[q] + 1]; ++k) {
+        t.at(pos[cols[k]]);
+        if ((int)t.list.size() > rule.most(q1 - q0)) return false;
+      }
+    return true;
+  };
+  std::vector<int32_t> out{0}, todo;  // todo: ends of the pieces still to look at, the next one last
+  for (size_t b = 0; b + 1 < first.size(); ++b) {
+    todo.assign(1, first[b + 1]);
+    while (!todo.empty()) {
+      const int32_t q0 = out.back(), q1 = todo.back();
+      if (fits(q0, q1)) {
+        out.push_back(q1);
+        todo.pop_back();
+      } else if (q1 - q0 <= 64) {
+        return {};
+      } else {
+        todo.push_back(q0 + ((q1 - q0 + 127) / 128) * 64);
+      }
+    }
+  }
+  return out;
 }
 
 using clk = std::chrono::steady_clock;
@@ -444,14 +479,28 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
       std::vector<int64_t> ptr;
       std::vector<int32_t> cols;
       adjacency(lv.h_el2nod, lv.nel, lv.nnod, 10, ALL10, 10, ALL10, ptr, cols);
-      const int w = l < nmg - 1 ? m3::sweep_window(lv.nnod) : 0;
+      const int w = l < nmg - 1 ? m3::sweep_window(c->sweep_rule, lv.nnod) : 0;
       if (w) {
         M3_REQUIRE(m->GCOORD, M3_E_ARG, "missing GCOORD");
-        const std::vector<int32_t> order = hilbert_order(m->GCOORD, lv.nnod), place = window_placement(order, w, ptr);
-        mark("space-filling order");
-        lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9, &place);
+        const std::vector<int32_t> order = hilbert_order(m->GCOORD, lv.nnod);
+        std::vector<int32_t> first;
+        for (int64_t q = 0; q < lv.nnod; q += w) first.push_back((int32_t)q);
+        first.push_back((int32_t)lv.nnod);
+        auto build = [&] {
+          const std::vector<int32_t> place = window_placement(order, first, ptr);
+          lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9, &place);
+        };
+        build();
         mark("level connectivity + K pattern");
-        if (!lv.K.build_windows(order, w, m3::SWEEP_CAP)) lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
+        if (!lv.K.build_windows(order, first, c->sweep_rule)) {
+          first = split_windows(order, first, ptr, cols, c->sweep_rule);
+          if (first.empty()) {
+            lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
+          } else {
+            build();
+            M3_REQUIRE(lv.K.build_windows(order, first, c->sweep_rule), M3_E_MESH, "sweep windows do not fit");
+          }
+        }
         mark("sweep windows");
       } else {
         lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
@@ -708,6 +757,18 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
     c->dens.alloc(f.nnod);
     mark("work space");
     c->have_mesh = true;
+  });
+}
+
+int m3_sweep_windows(m3_ctx *c, int64_t rows, int32_t split, int32_t limit) {
+  return guard(c, [&] {
+    M3_REQUIRE(rows >= 0 && split >= 0 && limit >= 0 && limit <= m3::SWEEP_LIMIT, M3_E_ARG,
+               "sweep windows: sizes must not be negative, limit at most 6300");
+    m3::SweepRule r;
+    if (rows) r.rows = rows;
+    if (split) r.split = split;
+    if (limit) r.limit = limit;
+    c->sweep_rule = r;
   });
 }
 
@@ -1446,6 +1507,8 @@ int m3_stats(m3_ctx *c, int64_t *out, int32_t nout) {
     v.push_back(c->chol.nlev);
     v.push_back(c->chol.H);
     for (int l = 0; l < c->nmg; ++l) v.push_back(c->L[l].K.nslot);
+    for (int l = 0; l < c->nmg; ++l) v.push_back(c->L[l].K.nwin);
+    for (int l = 0; l < c->nmg; ++l) v.push_back(c->L[l].K.nwin ? c->L[l].K.umax : 0);
     for (int i = 0; i < nout && i < (int)v.size(); ++i) out[i] = v[i];
   });
 }

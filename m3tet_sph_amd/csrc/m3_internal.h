@@ -5,6 +5,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <memory>
@@ -141,21 +142,44 @@ __device__ inline int64_t sell_base(const SellT<T> &K, int64_t row) {
 }
 
 // What a sweep reads of a 3x3 operator besides its values (k_sparse.hip).
-// win == 0: the rows are in index order and col holds their columns.  win > 0:
-// the vectors are in a space-filling order of the nodes, win of them per
-// window; a window's rows sit in the slices by decreasing length, lrow being a
-// position's place in the window's stretch of the vectors; window b gathers the
-// entries list[lptr[b] .. lptr[b+1]) of the vector and idx is a slot's place
-// among them.
+// Without windows the rows are in index order and col holds their columns.
+// With windows the vectors are in a space-filling order of the nodes; window b
+// is the rows at the places win[b].x .. win[b+1].x of it (from a multiple of 64
+// on, at most 512 of them); they sit in the slices by decreasing length, lrow
+// being a position's place in the window's stretch of the vectors; the window
+// gathers the entries list[win[b].y .. win[b+1].y) of the vector and idx is a
+// slot's place among them.
 struct SweepPat {
   const int64_t *slice_ptr;
   const int32_t *len;   // stored blocks per position
   const int32_t *col;
   const uint16_t *idx, *lrow;
-  const int32_t *lptr, *list;
+  const int2 *win;
+  const int32_t *list;
   int64_t n;
   int32_t nsl;          // slices
 };
+
+namespace m3 {
+// Which levels are swept in windows, and when a window is split.  The LDS of all
+// workgroups of a sweep is that of its largest window: up to 2,900 gathered
+// entries leave room for as many workgroups per CU as the waves allow (two in
+// FP64, four in FP32; the meshes here gather 1,350 to 1,450 and at most 1,837 per
+// 512 rows), so a window of more is halved, down to the 64 rows of a slice.
+// A slice may gather as many as fit into the LDS of a CU beside its sums; a
+// level with a slice of more (a node with thousands of neighbours) is swept
+// without windows.  337,986 rows, us per sweep in FP64 / BF16: 131 / 41.6 as they
+// are, 139 / 49.3 with all windows halved, 214 / 87.3 in slices of 64 rows, 157 /
+// 56.0 without windows: a piece costs more than its share, so only the windows
+// that need it are split, and one of them in a mesh does not cost the others
+// their form.
+constexpr int SWEEP_LIMIT = 6300;
+struct SweepRule {
+  int64_t rows = 131072;                      // fewest rows of a level with windows (sweep_window)
+  int32_t split = 2900, limit = SWEEP_LIMIT;  // most entries of a window, of a slice
+  int most(int64_t nr) const { return nr > 64 ? std::min(split, limit) : limit; }
+};
+}  // namespace m3
 
 struct Sell {
   int64_t nrow = 0, ncol = 0, nslot = 0, nnz = 0;
@@ -171,18 +195,21 @@ struct Sell {
   // place of each node
   std::vector<int32_t> h_vperm, h_vpos;
   DBuf<int32_t> vperm, vpos;
-  // windowed sweeps (SweepPat): rows per window (0: none), windows, the most
-  // vector entries that one window gathers
-  int win = 0, nwin = 0, umax = 0;
-  DBuf<int32_t> plen, lptr, list;
+  // windowed sweeps (SweepPat): windows (0: none), the most vector entries that
+  // one of them gathers
+  int nwin = 0, umax = 0;
+  DBuf<int2> win;
+  DBuf<int32_t> plen, list;
   DBuf<uint16_t> idx, lrow;
   // build from sorted per-row column lists (CSR); uploads pattern, allocates
   // val.  place (may be NULL): the row at each position
   void build(int64_t nrow_, int64_t ncol_, const std::vector<int64_t> &ptr,
              const std::vector<int32_t> &cols, int bs_, const std::vector<int32_t> *place = nullptr);
-  // window lists for windows of w rows of the vector order; false (and nothing
-  // kept) if one of them gathers more than cap entries
-  bool build_windows(const std::vector<int32_t> &order, int w, int cap);
+  // window lists; first: the first row of each window in the vector order, and
+  // nrow.  false (and nothing kept) if a window gathers more entries than rule
+  // allows one of its size
+  bool build_windows(const std::vector<int32_t> &order, const std::vector<int32_t> &first,
+                     const m3::SweepRule &rule);
   int64_t base_of(int64_t row) const {
     const int64_t q = h_ipos.empty() ? row : (int64_t)h_ipos[row];
     return h_slice_ptr[q >> 6] + (q & 63);
@@ -193,7 +220,7 @@ struct Sell {
   const int32_t *vpos_p() const { return h_vpos.empty() ? nullptr : vpos.p; }
   SellView view() { return SellView{slice_ptr.p, rowlen.p, col.p, val.p, nslot, perm_p(), ipos_p()}; }
   SweepPat sweep() const {
-    return SweepPat{slice_ptr.p, win ? plen.p : rowlen.p, col.p, idx.p, lrow.p, lptr.p, list.p, nrow,
+    return SweepPat{slice_ptr.p, nwin ? plen.p : rowlen.p, col.p, idx.p, lrow.p, win.p, list.p, nrow,
                     (int32_t)(h_slice_ptr.size() - 1)};
   }
 };
@@ -350,6 +377,7 @@ struct m3_ctx {
   DBuf<double> scal;               // device scalars
   double *h_scal = nullptr;        // pinned host mirror
   double *h_part = nullptr;        // pinned: partial sums that the host adds (512)
+  m3::SweepRule sweep_rule;        // of the meshes that are set from now on
   // CG / Patera vectors (3*nnod or nV)
   DBuf<double> cg_r, cg_q, cg_Kq, cg_x, cg_b;
   DBuf<double> Uv, Zv, Yv, Rhs;
@@ -476,10 +504,8 @@ void launch_diag_inv(m3_ctx *c, int l);
 void launch_lumped_mm(m3_ctx *c);
 
 // sparse kernels
-// rows per sweep window of a level of n nodes (0: no windows), and the most
-// vector entries a window may gather (96 KB of LDS in FP64)
-int sweep_window(int64_t n);
-constexpr int SWEEP_CAP = 4096;
+// rows per sweep window of a level of n nodes (0: no windows)
+int sweep_window(const SweepRule &r, int64_t n);
 void nan_flag(hipStream_t s, const double *x, int64_t n, int *flag);  // atomicOr(flag, 32) on a NaN
 void spmv_K(hipStream_t s, LevelDev &lv, const double *x, double *y);  // node order; lv.r0 and lv.r1 are work space
 // vectors of a level between the node order and K's vector order

@@ -1,7 +1,7 @@
 """The sweeps of the multigrid levels against the stored operator: levels below
 the window size limit (one slice per workgroup, its blocks dealt to waves), and
-levels that are swept in windows, with a last window that is not full, on
-generated shells and on the unstructured mesh file.  K x, the transfers and the
+levels that are swept in windows, with a last window that is not full, with
+windows split and given up, on generated shells and on the unstructured mesh file.  K x, the transfers and the
 diagonal against SciPy products of m3_get_operator's matrix; one velocity solve
 in both precisions against each other."""
 import os
@@ -14,20 +14,48 @@ from tests.conftest import relerr
 pytestmark = pytest.mark.gpu
 GOLD = os.path.join(os.path.dirname(__file__), "golden", "EarthShell_n37k.mat")
 
-# nodes of the finest level: 5,778 (a last slice of 18 rows), 92,178, 174,114
-# (a last window of 34 rows), 289,174 of the file
-CASES = [dict(level=1, nlayer=2, nmg=2), dict(level=2, nlayer=1, nmg=3), dict(level=1, nlayer=2, nmg=4), None]
+# nodes of the finest level: 5,778 (a last slice of 18 rows), 92,178, 337,986
+# (a last window of 66 rows), 289,174 of the file, 174,114 (a last window of 34 rows)
+CASES = [dict(level=1, nlayer=2, nmg=2), dict(level=2, nlayer=1, nmg=3), dict(level=1, nlayer=2, nmg=4), None,
+         dict(level=2, nlayer=2, nmg=3)]
+WINDOWS = [0, 0, 661, 565, 341]
+
+# The same with other windows (fewest rows, most entries of a window, of 64 rows;
+# 0: the default).  Unforced, the windows of the 174,114 nodes gather 1,349
+# entries on average and at most 1,705, their 64-row slices at most 447.  Levels
+# of 174,114 and 23,058 nodes in windows, so that both ends of a transfer are in
+# vector order; a few windows split; windows of 64 to 256 rows; of 64 rows alone;
+# and a slice that gathers too much, so that a large level has none
+FORCED = [(3, (2000, 0, 0), lambda w: w == [341, 46, 0]),
+          (3, (0, 1650, 0), lambda w: 341 < w[0] < 400),
+          (2, (1000, 600, 0), lambda w: 2 * 46 < w[0] < 361),
+          (2, (1000, 1, 0), lambda w: w[0] == 361),
+          (3, (0, 0, 300), lambda w: w == [0, 0, 0])]
 
 
-@pytest.mark.parametrize("shape", CASES, ids=["small", "direct", "windows", "file"])
-def test_level_operators(shape):
-    from m3tet_sph_amd import api, fields as F, mesh as M
-    m = M.build_from_file(GOLD, nmg=2, device=0) if shape is None else M.build_shell(**shape, device=0)
+@pytest.mark.parametrize("k", range(len(CASES)), ids=["small", "direct", "windows", "file", "windows34"])
+def test_level_operators(k):
+    from m3tet_sph_amd import mesh as M
+    m = M.build_from_file(GOLD, nmg=2, device=0) if CASES[k] is None else M.build_shell(**CASES[k], device=0)
+    _check_levels(m, None, lambda w: w[0] == WINDOWS[k] and not any(w[1:]))
+
+
+@pytest.mark.parametrize("nmg,rule,expect", FORCED, ids=["levels", "some_split", "split", "slices", "none"])
+def test_level_operators_with_other_windows(nmg, rule, expect):
+    from m3tet_sph_amd import mesh as M
+    _check_levels(M.build_shell(level=2, nlayer=2, nmg=nmg, device=0), rule, expect)
+
+
+def _check_levels(m, rule, expect):
+    from m3tet_sph_amd import api, fields as F
     T = (m.r_surf - m.GCOORD_SPH[:, 2]) / (m.r_surf - m.r_cmb) + 0.03 * np.sin(7 * m.GCOORD[:, 0])
     Visc, Dens = F.material(T, 1e3)
     ifix, vfix = F.plate_bcs(m)
-    ctx = api.StokesContext(m)
+    ctx = api.StokesContext(m, sweep_windows=rule)
     try:
+        st = ctx.stats()
+        print("nodes", [L.nnod for L in m.levels], "windows", st["windows"], "entries", st["window_entries"])
+        assert expect(st["windows"])
         ctx.set_bc(ifix, vfix)
         ctx.assemble(Visc, Dens, F.physics())
         ctx.restrict_stiffmat()
