@@ -60,7 +60,6 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 
 HBM_PEAK_GBS = 8000.0
-WINDOW_ROWS = 131072  # levels of this many nodes or more are swept in windows (m3::sweep_window)
 
 # HBM bytes per launch of the dominant kernel, measured with two rocprofv3
 # counter passes (FETCH_SIZE x 2.0000 + WRITE_SIZE x 1.0000, factors from the
@@ -76,14 +75,14 @@ def log(*a):
     print("[bench]", *a, file=sys.stderr, flush=True)
 
 
-def sweep_bytes(nnzb, nnod, blk_val_bytes=72, vec_bytes=8):
+def sweep_bytes(nnzb, nnod, blk_val_bytes=72, vec_bytes=8, windows=0):
     """Algorithmic bytes of one fused Jacobi sweep r = r0 - K d; d' = d + w D^-1 r
     on the fine level: every stored 3x3 block once (its nine values,
     blk_val_bytes: 72 in FP64, 20 in the packed BF16 layout of eight BF16
     values and an FP32 v8; + its column: an int32, or a two-byte place in the
-    window on the levels that are swept in windows), the row table, and per
+    window on a level that the context sweeps in windows), the row table, and per
     row the vectors d (gather, perfect reuse), r0, D^-1 read and d' written."""
-    return nnzb * (blk_val_bytes + (2 if nnod >= WINDOW_ROWS else 4)) + nnod * 4 + nnod * 3 * 4 * vec_bytes
+    return nnzb * (blk_val_bytes + (2 if windows else 4)) + nnod * 4 + nnod * 3 * 4 * vec_bytes
 
 
 def cpu_threads():
@@ -131,11 +130,12 @@ def roofline(ctx, mesh, api, run_once, form, config):
     run_once()
     pr = api.profile_read(ctx)
     api.profile(ctx, False)
-    nnzb, nnod = ctx.stats()["nnzb"][0], mesh.nnod
+    st = ctx.stats()
+    nnzb, nnod, windows = st["nnzb"][0], mesh.nnod, st["windows"][0]
     if form == "fp64":
-        nsw, tsw, bsw, bpl = pr["n_fp64"], pr["t_fp64"], pr["b_fp64"], sweep_bytes(nnzb, nnod, 72, 8)
+        nsw, tsw, bsw, bpl = pr["n_fp64"], pr["t_fp64"], pr["b_fp64"], sweep_bytes(nnzb, nnod, 72, 8, windows)
     else:
-        nsw, tsw, bsw, bpl = pr["n_mixed"], pr["t_mixed"], pr["b_mixed"], sweep_bytes(nnzb, nnod, 20, 4)
+        nsw, tsw, bsw, bpl = pr["n_mixed"], pr["t_mixed"], pr["b_mixed"], sweep_bytes(nnzb, nnod, 20, 4, windows)
     if nsw and abs(bsw / nsw - bpl) > 1e-6 * bpl:
         raise SystemExit(f"bench.py: sweep bytes disagree with the library ({bsw / nsw} vs {bpl})")
     avg = tsw / max(nsw, 1)
@@ -144,7 +144,7 @@ def roofline(ctx, mesh, api, run_once, form, config):
     t_all, b_all, n_all = tsw + pr["t_vcycle_other"], bsw + pr["b_vcycle_other"], nsw + pr["n_vcycle_other"]
     vc = b_all / t_all / 1e9
     log(f"V-cycle: {n_all} launches, {t_all * 1e3:.2f} ms, {b_all / 1e9:.2f} GB -> {vc:.0f} GB/s")
-    kern = ("k_sweep_win" if nnod >= WINDOW_ROWS else "k_sweep") + ("<double,double,6>" if form == "fp64" else "<B16P,float,6>")
+    kern = ("k_sweep_win" if windows else "k_sweep") + ("<double,double,6>" if form == "fp64" else "<B16P,float,6>")
     cp = round(api.copy_rate(1 << 30, 20), 1)   # plain copy kernel of 1 GiB, read + write bytes
     log(f"copy kernel: {cp:.0f} GB/s")
     return dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",
