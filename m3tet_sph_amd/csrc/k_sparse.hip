@@ -592,7 +592,7 @@ __global__ __launch_bounds__(RB) void k_dot(int64_t n, const double *a, const do
 // 135 / 1,403 us at 5,778 / 337,986 rows (FP64) and 106 / 682 us (mixed), so
 // 129 / 1,357 and 101 / 673 us.
 // scal: 0 r.d of the current direction, 3 alpha, 4 + parity: r.d by iteration
-constexpr int CGB = 512;  // workgroups (and partial sums) of these kernels, at most
+constexpr int CGB = m3::HOST_PARTS;  // workgroups (and partial sums) of these kernels, at most
 // partial sums of (r - rlast).d = -alpha Kq.d (0 in the first iteration) and
 // r.d, with d as the V-cycle leaves it
 template <class VT>

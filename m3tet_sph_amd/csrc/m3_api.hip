@@ -400,7 +400,7 @@ int m3_create(m3_ctx **ctx, int hip_device) {
     HIPCHECK(hipSetDevice(hip_device));
     HIPCHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIPCHECK(hipHostMalloc(&c->h_scal, 64 * sizeof(double)));
-    HIPCHECK(hipHostMalloc(&c->h_part, 512 * sizeof(double)));
+    HIPCHECK(hipHostMalloc(&c->h_part, m3::HOST_PARTS * sizeof(double)));
     c->scal.alloc(64);
     c->errflag.alloc(1);
     m3::upload_sf_tables();

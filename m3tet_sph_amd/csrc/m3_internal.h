@@ -161,6 +161,8 @@ struct SweepPat {
 };
 
 namespace m3 {
+// the most workgroups of a kernel that leaves its partial sums to the host
+constexpr int HOST_PARTS = 512;
 // Which levels are swept in windows, and when a window is split.  The LDS of all
 // workgroups of a sweep is that of its largest window: up to 2,900 gathered
 // entries leave room for as many workgroups per CU as the waves allow (two in
@@ -376,7 +378,7 @@ struct m3_ctx {
   DBuf<double> partial;            // per-block partial sums
   DBuf<double> scal;               // device scalars
   double *h_scal = nullptr;        // pinned host mirror
-  double *h_part = nullptr;        // pinned: partial sums that the host adds (512)
+  double *h_part = nullptr;        // pinned: partial sums that the host adds (m3::HOST_PARTS)
   m3::SweepRule sweep_rule;        // of the meshes that are set from now on
   // CG / Patera vectors (3*nnod or nV)
   DBuf<double> cg_r, cg_q, cg_Kq, cg_x, cg_b;
