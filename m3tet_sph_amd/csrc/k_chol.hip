@@ -447,8 +447,7 @@ struct PotrfLds {
   double RD[PW][TS];      // each wave's copy of 1 / L[c][c]
   double Tf[1024];        // B X_AA of the doubling steps
 };
-__device__ inline void potrf_tile(int J, double *A, const int32_t *pos2dof, double *dinv, double *dinvT, int *err,
-                                  PotrfLds &lds) {
+__device__ inline void potrf_tile(int J, double *A, const int32_t *pos2dof, double *dinv, int *err, PotrfLds &lds) {
   auto &S = lds.S;
   auto &P = lds.P;
   auto &RD = lds.RD;
@@ -589,12 +588,8 @@ __device__ inline void potrf_tile(int J, double *A, const int32_t *pos2dof, doub
   }
   __syncthreads();
   double *Di = dinv + (int64_t)J * TT;
-  double *DiT = dinvT + (int64_t)J * TT;
 #pragma unroll 4
-  for (int c = w; c < TS; c += PW) {
-    Di[t + TS * c] = X[t][c];   // Di[r + 64c] = X[r][c]
-    DiT[t + TS * c] = X[c][t];  // DiT[r + 64c] = X[c][r]
-  }
+  for (int c = w; c < TS; c += PW) Di[t + TS * c] = X[t][c];  // Di[r + 64c] = X[r][c]
   if (threadIdx.x == 0 && bad) atomicOr(err, 16);
 }
 
@@ -607,8 +602,8 @@ __device__ inline void potrf_tile(int J, double *A, const int32_t *pos2dof, doub
 // factorisation of 275 tile columns 2.74 -> 2.40 ms, of 1,844 (99 levels, bound by
 // the products) 18.59 -> 18.16, of 34 columns 0.64 -> 0.63.
 __global__ __launch_bounds__(64 * PW) void k_potrf_update(const int32_t *cols, int ncol, const int32_t *diagtile,
-                                                      const int32_t *pos2dof, double *dinv, double *dinvT, int *err,
-                                                      UpdArgs u, int chunk0) {
+                                                      const int32_t *pos2dof, double *dinv, int *err, UpdArgs u,
+                                                      int chunk0) {
   __shared__ union Lds {
     PairLds upd;
     PotrfLds potrf;
@@ -617,15 +612,15 @@ __global__ __launch_bounds__(64 * PW) void k_potrf_update(const int32_t *cols, i
   const int b = blockIdx.x;
   if (b < ncol) {
     const int J = cols[b];
-    potrf_tile(J, u.tiles + (int64_t)diagtile[J] * TT, pos2dof, dinv, dinvT, err, lds.potrf);
+    potrf_tile(J, u.tiles + (int64_t)diagtile[J] * TT, pos2dof, dinv, err, lds.potrf);
   } else {
     update_chunk(u, chunk0 + b - ncol, lds.upd);
   }
 }
 
-// L_IJ = C_IJ inv(L_JJ)'  and its transposed copy
+// L_IJ = C_IJ inv(L_JJ)'
 __global__ __launch_bounds__(256) void k_trsm(const int32_t *tile, const int32_t *col, int task0,
-                                              double *tiles, double *tilesT, const double *dinv) {
+                                              double *tiles, const double *dinv) {
   const int task = task0 + blockIdx.x;
   double *C = tiles + (int64_t)tile[task] * TT;
   __shared__ double sA[TS][TS + 1];
@@ -633,7 +628,7 @@ __global__ __launch_bounds__(256) void k_trsm(const int32_t *tile, const int32_t
   MfAcc m;
   mf_zero(m);
   tile_mm_mf(C, dinv + (int64_t)col[task] * TT, true, sA, sB, m);
-  // the product to LDS (row-major), then both copies written coalesced
+  // the product through LDS, to be written coalesced
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int r0 = 32 * (w >> 1), c0 = 32 * (w & 1), li = lane & 15, lq = lane >> 4;
   __syncthreads();
@@ -641,12 +636,10 @@ __global__ __launch_bounds__(256) void k_trsm(const int32_t *tile, const int32_t
     for (int bj = 0; bj < 2; ++bj)
       for (int r = 0; r < 4; ++r) sA[r0 + 16 * bi + lq + 4 * r][c0 + 16 * bj + li] = m.d[bi][bj][r];
   __syncthreads();
-  double *CT = tilesT + (int64_t)tile[task] * TT;
 #pragma unroll
   for (int q = 0; q < TT / 256; ++q) {
-    const int t = threadIdx.x + 256 * q, r = t & 63, c = t >> 6;
-    C[t] = sA[r][c];   // C[r + 64c]
-    CT[t] = sA[c][r];  // CT[r + 64c] = C[c + 64r]
+    const int t = threadIdx.x + 256 * q;
+    C[t] = sA[t & 63][t >> 6];  // C[r + 64c]
   }
 }
 
@@ -769,11 +762,6 @@ __global__ void k_from_tiles(int64_t n, const int32_t *dof2pos, const double *x,
   if (d >= n) return;
   const int p = dof2pos[d];
   out[d] = p >= 0 ? x[p] : 0.0;
-}
-
-__global__ void k_zero(int64_t n, double *x) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) x[i] = 0.0;
 }
 
 inline unsigned nblk(int64_t n, int bs = 256) { return (unsigned)((n + bs - 1) / bs); }
@@ -1190,9 +1178,7 @@ void chol_analyse(m3_ctx *c) {
   fw.upload(ch.fwd);
   bw.upload(ch.bwd);
   ch.tiles.alloc((size_t)ch.ntile * TT);
-  ch.tilesT.alloc((size_t)ch.ntile * TT);
   ch.dinv.alloc((size_t)T * TT);
-  ch.dinvT.alloc((size_t)T * TT);
   ch.X.alloc((size_t)(ch.nX + ch.nZ + ch.nT) * TT);
   ch.XT.alloc((size_t)(ch.nX + ch.nZ) * TT);
   ch.X32.alloc((size_t)(ch.nX + ch.nZ) * TT);
@@ -1216,11 +1202,11 @@ void chol_factor(m3_ctx *c) {
     const int c0 = ch.h_lev_ptr[l], nc = ch.h_lev_ptr[l + 1] - c0;
     const int e1 = l + 1 < ch.nlev ? ch.h_upd_ptr[2 * l + 3] : u1;
     hipLaunchKernelGGL(k_potrf_update, dim3(nc + (e1 - u1)), dim3(64 * PW), 0, s, ch.lev_cols.p + c0, nc, ch.diagtile.p,
-                       ch.pos2dof.p, ch.dinv.p, ch.dinvT.p, c->errflag.p, upd, u1);
+                       ch.pos2dof.p, ch.dinv.p, c->errflag.p, upd, u1);
     const int t0 = ch.h_trsm_ptr[l], t1 = ch.h_trsm_ptr[l + 1];
     if (t1 > t0)
       hipLaunchKernelGGL(k_trsm, dim3(t1 - t0), dim3(256), 0, s, ch.trsm_tile.p, ch.trsm_col.p, t0,
-                         ch.tiles.p, ch.tilesT.p, ch.dinv.p);
+                         ch.tiles.p, ch.dinv.p);
   }
   hipLaunchKernelGGL(k_inv, dim3((unsigned)ch.inv_x.n), dim3(256), 0, s, ch.inv_x.p, ch.inv_row.p, ch.dinv.p, ch.X.p,
                      ch.XT.p, ch.X32.p, ch.XT32.p);

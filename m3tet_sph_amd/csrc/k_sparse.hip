@@ -657,9 +657,9 @@ __global__ void k_axpy(int64_t n, double a, const double *x, double *y) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) y[i] += a * x[i];
 }
-__global__ void k_xpby(int64_t n, const double *x, double b, double *y) {
+__global__ void k_scal(int64_t n, double a, double *y) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) y[i] = (x ? x[i] : 0.0) + b * y[i];
+  if (i < n) y[i] *= a;
 }
 __global__ void k_copy(int64_t n, const double *x, double *y) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -989,10 +989,12 @@ thread_local hipEvent_t prof_start = nullptr, prof_stop = nullptr;
 // rows, 34.1 / 102 us on 256,050.
 int sweep_window(const SweepRule &r, int64_t n) { return n >= r.rows ? SW_WIN : 0; }
 
-// do the values stay in the last-level cache (256 MB) between sweeps?
+// do the values stay in the last-level cache (256 MB) between sweeps?  In BF16,
+// up to some 370,000 rows; FP64 values of a level that has windows do not (28
+// blocks a row of 74 bytes: 270 MB at 131,072 rows)
 template <class MT>
 static bool sweep_resident(const Sell &K) {
-  return (double)K.nnz * (block_value_bytes<MT>() + 2.0) < 230e6;
+  return !std::is_same<MT, double>::value && (double)K.nnz * (block_value_bytes<MT>() + 2.0) < 230e6;
 }
 // workgroups of a sweep, each with its partial sum (MODE bit 8)
 template <class MT>
@@ -1014,8 +1016,13 @@ static void launch_sweep(hipStream_t s, const Sell &K, const MT *val, const Swee
                                      (int)lds));
       launch_timed_lds(kern, dim3((unsigned)sweep_grid<MT>(K)), dim3(64 * SW_NW), lds, s, P, K.nwin, K.umax, val, v);
     };
-    if (sweep_resident<MT>(K)) go(k_sweep_win<MT, VT, MODE, UNR, true>);
-    else go(k_sweep_win<MT, VT, MODE, UNR, false>);
+    if constexpr (!std::is_same<MT, double>::value) {
+      if (sweep_resident<MT>(K)) {
+        go(k_sweep_win<MT, VT, MODE, UNR, true>);
+        return;
+      }
+    }
+    go(k_sweep_win<MT, VT, MODE, UNR, false>);
   } else {
     launch_timed(k_sweep<MT, VT, MODE, SD_W, SD_UNR>, dim3((unsigned)P.nsl), dim3(64 * SD_W), s, P, val, v);
   }
@@ -1084,15 +1091,15 @@ static const double WDOWN[3] = {0.25, 0.4, 0.9}, WUP[3] = {0.9, 0.4, 0.25};
 
 template <class VT>
 struct VecSet {
-  VT *r0, *r1, *d, *dn, *dd, *rr;
+  VT *r0, *r1, *d, *dn, *dd;
   const VT *dinv;
 };
 
 static VecSet<double> vecs64(LevelDev &l) {
-  return VecSet<double>{l.r0.p, l.r1.p, l.d.p, l.dn.p, l.dd.p, l.rr.p, l.dinv.p};
+  return VecSet<double>{l.r0.p, l.r1.p, l.d.p, l.dn.p, l.dd.p, l.dinv.p};
 }
 static VecSet<float> vecs32(LevelDev &l) {
-  return VecSet<float>{l.r0f.p, l.r1f.p, l.df.p, l.dnf.p, l.ddf.p, l.rrf.p, l.dinv32.p};
+  return VecSet<float>{l.r0f.p, l.r1f.p, l.df.p, l.dnf.p, l.ddf.p, l.dinv32.p};
 }
 
 template <class MT>
@@ -1133,7 +1140,7 @@ static void vcycle_impl(m3_ctx *c, VecSet<VT> (*vs)(LevelDev &)) {
     VecSet<VT> v = vs(lv);
     const double *wd = l == 0 ? WDOWN1 : WDOWN;
     // level 0: r0 and d = w1 Dinv r0 were written by k_entry
-    // d (= w1 Dinv r0) is in v.d; rr = r0 is kept (v.r0 not overwritten)
+    // d (= w1 Dinv r0) is in v.d; v.r0 is kept
     const int kind = l == 0 ? pk : 2;
     const double b6 = sweep_bytes<MT>(lv, 4, sv), b2 = sweep_bytes<MT>(lv, 3, sv);
     { ProfScope ps(c, kind, true, b6); sweep<MT, VT>(s, lv, v.d, v.r0, v.dinv, wd[1], nullptr, v.dn); }
@@ -1232,7 +1239,7 @@ void build_mixed(m3_ctx *c) {
     fit(lv.dinv32, n3);
     hipLaunchKernelGGL((k_convert<double, float>), dim3(nblk(n3)), dim3(256), 0, s, n3, lv.dinv.p,
                        lv.dinv32.p);
-    for (auto *b : {&lv.r0f, &lv.r1f, &lv.df, &lv.dnf, &lv.ddf, &lv.rrf}) fit(*b, n3);
+    for (auto *b : {&lv.r0f, &lv.r1f, &lv.df, &lv.dnf, &lv.ddf}) fit(*b, n3);
     if (l < c->nmg - 1) {
       const int64_t np = lv.P_val.n, nr = lv.R_val.n;
       fit(lv.P_val32, np);
@@ -1275,9 +1282,6 @@ void nan_flag(hipStream_t s, const double *x, int64_t n, int *flag) {
 void axpy(hipStream_t s, double a, const double *x, double *y, int64_t n) {
   hipLaunchKernelGGL(k_axpy, dim3(nblk(n)), dim3(256), 0, s, n, a, x, y);
 }
-void xpby(hipStream_t s, const double *x, double b, double *y, int64_t n) {
-  hipLaunchKernelGGL(k_xpby, dim3(nblk(n)), dim3(256), 0, s, n, x, b, y);
-}
 void copy(hipStream_t s, const double *x, double *y, int64_t n) {
   hipLaunchKernelGGL(k_copy, dim3(nblk(n)), dim3(256), 0, s, n, x, y);
 }
@@ -1286,7 +1290,7 @@ void scale_mask(hipStream_t s, const double *x, const double *m, double *y, int6
 }
 void add_scalar(hipStream_t s, double *a, double v, int64_t n) { add_scalar_impl(s, a, v, n); }
 void scal(hipStream_t s, double a, double *y, int64_t n) {
-  hipLaunchKernelGGL(k_xpby, dim3(nblk(n)), dim3(256), 0, s, n, (const double *)nullptr, a, y);
+  hipLaunchKernelGGL(k_scal, dim3(nblk(n)), dim3(256), 0, s, n, a, y);
 }
 
 // ---- one MGPCG iteration sequence, device-resident scalars -----------------------------

@@ -236,8 +236,8 @@ struct CholTiles {
   std::vector<int32_t> h_colptr, h_rowtile;   // tile CSC (row tiles sorted)
   DBuf<int32_t> pos2dof;         // T*64: coarse dof (0-based) or -1 (padding)
   DBuf<int32_t> dof2pos;         // 3*nnod: tile position or -1 (fixed dof)
-  DBuf<double> tiles, tilesT;    // L tiles (column-major) and transposed copies
-  DBuf<double> dinv, dinvT;      // inverses of the diagonal tiles of L
+  DBuf<double> tiles;            // L tiles (column-major)
+  DBuf<double> dinv;             // inverses of the diagonal tiles of L
   DBuf<int64_t> gsrc, gdst;      // gather: operator value index -> tile value index
   DBuf<int32_t> diagtile;        // T: tile index of (J,J)
   // factorisation: tile tasks by dependency level
@@ -319,7 +319,7 @@ struct LevelDev {
   int64_t nfree = 0;
   // V-cycle work vectors (FP64 and FP32 variants)
   DBuf<double> r0, r1, d, dn, dd, rr;
-  DBuf<float> r0f, r1f, df, dnf, ddf, rrf;
+  DBuf<float> r0f, r1f, df, dnf, ddf;
 };
 
 namespace m3 {
@@ -536,7 +536,6 @@ void sl_advect(m3_ctx *c, const double *T, const double *U, double dt, double T_
                double *T_out);
 void rock_prop(m3_ctx *c, const double *T, const m3_rock_params *rp, double *Visc, double *Dens);
 double calculate_dt(m3_ctx *c, const double *U, double dt_adv_limit, double dtmax);
-void xpby(hipStream_t s, const double *x, double b, double *y, int64_t n);  // y = x + b*y
 void copy(hipStream_t s, const double *x, double *y, int64_t n);
 void scale_mask(hipStream_t s, const double *x, const double *m, double *y, int64_t n);
 double mean(m3_ctx *c, const double *a, int64_t n);
