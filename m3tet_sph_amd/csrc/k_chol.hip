@@ -36,13 +36,19 @@ constexpr int TS = 64;
 constexpr int TT = TS * TS;
 // The solves take the blocks of the first dissection levels as one, as many
 // whole levels as fit into this many tiles: fewer dependent launches against a
-// longer inversion, once per factorisation.  0 / 16 / 32 / 36 / 48 tiles, us per
-// FP64 iteration of the whole solver and per factorisation:
-//   34 tiles in all   157 / 143 / 142 / 135 / 137 and 546 / 581 / 581 / 637 / 630
-//   130               225 / 222 / 216 / 216 / 212 and 1,097 / 1,093 / 1,156 / 1,156 / 1,197
-//   275             1,429 / 1,422 / 1,406 / 1,403 / 1,355 and 2,667 / 2,662 / 2,675 / 2,740 / 2,728
-// (runs differ by 20 and 15).  A factorisation serves a few hundred iterations.
-constexpr int ROOT_TILES = 36;
+// longer inversion, once per factorisation.  us per factorisation, and per FP64 /
+// mixed iteration of the whole solver, with 0, 36, 48, 64 and 96 tiles (medians of
+// two runs, which differ by 1 % and in mixed iterations by up to 4 %):
+//   34 tiles in all    522   115.5/94.0    628  100/79      one block from 36 on
+//   73                 898  2282/1063      978  2268/1053  1038 2267/1050  1038 2267/1051  1118 2264/1044
+//   130                999   178/143      1078   170/128   1132  165/120   1177  162/118   1178  163/118
+//   275               2210  1241/594      2305  1240/592   2299 1239/589   2410 1236/586   2654 1239/584
+//   1,844            15,077 1641/857    15,088 1640/860  15,082 1635/854  15,076 1638/856 15,520 1635/855
+// A factorisation serves 70 iterations (a step of the time loop) to a few hundred.
+// 48 is a twentieth off them at 130 columns and free or nearly so elsewhere; 64
+// would take another hundredth off at 130 and a third of that at 275, for a
+// factorisation a twentieth longer at both.
+constexpr int ROOT_TILES = 48;
 constexpr int LEAF = 80;  // nodes per leaf block (40 / 80 / 160: 309 / 306 / 305 ms per c1 solve)
 
 // ---- host: nested dissection into tile-aligned blocks ----------------------------------
