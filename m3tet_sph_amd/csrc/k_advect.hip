@@ -215,7 +215,7 @@ namespace m3 {
 
 void sl_advect(m3_ctx *c, const double *T, const double *U, double dt, double T_cmb, double T_surf,
                double *T_out) {
-  M3_REQUIRE(!c->L.empty(), M3_E_STATE, "m3_sl_advect before m3_set_mesh");
+  M3_REQUIRE(c->have_mesh, M3_E_STATE, "m3_sl_advect before m3_set_mesh");
   M3_REQUIRE(T && U && T_out, M3_E_ARG, "null argument");
   M3_REQUIRE(std::isfinite(dt) && dt >= 0, M3_E_ARG, "dt must be finite and non-negative");
   const int64_t nV0 = c->L[0].nV;

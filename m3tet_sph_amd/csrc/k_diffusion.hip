@@ -310,7 +310,7 @@ using clk = std::chrono::steady_clock;
 namespace m3 {
 
 void diffusion_mesh(m3_ctx *c, const uint32_t *EL2NOD, int64_t nel, int64_t nnodT, double theta_cone) {
-  M3_REQUIRE(!c->L.empty(), M3_E_STATE, "m3_diffusion_mesh before m3_set_mesh");
+  M3_REQUIRE(c->have_mesh, M3_E_STATE, "m3_diffusion_mesh before m3_set_mesh");
   M3_REQUIRE(EL2NOD && nel > 0, M3_E_ARG, "empty element list");
   M3_REQUIRE(nnodT > 0 && nnodT <= c->nnod, M3_E_ARG, "nnodT must be in 1..nnod of the finest mesh");
   M3_REQUIRE(theta_cone > 0 && theta_cone < 90, M3_E_ARG, "theta_cone must be in (0, 90) degrees");

@@ -74,7 +74,7 @@ __global__ void k_umax(int64_t n, const double *frames, const double *U, double 
 namespace m3 {
 
 void rock_prop(m3_ctx *c, const double *T, const m3_rock_params *rp, double *Visc, double *Dens) {
-  M3_REQUIRE(!c->L.empty(), M3_E_STATE, "m3_rock_prop before m3_set_mesh");
+  M3_REQUIRE(c->have_mesh, M3_E_STATE, "m3_rock_prop before m3_set_mesh");
   M3_REQUIRE(T && rp, M3_E_ARG, "null argument");
   M3_REQUIRE(!(rp->Ea > 0 && rp->Ea < 1000), M3_E_ARG,
              " Activation energy PHYSICS.Ea seems to be in kJ/mol. Convert to J/mol.");
@@ -98,7 +98,7 @@ void rock_prop(m3_ctx *c, const double *T, const m3_rock_params *rp, double *Vis
 }
 
 double calculate_dt(m3_ctx *c, const double *U, double dt_adv_limit, double dtmax) {
-  M3_REQUIRE(!c->L.empty(), M3_E_STATE, "m3_calculate_dt before m3_set_mesh");
+  M3_REQUIRE(c->have_mesh, M3_E_STATE, "m3_calculate_dt before m3_set_mesh");
   M3_REQUIRE(U, M3_E_ARG, "null argument");
   const int64_t n = c->L[0].nnod;
   double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};

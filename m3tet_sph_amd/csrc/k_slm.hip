@@ -413,7 +413,7 @@ namespace m3 {
 
 void slm_advect(m3_ctx *c, const double *Ux, const double *Uy, const double *Uz, double *T, double dt,
                 const m3_slm_opts *opts, m3_slm_info *info) {
-  M3_REQUIRE(!c->L.empty(), M3_E_STATE, "m3_advect3d_slm_p_sph before m3_set_mesh");
+  M3_REQUIRE(c->have_mesh, M3_E_STATE, "m3_advect3d_slm_p_sph before m3_set_mesh");
   M3_REQUIRE(Ux && Uy && Uz && T, M3_E_ARG, "null argument");
   M3_REQUIRE(std::isfinite(dt) && dt >= 0, M3_E_ARG, "dt must be finite and non-negative");
   const int method_BT = opts ? opts->method_BT : M3_SLM_PC2;

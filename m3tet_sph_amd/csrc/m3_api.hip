@@ -447,7 +447,7 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
       tp = now;
     };
     c->L.clear();
-    c->adv.ready = false;
+    c->adv.ready = c->slm.ready = c->dif.ready = c->dif.assembled = false;
     c->L.resize(nmg);
     c->have_mesh = c->have_bc = c->assembled = c->restricted = c->factored = c->have_mixed = false;
     c->pack16_fresh = false;
@@ -594,7 +594,6 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
     }
     c->h_coord = X;
     c->h_sph = S;
-    c->dif.ready = c->dif.assembled = false;
     c->X.upload(X);
     c->S.upload(S);
     c->frames.upload(fr);

@@ -124,3 +124,29 @@ def test_identities_on_c1():
     with pytest.raises(api.M3Error):
         ctx.advect3d_slm_p_sph(Ux, Uy, Uz, bad, 0.02)
     ctx.close()
+
+
+def test_another_mesh_in_the_same_context(tiny, c0):
+    """The face table and the node frames belong to the mesh they were made for;
+    a mesh that is refused leaves none to advect on."""
+    import copy
+    from m3tet_sph_amd import api
+    ctx, fresh = api.StokesContext(tiny), api.StokesContext(c0)
+    try:
+        ctx.advect3d_slm_p_sph(*_flow(tiny), _field(tiny), 0.05)
+        ctx._set_mesh(c0)
+        got, _ = ctx.advect3d_slm_p_sph(*_flow(c0), _field(c0), 0.05)
+        want, _ = fresh.advect3d_slm_p_sph(*_flow(c0), _field(c0), 0.05)
+        assert np.array_equal(got, want)
+        bad = copy.copy(c0)
+        bad.levels = [copy.copy(L) for L in c0.levels]
+        bad.levels[1].EL2NOD = c0.levels[1].EL2NOD + c0.levels[1].nnod
+        with pytest.raises(api.M3Error, match="EL2NOD entry out of range"):
+            ctx._set_mesh(bad)
+        with pytest.raises(api.M3Error, match="before m3_set_mesh"):
+            ctx.advect3d_slm_p_sph(*_flow(c0), _field(c0), 0.05)
+        with pytest.raises(api.M3Error, match="before m3_set_mesh"):
+            ctx.diffusion_mesh()
+    finally:
+        ctx.close()
+        fresh.close()
