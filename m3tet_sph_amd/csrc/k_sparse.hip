@@ -298,6 +298,13 @@ __global__ void k_to_nodes(int64_t n3, const int32_t *perm, const double *x, dou
   const int64_t q = i / 3;
   y[3 * (int64_t)perm[q] + (i - 3 * q)] = x[i];
 }
+// the mask as a byte per dof in vector order (perm NULL: node order)
+__global__ void k_vmask(int64_t n3, const int32_t *perm, const double *mask, uint8_t *vmask) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n3) return;
+  const int64_t q = i / 3;
+  vmask[i] = mask[perm ? 3 * (int64_t)perm[q] + (i - 3 * q) : i] != 0.0;
+}
 // r = mask b: b in node order, r and the mask in vector order
 __global__ void k_rhs_in(int64_t n3, const int32_t *perm, const uint8_t *vmask, const double *b, double *r) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -1040,6 +1047,13 @@ void to_nodes(hipStream_t s, const LevelDev &lv, const double *x, double *y) {
     hipLaunchKernelGGL(k_to_nodes, dim3(nblk(n3)), dim3(256), 0, s, n3, lv.K.vperm_p(), x, y);
   else
     copy(s, x, y, n3);
+}
+
+void launch_vmask(hipStream_t s, LevelDev &lv) {
+  const int64_t n3 = 3 * lv.nnod;
+  if (lv.vmask.n != (size_t)n3) lv.vmask.alloc(n3);
+  hipLaunchKernelGGL(k_vmask, dim3(nblk(n3)), dim3(256), 0, s, n3, lv.K.vperm_p(), lv.mask.p, lv.vmask.p);
+  HIPCHECK(hipGetLastError());
 }
 
 void spmv_K(hipStream_t s, LevelDev &lv, const double *x, double *y) {

@@ -790,12 +790,7 @@ int m3_set_bc(m3_ctx *c, const int64_t *ifix, const double *vfix, int64_t nfix) 
       LevelDev &lv = c->L[l];
       std::vector<double> ml(mask.begin(), mask.begin() + 3 * lv.nnod);
       lv.mask.upload(ml);
-      std::vector<uint8_t> vm(3 * lv.nnod);
-      for (int64_t q = 0; q < lv.nnod; ++q) {
-        const int64_t r = lv.K.h_vperm.empty() ? q : (int64_t)lv.K.h_vperm[q];
-        for (int k = 0; k < 3; ++k) vm[3 * q + k] = ml[3 * r + k] != 0.0;
-      }
-      lv.vmask.upload(vm);
+      m3::launch_vmask(c->stream, lv);
       lv.nfree = (int64_t)std::count(ml.begin(), ml.end(), 1.0);
     }
     c->U0.upload(U0);

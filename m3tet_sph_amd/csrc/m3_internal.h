@@ -513,6 +513,7 @@ void spmv_K(hipStream_t s, LevelDev &lv, const double *x, double *y);  // node o
 // vectors of a level between the node order and K's vector order
 void to_places(hipStream_t s, const LevelDev &lv, const double *x, double *y);
 void to_nodes(hipStream_t s, const LevelDev &lv, const double *x, double *y);
+void launch_vmask(hipStream_t s, LevelDev &lv);  // lv.vmask from lv.mask
 void spmv_G(hipStream_t s, Sell &G, const double *q, double *y, const double *mask, const double *add = nullptr);
 void spmv_GT(hipStream_t s, Sell &GT, const double *z, double *y);
 void spmv_M(hipStream_t s, Sell &M, const double *x, double *y);
