@@ -828,22 +828,32 @@ __global__ __launch_bounds__(RB) void k_pp_update(int64_t n, int64_t n3, double 
 }
 
 // ---- Jacobi-preconditioned CG on a scalar matrix (pcg_solver_p.m:49-186) --------------
-// Two launches per iteration and no host in between: the direction and the
-// product, then the update.  A workgroup that needs a dot product adds the
+// Two launches per iteration (three for large matrices) and no host in between: the
+// direction and the product, then the update.  A workgroup that needs a dot product adds the
 // previous launch's partial sums itself (all in the same order, so all hold the
-// same value).  Both launches end at once when the residual has met the
+// same value).  All launches end at once when the residual has met the
 // tolerance, so the host can queue several iterations and read the state after
 // them; the iterates are those of a loop that looks every time.  Seven launches
 // and a blocking read per iteration took 55 us at 43,554 rows, this 20.
 // state: 0 r.d of the current direction, 1 |r|^2, 2 iterations done, 3 stopped
 // (1 converged, 2 NaN) as the direction's launches read it, 4 + parity: r.d by
 // iteration, 6 stopped as a direction's launch finds it.  No launch of several
-// workgroups reads a value that it writes: k_pcg_dir reads 3 and writes 6, the
-// update after it reads 6 and writes 3.
+// workgroups reads a value that it writes: k_pcg_dir and k_pcg_q read 3 and write
+// 6, the update after them reads 6 and writes 3.
 constexpr int PC_T = RB;
 __device__ inline void pc_part(double s, double *part, double *sh) {
   s = rb_block(s, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+// what the launch of a direction leaves: s is |r|^2, (r - rlast).d, r.d
+__device__ inline void pcg_state(double *state, const double *s, bool stop, double rr_stop, int it) {
+  state[1] = s[0];
+  if (stop) {
+    state[6] = s[0] < rr_stop ? 1.0 : 2.0;
+  } else {
+    state[0] = s[2];
+    state[4 + ((it + 1) & 1)] = s[2];
+  }
 }
 // partial sums: |r|^2 at up, (r - rlast).d at up + nu, r.d at up + 2 nu
 __global__ __launch_bounds__(PC_T) void k_pcg_start(int64_t n, const double *r, const double *Adi, double *up, int nu) {
@@ -897,15 +907,7 @@ __global__ __launch_bounds__(64 * SP_W) void k_pcg_dir(SellView A, int64_t n, co
 #pragma unroll
   for (int j = 0; j < 3; ++j) s[j] = (tot[j][0] + tot[j][1]) + (tot[j][2] + tot[j][3]);
   const bool stop = it > 1 && !(s[0] >= rr_stop);  // |r|^2 below the tolerance's, or NaN
-  if (blockIdx.x == 0 && t == 0) {
-    state[1] = s[0];
-    if (stop) {
-      state[6] = s[0] < rr_stop ? 1.0 : 2.0;
-    } else {
-      state[0] = s[2];
-      state[4 + ((it + 1) & 1)] = s[2];
-    }
-  }
+  if (blockIdx.x == 0 && t == 0) pcg_state(state, s, stop, rr_stop, it);
   if (stop || w != 0) return;
   const double beta = it == 1 ? 0.0 : s[1] / rdlast;
   double dot = 0;
@@ -919,6 +921,44 @@ __global__ __launch_bounds__(64 * SP_W) void k_pcg_dir(SellView A, int64_t n, co
   }
   for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
   if (lane == 0) qp[blockIdx.x] = dot;
+}
+// The same as two launches for a large matrix: q in place, a vector stream, then
+// Aq with one gathered vector instead of three (r, Adi and qlast), PC_BLOCKS
+// workgroups and so as many partial sums at most (k_pcg_dir leaves one per
+// slice, and each workgroup of the update adds all of them).
+constexpr int PC_BLOCKS = 2048;
+__global__ __launch_bounds__(PC_T) void k_pcg_q(int64_t n, const double *r, const double *Adi, double *q,
+                                                const double *up, int nu, double *state, double rr_stop, int it) {
+  __shared__ double sh[4];
+  if (state[3] != 0.0) return;
+  const double rdlast = state[4 + (it & 1)];
+  double s[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) s[j] = rb_total(up + j * nu, nu, sh);
+  const bool stop = it > 1 && !(s[0] >= rr_stop);
+  if (blockIdx.x == 0 && threadIdx.x == 0) pcg_state(state, s, stop, rr_stop, it);
+  if (stop) return;
+  const double beta = it == 1 ? 0.0 : s[1] / rdlast;
+  for (int64_t i = blockIdx.x * (int64_t)PC_T + threadIdx.x; i < n; i += (int64_t)gridDim.x * PC_T)
+    q[i] = r[i] * Adi[i] + beta * q[i];
+}
+__global__ __launch_bounds__(64 * SP_W) void k_pcg_Aq(SellView A, int64_t n, const double *q, double *Aq, double *qp,
+                                                      const double *state) {
+  __shared__ double sh[SP_W][64];
+  if (state[3] != 0.0 || state[6] != 0.0) return;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double dot = 0;
+  for (int64_t b = blockIdx.x; 64 * b < n; b += gridDim.x) {
+    __syncthreads();
+    const int64_t i = 64 * b + lane;
+    const double a = spmv1_row(A, n, i, w, q, sh);
+    if (w == 0 && i < n) {
+      Aq[i] = a;
+      dot += q[i] * a;
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+  if (threadIdx.x == 0) qp[blockIdx.x] = dot;
 }
 // x += alpha q, r -= alpha Aq, and the partial sums of the next iteration
 __global__ __launch_bounds__(PC_T) void k_pcg_update(int64_t n, const double *q, const double *Aq, const double *Adi,
@@ -1411,13 +1451,22 @@ static double pcg_stop(double tol, double nfree) {
   return rr;
 }
 
+// Rows from which the direction and the product are launches of their own.  Small
+// ones are bound by the launches, large ones by the gathers.  20 to 23 iterations,
+// one launch / two, ms: 43,554 rows 0.469 / 0.479, 84,546 0.580 / 0.581, 174,114
+// 0.862 / 0.795, 337,986 1.50 / 1.21, 665,730 2.49 / 1.73, 2,662,530 12.4 / 7.3
+// (with seven launches and a read per iteration 1.37, 1.26, 1.41, 1.75, 2.21, 8.2).
+constexpr int64_t PC_SPLIT = 131072;
+
 // pcg_solver_p.m:49-186 with the 'diag' preconditioner (Polak-Ribiere beta,
-// alpha = r.d / q.Aq), k_pcg_dir and k_pcg_update; the norm is |r| / sqrt(nfree)
+// alpha = r.d / q.Aq), k_pcg_dir or k_pcg_q and k_pcg_Aq, k_pcg_update; the norm is |r| / sqrt(nfree)
 int pcg_diag_run(m3_ctx *c, SellView A, int64_t n, const double *Adi, double *x, double *r, double *q0, double *q1,
                  double *Aq, double nfree, double tol, int itmax, double *norm) {
   hipStream_t s = c->stream;
   double *state = c->scal.p + 16;  // 7 values
-  const int nu = (int)std::min<int64_t>(256, (n + PC_T - 1) / PC_T), nq = (int)((n + 63) / 64);
+  const bool split = n >= PC_SPLIT;
+  const int nu = (int)std::min<int64_t>(split ? 1024 : 256, (n + PC_T - 1) / PC_T);
+  const int nq = (int)std::min<int64_t>(split ? PC_BLOCKS : n, (n + 63) / 64);
   double *up = c->partial.p, *qp = c->partial.p + 3 * nu;
   M3_REQUIRE((size_t)(3 * nu + nq) <= c->partial.n, M3_E_STATE, "partial sums do not fit");
   const double rr_stop = pcg_stop(tol, nfree);
@@ -1429,10 +1478,15 @@ int pcg_diag_run(m3_ctx *c, SellView A, int64_t n, const double *Adi, double *x,
   constexpr int BATCH = 8;
   for (int it = 1;;) {
     for (const int last = std::min(itmax, it + BATCH - 1); it <= last; ++it) {
-      hipLaunchKernelGGL(k_pcg_dir, dim3(nq), dim3(64 * SP_W), 0, s, A, n, r, Adi, q0, q1, Aq, up, nu, qp, state,
-                         rr_stop, it);
-      hipLaunchKernelGGL(k_pcg_update, dim3(nu), dim3(PC_T), 0, s, n, q1, Aq, Adi, qp, nq, x, r, up, nu, state, it);
-      std::swap(q0, q1);
+      if (split) {
+        hipLaunchKernelGGL(k_pcg_q, dim3(nu), dim3(PC_T), 0, s, n, r, Adi, q0, up, nu, state, rr_stop, it);
+        hipLaunchKernelGGL(k_pcg_Aq, dim3(nq), dim3(64 * SP_W), 0, s, A, n, q0, Aq, qp, state);
+      } else {
+        hipLaunchKernelGGL(k_pcg_dir, dim3(nq), dim3(64 * SP_W), 0, s, A, n, r, Adi, q0, q1, Aq, up, nu, qp, state,
+                           rr_stop, it);
+        std::swap(q0, q1);
+      }
+      hipLaunchKernelGGL(k_pcg_update, dim3(nu), dim3(PC_T), 0, s, n, q0, Aq, Adi, qp, nq, x, r, up, nu, state, it);
     }
     hipLaunchKernelGGL(k_pcg_look, dim3(1), dim3(PC_T), 0, s, up, nu, state, rr_stop);
     HIPCHECK(hipMemcpyAsync(c->h_scal + 16, state, 4 * sizeof(double), hipMemcpyDeviceToHost, s));

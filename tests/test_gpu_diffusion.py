@@ -211,3 +211,31 @@ def test_tolerance_whose_square_underflows(c0, ctx0):
     # sums in another order, each iteration 1e-6 of the one before: a few more or fewer
     assert abs(info["nit"] - io["nit"]) <= 5
     assert relerr(T, To) < 1e-10
+
+
+def test_large_grid_matches_the_oracle():
+    """The form of the iteration for large grids (the direction and the product in
+    launches of their own): 174,114 nodes, 983,040 tetrahedra of the split P2
+    elements, more slices of rows than workgroups and a last one of 34 rows; to
+    the tolerance and to a limit behind the first eight iterations."""
+    from m3tet_sph_amd import api, mesh as M
+    from oracle import diffusion as D
+    m = M.build_shell(2, 2, 3, device=0)
+    E, _ = M.p2_to_p1(m.GCOORD, m.levels[0].EL2NOD)
+    X, n = m.GCOORD, m.nnod
+    kdt = min(float(np.sum((X[E[:, i]] - X[E[:, j]]) ** 2, axis=1).min()) for i in range(4) for j in range(i))
+    T0 = np.random.default_rng(9).random(n)
+    ifix, vfix = _fixed(m, n)
+    ctx = api.StokesContext(m)
+    try:
+        ctx.diffusion_mesh(E, n)
+        T, info = ctx.diffusion3d(T0, kdt, 1.0, ifix, vfix, tol=1e-12)
+        _, info9 = ctx.diffusion3d(T0, kdt, 1.0, ifix, vfix, tol=1e-12, itmax=9)
+    finally:
+        ctx.close()
+    To, io = D.diffusion3d_p(T0, kdt, X, m.GCOORD_SPH, E, ifix, vfix, 1.0, tol=1e-12)
+    log("large grid", info["nit"], io["nit"], relerr(T, To))
+    assert info["nit"] == io["nit"] and info9["nit"] == 9 and len(io["hist"]) == io["nit"] + 1
+    assert relerr(info9["norm_r"], io["hist"][9]) < 1e-8 and relerr(info["norm_r"], io["hist"][-1]) < 1e-4
+    # a step's matrix and its solve to 1e-12 of the initial residual
+    assert relerr(T, To) < 1e-10
