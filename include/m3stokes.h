@@ -146,7 +146,11 @@ typedef struct {
   int32_t nitP, nitU, nitZ;
   double norm_rP;            /* final pressure residual (RMS) */
   double norm_rP0;           /* initial pressure residual (RMS) */
-  double t_assemble, t_restrict, t_factor, t_pressure, t_velocity, t_total; /* s */
+  /* s.  Host times: the solve waits for the device once per CG iteration, so
+   * pressure kernels that are queued ahead of a velocity solve end in its first
+   * wait and count as t_velocity; t_pressure is the host's time between the
+   * velocity solves, the wait for a pressure step's norm included. */
+  double t_assemble, t_restrict, t_factor, t_pressure, t_velocity, t_total;
 } m3_info;
 
 int m3_create(m3_ctx **ctx, int hip_device);

@@ -388,8 +388,8 @@ __device__ inline void pair_sum(const double *Abase, const double *Bbase, const 
 
 // C_IJ -= sum_pairs L_IK L_JK'  (one workgroup per chunk of at most UCH pairs
 // of a target tile; chunks of one tile subtract atomically).  Factorisation of
-// 34 / 275 / 1,844 tile columns with 3, 4, 6 and 8 pairs per chunk: 635 / 2,370 /
-// 15,655, 635 / 2,350 / 15,690, 625 / 2,340 / 15,406 and 681 / 2,555 / 15,833 us.
+// 34 / 275 / 1,844 tile columns with 3, 4, 6 and 8 pairs per chunk: 628 / 2,307 /
+// 15,297, 621 / 2,282 / 15,363, 628 / 2,302 / 15,045 and 670 / 2,503 / 15,510 us.
 constexpr int UCH = 6;
 struct UpdArgs {
   const int32_t *tile;         // per chunk: target tile
