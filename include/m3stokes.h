@@ -161,11 +161,12 @@ const char *m3_last_error(const m3_ctx *ctx);
 
 int m3_set_mesh(m3_ctx *ctx, const m3_mesh_desc *mesh);
 /* Which multigrid levels the m3_set_mesh calls from now on sweep in windows: the
- * fewest rows of such a level, and the most vector entries that a window of more
- * than 64 rows / one of 64 rows gathers (at most 6300; larger windows are split,
- * and a level whose 64 rows gather more has no windows).  0: the library's own
- * choice.  It moves work, not results.  No reference counterpart. */
-int m3_sweep_windows(m3_ctx *ctx, int64_t rows, int32_t split, int32_t limit);
+ * fewest rows of such a level, the most vector entries that a window of more than
+ * 64 rows / one of 64 rows gathers (at most 6300; larger windows are split), and
+ * the most that all windows of a level gather per row; a level that meets one of
+ * the last two has no windows.  0: the library's own choice.  It moves work, not
+ * results.  No reference counterpart. */
+int m3_sweep_windows(m3_ctx *ctx, int64_t rows, int32_t split, int32_t limit, int32_t per_row);
 /* ifix: 1-based rotated-frame dofs, vfix: values (UBC.ifix / UBC.vfix). */
 int m3_set_bc(m3_ctx *ctx, const int64_t *ifix, const double *vfix, int64_t nfix);
 

@@ -105,7 +105,7 @@ LIB.m3_set_fields.argtypes = [C.c_void_p, D, D]
 LIB.m3_apply.argtypes = [C.c_void_p, C.c_int32, C.c_int32, D, D]
 LIB.m3_get_vector.argtypes = [C.c_void_p, C.c_int32, C.c_int32, D]
 LIB.m3_stats.argtypes = [C.c_void_p, I64, C.c_int32]
-LIB.m3_sweep_windows.argtypes = [C.c_void_p, C.c_int64, C.c_int32, C.c_int32]
+LIB.m3_sweep_windows.argtypes = [C.c_void_p, C.c_int64, C.c_int32, C.c_int32, C.c_int32]
 LIB.m3_sl_advect.argtypes = [C.c_void_p, D, D, C.c_double, C.c_double, C.c_double, D]
 
 
@@ -401,7 +401,7 @@ class StokesContext:
     """Device state of one mesh (patterns, operators, hierarchy, factor)."""
 
     def __init__(self, mesh: meshmod.ShellMesh, device=0, sweep_windows=None):
-        """sweep_windows: (rows, split, limit) of m3_sweep_windows."""
+        """sweep_windows: (rows, split, limit, per_row) of m3_sweep_windows."""
         self._h = C.c_void_p()
         rc = LIB.m3_create(C.byref(self._h), device)
         if rc:

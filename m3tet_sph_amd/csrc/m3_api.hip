@@ -108,8 +108,8 @@ struct WindowTable {
 
 }  // namespace
 
-bool Sell::build_windows(const std::vector<int32_t> &order, const std::vector<int32_t> &first,
-                         const m3::SweepRule &rule) {
+m3::WindowFit Sell::build_windows(const std::vector<int32_t> &order, const std::vector<int32_t> &first,
+                                  const m3::SweepRule &rule) {
   const int64_t nw = (int64_t)first.size() - 1;
   std::vector<std::vector<int32_t>> lists(nw);
   HostArr<uint16_t> h_idx((size_t)nslot), h_lrow(nrow);
@@ -157,7 +157,10 @@ bool Sell::build_windows(const std::vector<int32_t> &order, const std::vector<in
     }
   }
   if (!memory) throw std::bad_alloc();
-  if (!fits) return false;
+  if (!fits) return m3::WindowFit::oversized;
+  int64_t total = 0;
+  for (const auto &l : lists) total += (int64_t)l.size();
+  if (total > rule.per_row * nrow || total > INT32_MAX) return m3::WindowFit::scattered;
   std::vector<int2> h_win(nw + 1, int2{0, 0});
   umax = 0;
   for (int64_t b = 0; b < nw; ++b) {
@@ -177,7 +180,7 @@ bool Sell::build_windows(const std::vector<int32_t> &order, const std::vector<in
   h_vpos.swap(pos);
   vperm.upload(h_vperm);
   vpos.upload(h_vpos);
-  return true;
+  return m3::WindowFit::ok;
 }
 
 namespace {
@@ -492,15 +495,15 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
         };
         build();
         mark("level connectivity + K pattern");
-        if (!lv.K.build_windows(order, first, c->sweep_rule)) {
+        m3::WindowFit fit = lv.K.build_windows(order, first, c->sweep_rule);
+        if (fit == m3::WindowFit::oversized) {
           first = split_windows(order, first, ptr, cols, c->sweep_rule);
-          if (first.empty()) {
-            lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
-          } else {
+          if (!first.empty()) {
             build();
-            M3_REQUIRE(lv.K.build_windows(order, first, c->sweep_rule), M3_E_MESH, "sweep windows do not fit");
+            fit = lv.K.build_windows(order, first, c->sweep_rule);
           }
         }
+        if (fit != m3::WindowFit::ok) lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
         mark("sweep windows");
       } else {
         lv.K.build(lv.nnod, lv.nnod, ptr, cols, 9);
@@ -759,14 +762,15 @@ int m3_set_mesh(m3_ctx *c, const m3_mesh_desc *m) {
   });
 }
 
-int m3_sweep_windows(m3_ctx *c, int64_t rows, int32_t split, int32_t limit) {
+int m3_sweep_windows(m3_ctx *c, int64_t rows, int32_t split, int32_t limit, int32_t per_row) {
   return guard(c, [&] {
-    M3_REQUIRE(rows >= 0 && split >= 0 && limit >= 0 && limit <= m3::SWEEP_LIMIT, M3_E_ARG,
+    M3_REQUIRE(rows >= 0 && split >= 0 && per_row >= 0 && limit >= 0 && limit <= m3::SWEEP_LIMIT, M3_E_ARG,
                "sweep windows: sizes must not be negative, limit at most 6300");
     m3::SweepRule r;
     if (rows) r.rows = rows;
     if (split) r.split = split;
     if (limit) r.limit = limit;
+    if (per_row) r.per_row = per_row;
     c->sweep_rule = r;
   });
 }

@@ -170,17 +170,20 @@ constexpr int HOST_PARTS = 512;
 // 512 rows), so a window of more is halved, down to the 64 rows of a slice.
 // A slice may gather as many as fit into the LDS of a CU beside its sums; a
 // level with a slice of more (a node with thousands of neighbours) is swept
-// without windows.  337,986 rows, us per sweep in FP64 / BF16: 131 / 41.6 as they
-// are, 139 / 49.3 with all windows halved, 214 / 87.3 in slices of 64 rows, 157 /
-// 56.0 without windows: a piece costs more than its share, so only the windows
-// that need it are split, and one of them in a mesh does not cost the others
-// their form.
+// without windows, and so is one whose windows gather more than four entries per
+// row in all, because they had to be split or the space-filling order is none for
+// its numbering.  337,986 rows, entries per row and us per sweep in FP64 / BF16:
+// windows of 512 rows 2.7, 131 / 41.6; 256 rows 3.3, 139 / 49.3; 148 on average 3.9,
+// 158 / 56.4; 64 rows 5.1, 214 / 87.3; with the coordinates of two thirds of the
+// nodes dealt out anew 20, 239 / 110; without windows 157 / 56.0 on both.
 constexpr int SWEEP_LIMIT = 6300;
 struct SweepRule {
   int64_t rows = 131072;                      // fewest rows of a level with windows (sweep_window)
   int32_t split = 2900, limit = SWEEP_LIMIT;  // most entries of a window, of a slice
+  int32_t per_row = 4;                        // most entries per row of the level
   int most(int64_t nr) const { return nr > 64 ? std::min(split, limit) : limit; }
 };
+enum class WindowFit { ok, oversized, scattered };
 }  // namespace m3
 
 struct Sell {
@@ -208,10 +211,10 @@ struct Sell {
   void build(int64_t nrow_, int64_t ncol_, const std::vector<int64_t> &ptr,
              const std::vector<int32_t> &cols, int bs_, const std::vector<int32_t> *place = nullptr);
   // window lists; first: the first row of each window in the vector order, and
-  // nrow.  false (and nothing kept) if a window gathers more entries than rule
-  // allows one of its size
-  bool build_windows(const std::vector<int32_t> &order, const std::vector<int32_t> &first,
-                     const m3::SweepRule &rule);
+  // nrow.  Nothing is kept if a window gathers more entries than rule allows one
+  // of its size (oversized) or all of them more than it allows the level (scattered)
+  m3::WindowFit build_windows(const std::vector<int32_t> &order, const std::vector<int32_t> &first,
+                              const m3::SweepRule &rule);
   int64_t base_of(int64_t row) const {
     const int64_t q = h_ipos.empty() ? row : (int64_t)h_ipos[row];
     return h_slice_ptr[q >> 6] + (q & 63);
